@@ -113,3 +113,33 @@ def test_config3_norm_sampled_within_one_bf16_ulp(device):
     rows = torch.randperm(131072, generator=g)[:8192]
     want, _ = oracle.rmsnorm_silu_f64(h[rows].float().numpy(), gamma.float().numpy())
     assert bf16_ulps(y[rows.to(device)], want).max() <= 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,hidden,offset", [
+    (1, 1, 0), (70, 128, 0), (33, 136, 0), (17, 512, 1), (1030, 520, 0), (19, 1024, 0), (5, 1032, 0), (7, 8192, 0),
+    (5, 8200, 0), (35, 129, 0), (9, 257, 3), (21, 513, 0), (1027, 1021, 0), (6, 1025, 1), (3, 4097, 0),
+])
+def test_rows_of_every_layout(device, dtype, rows, hidden, offset):
+    """Forward and both gradients at the edges of the row layouts (lanes per row, vectors or single
+    elements by width and alignment, more rows than one sweep of the workgroups), against float64.
+    Bounds: half an ulp of the result's type, and 2^-24 per term of the fp32 sums behind it (a row's
+    or a column's length, the result's own scale), with 16 for the few roundings around them."""
+
+    g = torch.Generator().manual_seed(rows * 10007 + hidden)
+    def make(*shape):
+        flat = torch.randn((int(np.prod(shape)) + offset,), generator=g).to(dtype).to(device)
+        return flat[offset:].view(*shape)
+    x, up, w = make(rows, hidden), make(rows, hidden), make(hidden)
+    xs, ws = x.detach().requires_grad_(), w.detach().requires_grad_()
+    y = core.fused_rmsnorm_silu(xs, ws, 1e-6)
+    dx, dw = torch.autograd.grad(y, (xs, ws), up)
+    x64, w64, up64 = (t.detach().double().cpu() for t in (x, w, up))
+    x64.requires_grad_(), w64.requires_grad_()
+    ref = F.silu(x64 * torch.rsqrt(x64.square().mean(dim=-1, keepdim=True) + 1e-6) * w64)
+    rx, rw = torch.autograd.grad(ref, (x64, w64), up64)
+    half_ulp = {torch.float32: 2.0**-24, torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[dtype]
+    for got, want, terms in ((y, ref.detach(), hidden), (dx, rx, hidden), (dw, rw, rows)):
+        got = got.detach().double().cpu()
+        bound = half_ulp * want.abs() + (16 + terms) * 2.0**-24 * (1.0 + want.abs().max())
+        assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
