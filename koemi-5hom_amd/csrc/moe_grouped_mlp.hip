@@ -18,6 +18,7 @@
 // valid pairs are zero-filled.
 #include "common.hpp"
 #include "mfma_stage.hpp"
+#include "split_gemm.hpp"
 
 #include <type_traits>
 
@@ -57,28 +58,38 @@ constexpr int kMaxSplit = 4;  // chunks per leftover tile (the fixup reads every
 constexpr size_t kPartialTileFloats = static_cast<size_t>(kBM) * kBN;  // the workspace's room per partial tile
 
 struct MlpWorkspace {
-    size_t hidden_off, slot_expert_off, slot_row_off, slot_end_off, partial_off, total;
+    size_t hidden_off, slot_expert_off, slot_row_off, slot_end_off, first_tile_off, partial_off, total;
     int64_t max_slots;
 };
 
-// The MFMA path (both GEMM K dimensions multiples of kKAlign) keeps H in bf16; the
-// SIMT path keeps it in fp32.
+// The bf16 tile path (both GEMM K dimensions multiples of kKAlign) keeps H in
+// bf16; the any-shape path keeps it in fp32, rows padded to hidden_stride.
 inline bool mfma_shape(int64_t width, int64_t hidden, int dtype) {
     return dtype == KOEMI_BF16 && width % kKAlign == 0 && hidden % kKAlign == 0;
 }
+inline int64_t hidden_stride(int64_t hidden) { return (hidden + 7) / 8 * 8; }  // 32-byte fp32 octets
+
+// Rows of the any-shape path's tiles: 128, or 64 when the experts' segments
+// average at most kAnySmallRows rows (a 128-row tile would be mostly padding).
+constexpr int64_t kAnySmallRows = 96;
+inline int any_rows(int64_t pairs, int64_t E) { return pairs <= kAnySmallRows * E ? 64 : 128; }
 
 inline MlpWorkspace mlp_workspace(int64_t pairs, int64_t width, int64_t hidden, int64_t E, int dtype) {
     MlpWorkspace w;
-    w.max_slots = (pairs + kBM - 1) / kBM + E;
-    const size_t elem = mfma_shape(width, hidden, dtype) ? 2 : 4;
+    const bool tiles = mfma_shape(width, hidden, dtype);
+    const int64_t bm = tiles ? kBM : any_rows(pairs, E);
+    w.max_slots = (pairs + bm - 1) / bm + E;
+    if (!tiles && pairs < w.max_slots) w.max_slots = pairs > 0 ? pairs : 1;  // a slot holds at least one pair
+    const size_t row = tiles ? static_cast<size_t>(hidden) * 2 : static_cast<size_t>(hidden_stride(hidden)) * 4;
     w.hidden_off = 0;
-    w.slot_expert_off = align256(static_cast<size_t>(pairs > 0 ? pairs : 1) * static_cast<size_t>(hidden) * elem);
+    w.slot_expert_off = align256(static_cast<size_t>(pairs > 0 ? pairs : 1) * row);
     // slot_expert has one more entry: the number of slots in use.
     w.slot_row_off = w.slot_expert_off + align256(static_cast<size_t>(w.max_slots + 1) * sizeof(int32_t));
     w.slot_end_off = w.slot_row_off + align256(static_cast<size_t>(w.max_slots) * sizeof(int64_t));
-    w.partial_off = w.slot_end_off + align256(static_cast<size_t>(w.max_slots) * sizeof(int64_t));
+    w.first_tile_off = w.slot_end_off + align256(static_cast<size_t>(w.max_slots) * sizeof(int64_t));
+    w.partial_off = w.first_tile_off + (tiles ? 0 : align256(static_cast<size_t>(E + 1) * sizeof(int32_t)));
     w.total = w.partial_off;
-    if (mfma_shape(width, hidden, dtype)) w.total += kMaxSplitUnits * kPartialTileFloats * sizeof(float);
+    if (tiles) w.total += kMaxSplitUnits * kPartialTileFloats * sizeof(float);
     return w;
 }
 
@@ -87,9 +98,10 @@ __device__ __forceinline__ float silu_f(float v) {
     return v * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-// slot -> (expert, first row, segment end) for every BM-row tile of every
+// slot -> (expert, first row, segment end) for every bm-row tile of every
 // expert segment, built by one workgroup: per-expert tile counts, their
-// exclusive prefix in LDS, then a binary search per slot. Segment bounds are
+// exclusive prefix in LDS (in `scratch`, E + 1 entries of global memory, where
+// the experts are too many for it), then a binary search per slot. Segment bounds are
 // clamped to [0, pairs] so that malformed offsets can never address rows
 // outside the operands.
 constexpr int kSchedThreads = 1024;
@@ -103,15 +115,17 @@ __device__ __forceinline__ void segment_bounds(const int64_t* __restrict__ offse
 
 __global__ __launch_bounds__(kSchedThreads) void build_schedule_kernel(
     const int64_t* __restrict__ offsets, int64_t E, int64_t pairs, int64_t max_slots,
-    int32_t* __restrict__ slot_expert, int64_t* __restrict__ slot_row, int64_t* __restrict__ slot_end) {
-    extern __shared__ int32_t first_tile[];  // E + 1 entries
+    int32_t* __restrict__ slot_expert, int64_t* __restrict__ slot_row, int64_t* __restrict__ slot_end,
+    int64_t bm, int32_t* scratch) {
+    extern __shared__ int32_t first_tile_lds[];  // E + 1 entries
+    int32_t* const first_tile = scratch ? scratch : first_tile_lds;
     __shared__ int32_t wave_tot[kSchedThreads / kWave];
     const int tid = threadIdx.x;
     const int64_t n = E + 1;
     for (int64_t e = tid; e < E; e += kSchedThreads) {
         int64_t lo, hi;
         segment_bounds(offsets, e, pairs, lo, hi);
-        first_tile[e] = static_cast<int32_t>((hi - lo + kBM - 1) / kBM);
+        first_tile[e] = static_cast<int32_t>((hi - lo + bm - 1) / bm);
     }
     if (tid == 0) first_tile[E] = 0;
     __syncthreads();
@@ -145,7 +159,7 @@ __global__ __launch_bounds__(kSchedThreads) void build_schedule_kernel(
         int64_t lo, hi;
         segment_bounds(offsets, lo_e, pairs, lo, hi);
         slot_expert[slot] = static_cast<int32_t>(lo_e);
-        slot_row[slot] = lo + (slot - first_tile[lo_e]) * kBM;
+        slot_row[slot] = lo + (slot - first_tile[lo_e]) * bm;
         slot_end[slot] = hi;
     }
 }
@@ -569,46 +583,95 @@ __global__ __launch_bounds__(256) void split_fixup_kernel(
     }
 }
 
-// ------------------------------------------------- fp32-accumulating SIMT path
-// One 256-thread block per sorted pair (the reference's decomposition), used for
-// float32 / float16 weights and for shapes the MFMA tiles do not cover.
-template <typename T>
-__global__ __launch_bounds__(256) void glu_hidden_simt_kernel(
-    const T* __restrict__ x, const int64_t* __restrict__ experts, const int64_t* __restrict__ offsets, int64_t E,
-    const T* __restrict__ Wg, const T* __restrict__ bg, const T* __restrict__ Wv, const T* __restrict__ bv,
-    float* __restrict__ H, int64_t D, int64_t Hd) {
-    const int64_t p = blockIdx.x;
-    if (p >= offsets[E]) return;  // the grid covers exactly the pairs, so p < pairs
-    const int64_t e = experts[p];
-    if (e < 0 || e >= E) return;
-    const T* xr = x + p * D;
-    for (int64_t h = threadIdx.x; h < Hd; h += 256) {
-        const T* wg = Wg + (e * Hd + h) * D;
-        const T* wv = Wv + (e * Hd + h) * D;
-        float g = to_f32(bg[e * Hd + h]), u = to_f32(bv[e * Hd + h]);
-        for (int64_t c = 0; c < D; ++c) {
-            const float xv = to_f32(xr[c]);
-            g = __builtin_fmaf(xv, to_f32(wg[c]), g);
-            u = __builtin_fmaf(xv, to_f32(wv[c]), u);
+// ------------------------------------------------------- any-shape path ---
+// float32 and float16 operands, and bf16 of any width and alignment, as tiles of
+// split_gemm.hpp: BM pairs of one expert x 128 weight rows, whatever is past
+// the segment, the weights or K filled with zeros on the way into LDS. The
+// hidden activations stay fp32 (GEMM 2 splits them into three bf16 planes).
+// Bound by the matrix cores (one product per operand pair for 16-bit GEMM 1,
+// three to six otherwise) with the splits on the vector units beside them.
+// 5400 pairs over 12 experts, 768 -> 2000 -> 768 (both GEMMs): fp16 68 + 129 us
+// (GEMM 1 at 540 TFLOP/s, GEMM 2 at 143, 715 counting its five products), fp32
+// 210 + 149 us (176 TFLOP/s, 1.06 PFLOP/s counting six); a thread per output
+// with a scalar multiply-add chain, as these types ran before, took 107 and
+// 181 ms. bf16 1000 -> 1400 -> 1000: 70 + 83 us against 89 ms.
+template <bool GLU, typename TA, typename TW, int BM, int BN, bool VEC>
+__global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kernel(
+    const TA* __restrict__ A, const TW* __restrict__ W0, const TW* __restrict__ W1, const TW* __restrict__ bias0,
+    const TW* __restrict__ bias1, void* __restrict__ out, const int32_t* __restrict__ slot_expert,
+    const int64_t* __restrict__ slot_row, const int64_t* __restrict__ slot_end, int64_t n_out, int64_t K,
+    int64_t lda, int64_t ldc, int64_t max_slots, int64_t n_tiles) {
+    static_assert(!GLU || BN == 128, "a wave holds one gate and one value tile of the same hidden units");
+    using G = split_gemm::Tile<TA, TW, BM, BN>;
+    __shared__ __attribute__((aligned(16))) char lds[G::kLdsBytes];
+    // workgroup b runs on XCD b % 8: every XCD takes a contiguous range of
+    // tiles, in groups of kGroupM slots, so that its L2 serves the operands
+    // that concurrently running tiles share
+    const uint32_t slots = static_cast<uint32_t>(min(static_cast<int64_t>(slot_expert[max_slots]), max_slots));
+    const uint32_t tiles = slots * static_cast<uint32_t>(n_tiles);
+    const uint32_t per_xcd = (tiles + 7) / 8;
+    if ((blockIdx.x >> 3) >= per_xcd) return;
+    const uint32_t logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (logical >= tiles) return;
+    uint32_t slot, tile_n;
+    tile_coords(logical, slots, static_cast<uint32_t>(n_tiles), slot, tile_n);
+    const int e = slot_expert[slot];
+    if (e < 0) return;
+    const int64_t row0 = slot_row[slot], row_end = slot_end[slot];
+    // GLU: B rows 0-63 are gate rows and 64-127 the value rows of the same 64
+    // hidden units; a wave's n-tile 0 is gate, 1 value.
+    const int64_t n0 = static_cast<int64_t>(tile_n) * (GLU ? BN / 2 : BN);
+    const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
+    const TW* w0 = W0 + static_cast<int64_t>(e) * n_out * K;
+    const TW* w1 = W1 + static_cast<int64_t>(e) * n_out * K;
+    G tile;
+    tile.template run<VEC>(
+             lds, lda, K, 0, (K + G::BK - 1) / G::BK * G::BK,
+             [&](int r) { return A + min(row0 + r, row_end - 1) * lda; },
+             [&](int r) {
+                 if (GLU) return (r < BN / 2 ? w0 : w1) + min(n0 + (r & (BN / 2 - 1)), n_out - 1) * K;
+                 return w0 + min(n0 + r, n_out - 1) * K;
+             },
+             [&](int t) { return GLU ? t * (BN / 2) + wn * 32 : wn * (BN / 2) + t * 32; });
+#pragma unroll
+    for (int i = 0; i < G::MT; ++i) {
+        const int64_t row = row0 + wm * (BM / 2) + i * 32 + (lane_id() & 31);
+        if (row >= row_end) continue;
+        const TA* a = A + row * lda;
+#pragma unroll
+        for (int j = 0; j < (GLU ? 1 : G::NT); ++j) {
+            const int64_t first = n0 + (GLU ? wn * 32 : wn * (BN / 2) + j * 32);
+#pragma unroll
+            for (int v = 0; v < 16; v += 4) {
+                const int64_t col = first + split_gemm::acc_column(v);  // four columns from here
+                float o[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t c = col + q;
+                    o[q] = 0.0f;
+                    if (c >= n_out) continue;
+                    const float b0 = to_f32(bias0[static_cast<int64_t>(e) * n_out + c]);
+                    float x = tile.acc[i][j][v + q] + b0;
+                    if (!G::kNative && !split_gemm::finite(x)) x = split_gemm::scalar_dot(a, w0 + c * K, K, b0);
+                    o[q] = x;
+                    if constexpr (GLU) {
+                        const float b1 = to_f32(bias1[static_cast<int64_t>(e) * n_out + c]);
+                        float u = tile.acc[i][G::NT - 1][v + q] + b1;
+                        if (!G::kNative && !split_gemm::finite(u)) u = split_gemm::scalar_dot(a, w1 + c * K, K, b1);
+                        o[q] = silu_f(x) * u;
+                    }
+                }
+                if constexpr (GLU) {
+                    // H rows are padded to a multiple of 8 columns, zeros past n_out
+                    if (col < ldc) store4(static_cast<float*>(out) + row * ldc + col, o[0], o[1], o[2], o[3]);
+                } else {
+                    TW* y = static_cast<TW*>(out) + row * ldc + col;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (col + q < n_out) y[q] = from_f32<TW>(o[q]);
+                }
+            }
         }
-        H[p * Hd + h] = silu_f(g) * u;
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void glu_output_simt_kernel(
-    const float* __restrict__ H, const int64_t* __restrict__ experts, const int64_t* __restrict__ offsets, int64_t E,
-    const T* __restrict__ Wo, const T* __restrict__ bo, T* __restrict__ y, int64_t D, int64_t Hd) {
-    const int64_t p = blockIdx.x;
-    if (p >= offsets[E]) return;
-    const int64_t e = experts[p];
-    if (e < 0 || e >= E) return;
-    const float* hr = H + p * Hd;
-    for (int64_t c = threadIdx.x; c < D; c += 256) {
-        const T* wo = Wo + (e * D + c) * Hd;
-        float acc = to_f32(bo[e * D + c]);
-        for (int64_t h = 0; h < Hd; ++h) acc = __builtin_fmaf(hr[h], to_f32(wo[h]), acc);
-        y[p * D + c] = from_f32<T>(acc);
     }
 }
 
@@ -835,25 +898,6 @@ __global__ void zero_tail_rows_kernel(T* __restrict__ y, const int64_t* __restri
 
 inline unsigned tail_blocks(int64_t pairs) { return static_cast<unsigned>(pairs < 1024 ? (pairs > 0 ? pairs : 1) : 1024); }
 
-template <typename T>
-int run_simt(const void* x, const int64_t* experts, const int64_t* offsets, const void* Wg, const void* bg,
-             const void* Wv, const void* bv, const void* Wo, const void* bo, void* y, int64_t P, int64_t D, int64_t Hd,
-             int64_t E, float* H, hipStream_t s) {
-    if (P > 0x7fffffffLL) return fail(KOEMI_ERR_UNSUPPORTED, "too many pairs for the SIMT grouped MLP");
-    const dim3 grid(static_cast<unsigned>(P)), block(256);
-    hipLaunchKernelGGL(glu_hidden_simt_kernel<T>, grid, block, 0, s, static_cast<const T*>(x), experts, offsets, E,
-                       static_cast<const T*>(Wg), static_cast<const T*>(bg), static_cast<const T*>(Wv),
-                       static_cast<const T*>(bv), H, D, Hd);
-    int st = check_launch("koemi_moe_grouped_mlp(hidden)");
-    if (st != KOEMI_OK) return st;
-    hipLaunchKernelGGL(glu_output_simt_kernel<T>, grid, block, 0, s, H, experts, offsets, E, static_cast<const T*>(Wo),
-                       static_cast<const T*>(bo), static_cast<T*>(y), D, Hd);
-    st = check_launch("koemi_moe_grouped_mlp(output)");
-    if (st != KOEMI_OK) return st;
-    hipLaunchKernelGGL(zero_tail_rows_kernel<T>, dim3(tail_blocks(P)), block, 0, s, static_cast<T*>(y), offsets + E, P, D);
-    return check_launch("koemi_moe_grouped_mlp(zero)");
-}
-
 // Compute units of the current device (the rounds of one-workgroup-per-CU tiles).
 int64_t device_cus() {
     static int cached[64] = {};
@@ -864,6 +908,60 @@ int64_t device_cus() {
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
     cached[dev] = n;
     return n;
+}
+
+template <typename T, int BM>
+int run_any(const void* x, const int64_t* offsets, const void* Wg, const void* bg, const void* Wv, const void* bv,
+            const void* Wo, const void* bo, void* y, int64_t P, int64_t D, int64_t Hd, int64_t E,
+            const MlpWorkspace& ws, char* base, hipStream_t s) {
+    float* H = reinterpret_cast<float*>(base + ws.hidden_off);
+    int32_t* slot_expert = reinterpret_cast<int32_t*>(base + ws.slot_expert_off);
+    int64_t* slot_row = reinterpret_cast<int64_t*>(base + ws.slot_row_off);
+    int64_t* slot_end = reinterpret_cast<int64_t*>(base + ws.slot_end_off);
+    const bool lds_prefix = E <= kMaxScheduleExperts;
+    const int64_t ld_h = hidden_stride(Hd);
+    const int64_t tiles1 = (Hd + 63) / 64;
+    // GEMM 2 in 64-column tiles where 128-column ones would give the CUs fewer
+    // than two each (fp16 at the sizes above: 129 against 135 us, fp32 149 against 162)
+    const bool narrow = ws.max_slots * ((D + 127) / 128) < 2 * device_cus();
+    const int64_t tiles2 = narrow ? (D + 63) / 64 : (D + 127) / 128;
+    if (ws.max_slots * (tiles1 > tiles2 ? tiles1 : tiles2) > 0x7ffffff0LL)
+        return fail(KOEMI_ERR_UNSUPPORTED, "too many tiles for the grouped MLP");
+    hipLaunchKernelGGL(build_schedule_kernel, dim3(1), dim3(kSchedThreads),
+                       lds_prefix ? static_cast<size_t>(E + 1) * sizeof(int32_t) : 0, s, offsets, E, P, ws.max_slots,
+                       slot_expert, slot_row, slot_end, static_cast<int64_t>(BM),
+                       lds_prefix ? nullptr : reinterpret_cast<int32_t*>(base + ws.first_tile_off));
+    int st = check_launch("koemi_moe_grouped_mlp(schedule)");
+    if (st != KOEMI_OK) return st;
+    const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    const T* wg = static_cast<const T*>(Wg);
+    const T* wv = static_cast<const T*>(Wv);
+    const T* wo = static_cast<const T*>(Wo);
+    const auto launch = [&](auto vec_kernel, auto kernel, bool vec, const auto* a, const T* w0, const T* w1, const void* b0,
+                            const void* b1, void* out, int64_t n_out, int64_t K, int64_t lda, int64_t ldc, int64_t n_tiles,
+                            const char* what) {
+        hipLaunchKernelGGL(vec ? vec_kernel : kernel, dim3(static_cast<unsigned>((ws.max_slots * n_tiles + 7) / 8 * 8)),
+                           dim3(split_gemm::kThreads), 0, s, a, w0, w1, static_cast<const T*>(b0),
+                           static_cast<const T*>(b1), out, slot_expert, slot_row, slot_end, n_out, K, lda, ldc,
+                           ws.max_slots, n_tiles);
+        return check_launch(what);
+    };
+    st = launch(grouped_gemm_any_kernel<true, T, T, BM, 128, true>, grouped_gemm_any_kernel<true, T, T, BM, 128, false>,
+                D % 8 == 0 && aligned(x) && aligned(Wg) && aligned(Wv), static_cast<const T*>(x), wg, wv, bg, bv, H, Hd, D,
+                D, ld_h, tiles1, "koemi_moe_grouped_mlp(hidden)");
+    if (st != KOEMI_OK) return st;
+    const auto second = [&](auto vec_kernel, auto kernel) {
+        return launch(vec_kernel, kernel, Hd % 8 == 0 && aligned(Wo), H, wo, wo, bo, bo, y, D, Hd, ld_h, D, tiles2,
+                      "koemi_moe_grouped_mlp(output)");
+    };
+    st = narrow ? second(grouped_gemm_any_kernel<false, float, T, BM, 64, true>,
+                         grouped_gemm_any_kernel<false, float, T, BM, 64, false>)
+                : second(grouped_gemm_any_kernel<false, float, T, BM, 128, true>,
+                         grouped_gemm_any_kernel<false, float, T, BM, 128, false>);
+    if (st != KOEMI_OK) return st;
+    hipLaunchKernelGGL(zero_tail_rows_kernel<T>, dim3(tail_blocks(P)), dim3(256), 0, s, static_cast<T*>(y),
+                       offsets + E, P, D);
+    return check_launch("koemi_moe_grouped_mlp(zero)");
 }
 
 // x_index (or null): GEMM 1 reads context row x_index[i] (of x_rows) for pair i.
@@ -886,7 +984,8 @@ int run_mfma(const void* x, const int64_t* x_index, int64_t x_rows, const int64_
         return run_skinny<false>(x, x_index, x_rows, offsets, Wg, bg, Wv, bv, Wo, bo, y, P, D, Hd, E, H, s, zero_tail);
     }
     hipLaunchKernelGGL(build_schedule_kernel, dim3(1), dim3(kSchedThreads), static_cast<size_t>(E + 1) * sizeof(int32_t),
-                       s, offsets, E, P, ws.max_slots, slot_expert, slot_row, slot_end);
+                       s, offsets, E, P, ws.max_slots, slot_expert, slot_row, slot_end, static_cast<int64_t>(kBM),
+                       static_cast<int32_t*>(nullptr));
     int st = check_launch("koemi_moe_grouped_mlp(schedule)");
     if (st != KOEMI_OK) return st;
     const int64_t slots = ws.max_slots;
@@ -965,20 +1064,17 @@ extern "C" int koemi_moe_grouped_mlp(const void* sorted_context, const int64_t* 
         return run_mfma(sorted_context, nullptr, pairs, segment_offsets, gate_weights, gate_biases, value_weights,
                         value_biases, output_weights, output_biases, output, pairs, width, hidden, expert_count, ws,
                         base, s, true);
-    float* H = reinterpret_cast<float*>(base + ws.hidden_off);
+    const bool small = any_rows(pairs, expert_count) == 64;
+    const auto run = [&](auto tag) {
+        using T = decltype(tag);
+        const auto go = small ? run_any<T, 64> : run_any<T, 128>;
+        return go(sorted_context, segment_offsets, gate_weights, gate_biases, value_weights, value_biases,
+                  output_weights, output_biases, output, pairs, width, hidden, expert_count, ws, base, s);
+    };
     switch (dtype) {
-        case KOEMI_F32:
-            return run_simt<float>(sorted_context, sorted_experts, segment_offsets, gate_weights, gate_biases,
-                                   value_weights, value_biases, output_weights, output_biases, output, pairs, width,
-                                   hidden, expert_count, H, s);
-        case KOEMI_F16:
-            return run_simt<f16>(sorted_context, sorted_experts, segment_offsets, gate_weights, gate_biases,
-                                 value_weights, value_biases, output_weights, output_biases, output, pairs, width,
-                                 hidden, expert_count, H, s);
-        default:
-            return run_simt<bf16>(sorted_context, sorted_experts, segment_offsets, gate_weights, gate_biases,
-                                  value_weights, value_biases, output_weights, output_biases, output, pairs, width,
-                                  hidden, expert_count, H, s);
+        case KOEMI_F32: return run(float{});
+        case KOEMI_F16: return run(f16{});
+        default: return run(bf16{});
     }
 }
 

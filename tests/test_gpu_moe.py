@@ -532,3 +532,76 @@ def test_small_combine_bit_exact(device, tokens, k, E, learned):
     want = oracle.combine(y.float().cpu().numpy(), rows.cpu().numpy(), offsets.cpu().numpy(), tokens, k,
                           pair_weights=sw.cpu().numpy() if sw is not None else None)
     np.testing.assert_array_equal(out.cpu().view(torch.int16).numpy(), oracle.f32_to_bf16(want).view(np.int16))
+
+
+def any_shape_mlp(device, dtype, sizes, D, H, scale=0.05, seed=0):
+    """(inputs, output, float64 reference, bound) of a grouped MLP outside the bf16 tile shapes.
+
+    bound = half an ulp of the output's type + 4 sqrt(n) 2^-24 sum |terms| for each fp32 sum (Higham's
+    sqrt(n) model with a factor of 4), the gate and value sums' errors carried through silu(g) u
+    (|silu'| <= 1.1; 16 ulps for its exp, reciprocal and products) and the output weights."""
+
+    g = torch.Generator().manual_seed(seed + sum(sizes) * 31 + D)
+    E = len(sizes)
+    offsets = np.concatenate([[0], np.cumsum(sizes)])
+    P = int(offsets[-1]) + 3
+    x = torch.randn((P, D), generator=g).to(dtype)
+    experts = torch.full((P,), E, dtype=torch.int64)
+    for e in range(E):
+        experts[offsets[e]:offsets[e + 1]] = e
+    ws = [(scale * torch.randn(s, generator=g)).to(dtype) for s in ((E, H, D), (E, H), (E, H, D), (E, H), (E, D, H), (E, D))]
+    got = moe.grouped_expert_mlp_inference(x.to(device), experts.to(device), torch.from_numpy(offsets).to(device),
+                                           *(w.to(device) for w in ws))
+    f = [w.double().numpy() for w in ws]
+    x64 = x.double().numpy()
+    want = oracle.grouped_mlp(x64, experts.numpy(), offsets, *f)
+    u = 2.0**-24
+    half_ulp = {torch.float32: u, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+    bound = half_ulp * np.abs(want) + 2.0**-25  # and half of fp16's smallest step
+    for e in range(E):
+        s = slice(int(offsets[e]), int(offsets[e + 1]))
+        xe = x64[s]
+        gate, value = xe @ f[0][e].T + f[1][e], xe @ f[2][e].T + f[3][e]
+        eg = 4 * np.sqrt(D) * u * (np.abs(xe) @ np.abs(f[0][e]).T + np.abs(f[1][e]))
+        ev = 4 * np.sqrt(D) * u * (np.abs(xe) @ np.abs(f[2][e]).T + np.abs(f[3][e]))
+        act = gate / (1 + np.exp(-gate))
+        eh = 1.1 * eg * np.abs(value) + np.abs(act) * ev + 16 * u * np.abs(act * value)
+        w = np.abs(f[4][e]).T
+        bound[s] += eh @ w + 4 * np.sqrt(H) * u * (np.abs(act * value) @ w + np.abs(f[5][e]))
+    return (x, experts, offsets, ws), got, want, bound
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sizes, D, H", [
+    ((1,), 1, 1), ((5, 0, 2), 7, 9), ((64, 65, 0, 1), 31, 65), ((130, 97, 128, 127), 33, 64), ((300, 1), 72, 200),
+    ((129, 0, 257, 90), 264, 130), ((3, 1, 2), 1000, 300), ((200, 150), 100, 513),
+])
+def test_grouped_mlp_any_type_and_shape(device, dtype, sizes, D, H):
+    """Tile edges (64 and 128 rows, 64 and 128 columns), K remainders and unaligned rows of the any-shape path."""
+
+    (_, _, offsets, _), got, want, bound = any_shape_mlp(device, dtype, sizes, D, H)
+    err = np.abs(got.double().cpu().numpy() - want)
+    assert (err <= bound).all(), float((err / np.maximum(bound, 1e-300)).max())
+    assert not got[int(offsets[-1]):].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_grouped_mlp_any_shape_subnormals_and_infinities(device, dtype):
+    """Weights far below one keep their low bits through the splits (fp16 subnormals among them), and
+    rows with infinities, NaN or values past bf16's range give what a plain multiply-add chain gives."""
+
+    _, got, want, bound = any_shape_mlp(device, dtype, (70, 40), 96, 80, scale=2.0**-13, seed=5)
+    err = np.abs(got.double().cpu().numpy() - want)
+    assert (err <= bound).all(), float((err / bound).max())
+    (x, experts, offsets, ws), clean, _, _ = any_shape_mlp(device, dtype, (70, 40), 96, 80, seed=6)
+    big = 65504.0 if dtype == torch.float16 else 3.4e38
+    x[3, 5], x[9, 0], x[20, 95], x[100, 1] = float("inf"), float("nan"), -float("inf"), big
+    ws[0][0] = ws[0][0].abs()  # an infinite input then keeps its gate infinite instead of NaN
+    ws[2][0] = ws[2][0].abs()
+    ws[4][0] = ws[4][0].abs()
+    got = moe.grouped_expert_mlp_inference(x.to(device), experts.to(device), torch.from_numpy(offsets).to(device),
+                                           *(w.to(device) for w in ws)).cpu()
+    assert torch.isposinf(got[3]).all() and torch.isnan(got[9]).all() and torch.isnan(got[20]).all()
+    rows = [r for r in range(70, 110) if r != 100]
+    assert torch.equal(got[rows], clean.cpu()[rows])
+    assert not torch.isfinite(got[100]).all() or dtype == torch.float16
