@@ -111,6 +111,27 @@ int koemi_surprise_rows_backward(const float* logits, const void* bias, const in
                                  float* grad_logits, int64_t rows, int64_t vocab, float log_vocab,
                                  int dtype, koemi_stream_t stream);
 
+/* causal_surprise (think/surprise_kernel.cu:194-328) with the content head's
+ * product inside: prior [rows, width], weight [vocab, width], bias [vocab] and
+ * surprise [rows] of `dtype` (F32/F16/BF16), fp32 accumulation of exact
+ * products. stats fp32 [3, rows] (maximum, sum of exponentials and negative
+ * log-likelihood of each row's logits) is what the backward reads. The workspace
+ * (where the vocabulary takes several tiles) holds their parts of them. */
+size_t koemi_surprise_head_forward_workspace_bytes(int64_t rows, int64_t vocab);
+int koemi_surprise_head_forward(const void* prior, const void* weight, const void* bias, const int64_t* target_ids,
+                                const uint8_t* valid_mask, void* surprise, float* stats, int64_t rows, int64_t width,
+                                int64_t vocab, float log_vocab, int dtype, void* workspace, size_t workspace_bytes,
+                                koemi_stream_t stream);
+/* Gradients of the same for an upstream gradient grad_surprise [rows] of
+ * `dtype`: grad_prior, grad_weight and grad_bias of `dtype`. The workspace
+ * holds the logits' gradient (fp32) and partial sums. */
+size_t koemi_surprise_head_backward_workspace_bytes(int64_t rows, int64_t width, int64_t vocab);
+int koemi_surprise_head_backward(const void* prior, const void* weight, const void* bias, const int64_t* target_ids,
+                                 const uint8_t* valid_mask, const float* stats, const void* grad_surprise,
+                                 void* grad_prior, void* grad_weight, void* grad_bias, int64_t rows, int64_t width,
+                                 int64_t vocab, float log_vocab, int dtype, void* workspace, size_t workspace_bytes,
+                                 koemi_stream_t stream);
+
 /* Salience admission with a fixed threshold (model/network.py:349):
  * admission[i] = valid[i] && surprise[i] > threshold. surprise of `dtype`. */
 int koemi_admission_threshold(const void* surprise, const uint8_t* valid_mask, uint8_t* admission,

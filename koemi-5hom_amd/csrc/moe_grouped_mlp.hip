@@ -20,6 +20,7 @@
 #include "mfma_stage.hpp"
 #include "split_gemm.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace koemi {
@@ -590,17 +591,17 @@ __global__ __launch_bounds__(256) void split_fixup_kernel(
 // hidden activations stay fp32 (GEMM 2 splits them into three bf16 planes).
 // Bound by the matrix cores (one product per operand pair for 16-bit GEMM 1,
 // three to six otherwise) with the splits on the vector units beside them.
-// 5400 pairs over 12 experts, 768 -> 2000 -> 768 (both GEMMs): fp16 68 + 129 us
-// (GEMM 1 at 540 TFLOP/s, GEMM 2 at 143, 715 counting its five products), fp32
-// 210 + 149 us (176 TFLOP/s, 1.06 PFLOP/s counting six); a thread per output
+// 5400 pairs over 12 experts, 768 -> 2000 -> 768 (both GEMMs): fp16 59 + 118 us
+// (GEMM 1 at 620 TFLOP/s, GEMM 2 at 156, 780 counting its five products), fp32
+// 199 + 138 us (185 TFLOP/s, 1.1 PFLOP/s counting six); a thread per output
 // with a scalar multiply-add chain, as these types ran before, took 107 and
-// 181 ms. bf16 1000 -> 1400 -> 1000: 70 + 83 us against 89 ms.
-template <bool GLU, typename TA, typename TW, int BM, int BN, bool VEC>
+// 181 ms. bf16 1000 -> 1400 -> 1000: 63 + 76 us against 89 ms.
+template <bool GLU, typename TA, typename TW, int BM, int BN, int BYTES>
 __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kernel(
     const TA* __restrict__ A, const TW* __restrict__ W0, const TW* __restrict__ W1, const TW* __restrict__ bias0,
     const TW* __restrict__ bias1, void* __restrict__ out, const int32_t* __restrict__ slot_expert,
     const int64_t* __restrict__ slot_row, const int64_t* __restrict__ slot_end, int64_t n_out, int64_t K,
-    int64_t lda, int64_t ldc, int64_t max_slots, int64_t n_tiles) {
+    int64_t lda, int64_t ldc, int64_t max_slots, int64_t n_tiles, int vec_out) {
     static_assert(!GLU || BN == 128, "a wave holds one gate and one value tile of the same hidden units");
     using G = split_gemm::Tile<TA, TW, BM, BN>;
     __shared__ __attribute__((aligned(16))) char lds[G::kLdsBytes];
@@ -625,7 +626,7 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
     const TW* w0 = W0 + static_cast<int64_t>(e) * n_out * K;
     const TW* w1 = W1 + static_cast<int64_t>(e) * n_out * K;
     G tile;
-    tile.template run<VEC>(
+    tile.template run<GLU ? BYTES : 16, BYTES>(  // H rows are padded to 32 bytes
              lds, lda, K, 0, (K + G::BK - 1) / G::BK * G::BK,
              [&](int r) { return A + min(row0 + r, row_end - 1) * lda; },
              [&](int r) {
@@ -633,45 +634,52 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
                  return w0 + min(n0 + r, n_out - 1) * K;
              },
              [&](int t) { return GLU ? t * (BN / 2) + wn * 32 : wn * (BN / 2) + t * 32; });
+    split_gemm::lds_barrier();  // the output rows pass through LDS
+    constexpr int J = GLU ? 1 : G::NT;
+    using Out = std::conditional_t<GLU, float, TW>;
+    constexpr int kRegion = split_gemm::store_bytes<Out, J>();
+    static_assert(4 * kRegion <= G::kLdsBytes, "the output regions fit the operands' LDS");
+    const int64_t first = n0 + (GLU ? wn * 32 : wn * (BN / 2));  // the wave's first column
+    // H rows are padded to a multiple of 8 columns, zeros past n_out
+    const int64_t cols = (GLU ? ldc : n_out) - first;
+    const int here = static_cast<int>(min(n_out - first, int64_t(1) << 20));  // columns that exist from there
+    const TW* bias_g = bias0 + static_cast<int64_t>(e) * n_out;
+    const TW* bias_v = bias1 + static_cast<int64_t>(e) * n_out;
+    float b0[J][16], b1[16];  // the same for every m-tile
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int64_t c = min(first + j * 32 + split_gemm::acc_column(v), n_out - 1);
+            b0[j][v] = to_f32(bias_g[c]);
+            if constexpr (GLU) b1[v] = to_f32(bias_v[c]);
+        }
 #pragma unroll
     for (int i = 0; i < G::MT; ++i) {
-        const int64_t row = row0 + wm * (BM / 2) + i * 32 + (lane_id() & 31);
-        if (row >= row_end) continue;
-        const TA* a = A + row * lda;
+        const int64_t block_row = row0 + wm * (BM / 2) + i * 32;
+        float o[J][16];
 #pragma unroll
-        for (int j = 0; j < (GLU ? 1 : G::NT); ++j) {
-            const int64_t first = n0 + (GLU ? wn * 32 : wn * (BN / 2) + j * 32);
+        for (int j = 0; j < J; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; v += 4) {
-                const int64_t col = first + split_gemm::acc_column(v);  // four columns from here
-                float o[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int64_t c = col + q;
-                    o[q] = 0.0f;
-                    if (c >= n_out) continue;
-                    const float b0 = to_f32(bias0[static_cast<int64_t>(e) * n_out + c]);
-                    float x = tile.acc[i][j][v + q] + b0;
-                    if (!G::kNative && !split_gemm::finite(x)) x = split_gemm::scalar_dot(a, w0 + c * K, K, b0);
-                    o[q] = x;
-                    if constexpr (GLU) {
-                        const float b1 = to_f32(bias1[static_cast<int64_t>(e) * n_out + c]);
-                        float u = tile.acc[i][G::NT - 1][v + q] + b1;
-                        if (!G::kNative && !split_gemm::finite(u)) u = split_gemm::scalar_dot(a, w1 + c * K, K, b1);
-                        o[q] = silu_f(x) * u;
-                    }
-                }
-                if constexpr (GLU) {
-                    // H rows are padded to a multiple of 8 columns, zeros past n_out
-                    if (col < ldc) store4(static_cast<float*>(out) + row * ldc + col, o[0], o[1], o[2], o[3]);
-                } else {
-                    TW* y = static_cast<TW*>(out) + row * ldc + col;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (col + q < n_out) y[q] = from_f32<TW>(o[q]);
-                }
+            for (int v = 0; v < 16; ++v) {
+                const float x = tile.acc[i][j][v] + b0[j][v];
+                if constexpr (GLU) o[j][v] = silu_f(x) * (tile.acc[i][G::NT - 1][v] + b1[v]);
+                else o[j][v] = x;
+                if (j * 32 + split_gemm::acc_column(v) >= here) o[j][v] = 0.0f;
             }
-        }
+        Out* y = static_cast<Out*>(out) + block_row * ldc + first;
+        split_gemm::store_rows<Out, J>(lds + (threadIdx.x / kWave) * kRegion, o, y, ldc, row_end - block_row, cols,
+                                       GLU || vec_out);
+        if constexpr (!G::kNative)
+            split_gemm::fix_not_finite(o, [&](int j, int v) {
+                const int r = lane_id() & 31, c = j * 32 + split_gemm::acc_column(v);
+                if (block_row + r >= row_end) return;
+                const TA* a = A + (block_row + r) * lda;
+                float x = split_gemm::scalar_dot(a, w0 + (first + c) * K, K, to_f32(bias_g[first + c]));
+                if constexpr (GLU)
+                    x = silu_f(x) * split_gemm::scalar_dot(a, w1 + (first + c) * K, K, to_f32(bias_v[first + c]));
+                y[r * ldc + c] = from_f32<Out>(x);
+            });
     }
 }
 
@@ -937,27 +945,36 @@ int run_any(const void* x, const int64_t* offsets, const void* Wg, const void* b
     const T* wg = static_cast<const T*>(Wg);
     const T* wv = static_cast<const T*>(Wv);
     const T* wo = static_cast<const T*>(Wo);
-    const auto launch = [&](auto vec_kernel, auto kernel, bool vec, const auto* a, const T* w0, const T* w1, const void* b0,
-                            const void* b1, void* out, int64_t n_out, int64_t K, int64_t lda, int64_t ldc, int64_t n_tiles,
-                            const char* what) {
-        hipLaunchKernelGGL(vec ? vec_kernel : kernel, dim3(static_cast<unsigned>((ws.max_slots * n_tiles + 7) / 8 * 8)),
+    const auto launch = [&](auto kernel, const auto* a, const T* w0, const T* w1, const void* b0, const void* b1, void* out,
+                            int64_t n_out, int64_t K, int64_t lda, int64_t ldc, int64_t n_tiles, const char* what) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((ws.max_slots * n_tiles + 7) / 8 * 8)),
                            dim3(split_gemm::kThreads), 0, s, a, w0, w1, static_cast<const T*>(b0),
                            static_cast<const T*>(b1), out, slot_expert, slot_row, slot_end, n_out, K, lda, ldc,
-                           ws.max_slots, n_tiles);
+                           ws.max_slots, n_tiles, static_cast<int>(D % 8 == 0 && aligned(y)));
         return check_launch(what);
     };
-    st = launch(grouped_gemm_any_kernel<true, T, T, BM, 128, true>, grouped_gemm_any_kernel<true, T, T, BM, 128, false>,
-                D % 8 == 0 && aligned(x) && aligned(Wg) && aligned(Wv), static_cast<const T*>(x), wg, wv, bg, bv, H, Hd, D,
-                D, ld_h, tiles1, "koemi_moe_grouped_mlp(hidden)");
-    if (st != KOEMI_OK) return st;
-    const auto second = [&](auto vec_kernel, auto kernel) {
-        return launch(vec_kernel, kernel, Hd % 8 == 0 && aligned(Wo), H, wo, wo, bo, bo, y, D, Hd, ld_h, D, tiles2,
-                      "koemi_moe_grouped_mlp(output)");
+    using split_gemm::load_bytes;
+    const auto first = [&](auto kernel) {
+        return launch(kernel, static_cast<const T*>(x), wg, wv, bg, bv, H, Hd, D, D, ld_h, tiles1,
+                      "koemi_moe_grouped_mlp(hidden)");
     };
-    st = narrow ? second(grouped_gemm_any_kernel<false, float, T, BM, 64, true>,
-                         grouped_gemm_any_kernel<false, float, T, BM, 64, false>)
-                : second(grouped_gemm_any_kernel<false, float, T, BM, 128, true>,
-                         grouped_gemm_any_kernel<false, float, T, BM, 128, false>);
+    const int bytes1 = std::min(load_bytes<T>(x, D), std::min(load_bytes<T>(Wg, D), load_bytes<T>(Wv, D)));
+    st = bytes1 == 16  ? first(grouped_gemm_any_kernel<true, T, T, BM, 128, 16>)
+         : bytes1 == 8 ? first(grouped_gemm_any_kernel<true, T, T, BM, 128, 8>)
+                       : first(grouped_gemm_any_kernel<true, T, T, BM, 128, 0>);
+    if (st != KOEMI_OK) return st;
+    const auto second = [&](auto kernel) {
+        return launch(kernel, H, wo, wo, bo, bo, y, D, Hd, ld_h, D, tiles2, "koemi_moe_grouped_mlp(output)");
+    };
+    const int bytes2 = load_bytes<T>(Wo, Hd);
+    if (narrow)
+        st = bytes2 == 16  ? second(grouped_gemm_any_kernel<false, float, T, BM, 64, 16>)
+             : bytes2 == 8 ? second(grouped_gemm_any_kernel<false, float, T, BM, 64, 8>)
+                           : second(grouped_gemm_any_kernel<false, float, T, BM, 64, 0>);
+    else
+        st = bytes2 == 16  ? second(grouped_gemm_any_kernel<false, float, T, BM, 128, 16>)
+             : bytes2 == 8 ? second(grouped_gemm_any_kernel<false, float, T, BM, 128, 8>)
+                           : second(grouped_gemm_any_kernel<false, float, T, BM, 128, 0>);
     if (st != KOEMI_OK) return st;
     hipLaunchKernelGGL(zero_tail_rows_kernel<T>, dim3(tail_blocks(P)), dim3(256), 0, s, static_cast<T*>(y),
                        offsets + E, P, D);

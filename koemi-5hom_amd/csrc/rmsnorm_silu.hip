@@ -7,6 +7,7 @@
 // butterfly over the row's lanes, and y = silu(x * inv * w) is produced from
 // the same registers, so x is read from HBM exactly once and y written once.
 // Rows whose width does not fit that layout use a generic block-per-row path.
+#include "column_sum.hpp"
 #include "common.hpp"
 
 namespace koemi {
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256) void rmsnorm_silu_fwd_block(const T* __restric
 // dx = inv * d * w - x * inv^3 / H * sum_c(d_c w_c x_c),  d = g * silu'(x inv w),
 // dw = sum_rows d * x * inv. Stage 1 walks the rows with a fixed number of
 // workgroups, each keeping its share of dw in registers and writing it once as
-// an fp32 partial row; stage 2 adds the partial rows in a fixed order. No
+// an fp32 partial row; stage 2 (column_sum.hpp) adds the partial rows in a fixed order. No
 // atomics: the same bits on every run.
 constexpr int kBwdMaxBlocks = 1024;  // 4 workgroups per CU in flight; the partial rows stay in L2
 
@@ -394,38 +395,6 @@ __global__ __launch_bounds__(256) void rmsnorm_silu_bwd_wide(
     }
 }
 
-// Stage 2: dw[c] = sum over the partial rows. A workgroup takes 32 columns (one
-// 128-byte line of every partial row) and its 32 row lanes stride the partial
-// rows, eight loads in flight each; the row lanes' sums meet in LDS in order.
-// Bound by latency (the partials sit in L2). 1024 x 512: 240 -> 4.8 us (two
-// workgroups walking all partial rows one by one before).
-constexpr int kBwdCols = 32, kBwdLanes = 32;
-template <typename T>
-__global__ __launch_bounds__(kBwdCols * kBwdLanes) void rmsnorm_silu_bwd_stage2(
-    const float* __restrict__ partial, T* __restrict__ dw, int64_t blocks, int H) {
-    __shared__ float sums[kBwdLanes][kBwdCols + 1];
-    const int col = threadIdx.x % kBwdCols, lane = threadIdx.x / kBwdCols;
-    const int c = blockIdx.x * kBwdCols + col;
-    const float* p = partial + min(c, H - 1);
-    float acc = 0.0f;
-    for (int64_t b0 = lane; b0 < blocks; b0 += 8 * kBwdLanes) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = p[min(b0 + i * kBwdLanes, blocks - 1) * H];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc += b0 + i * kBwdLanes < blocks ? v[i] : 0.0f;
-    }
-    sums[lane][col] = acc;
-    __syncthreads();
-    // thread (lane, col) of the first wave pair: a fixed tree over the row lanes
-#pragma unroll
-    for (int half = kBwdLanes / 2; half > 0; half >>= 1) {
-        if (lane < half) sums[lane][col] += sums[lane + half][col];
-        __syncthreads();
-    }
-    if (lane == 0 && c < H) dw[c] = from_f32<T>(sums[0][col]);
-}
-
 template <typename T>
 int launch_forward(const void* x, const void* w, void* y, float* inv, int64_t rows, int64_t H,
                    float eps, hipStream_t stream) {
@@ -527,8 +496,7 @@ int launch_backward(const void* g, const void* x, const void* w, const float* in
                            inv, dxp, partial, rows, Hi);
     int st = check_launch("koemi_rmsnorm_silu_backward");
     if (st != KOEMI_OK) return st;
-    hipLaunchKernelGGL(rmsnorm_silu_bwd_stage2<T>, dim3(grid_for(H, kBwdCols)), dim3(kBwdCols * kBwdLanes), 0, stream,
-                       partial, static_cast<T*>(dw), blocks, Hi);
+    launch_column_sum(partial, static_cast<T*>(dw), blocks, H, stream);
     return check_launch("koemi_rmsnorm_silu_backward");
 }
 

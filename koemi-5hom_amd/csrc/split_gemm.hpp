@@ -47,19 +47,33 @@ struct Octet {
     }
 };
 
-// K values [k, k + 8) of a row. VEC: K is a multiple of 8 and rows are 16-byte
-// aligned, so an octet is all in or all out and is read by 16-byte loads;
-// otherwise element by element. What lies past K is read at a clamped address
-// and cleared by clear_past, which the caller runs when it uses the octet: a
-// select beside the load would wait for it. K >= 1.
-template <bool VEC, typename T>
+// Bytes per load that the rows of an operand allow: 16 or 8 where every row starts
+// aligned to them (the base and the row length), else kElementLoads.
+constexpr int kElementLoads = 0;
+template <typename T>
+inline int load_bytes(const void* base, int64_t K) {
+    const uintptr_t both = reinterpret_cast<uintptr_t>(base) | static_cast<uintptr_t>(K * static_cast<int64_t>(sizeof(T)));
+    return both % 16 == 0 ? 16 : both % 8 == 0 ? 8 : kElementLoads;
+}
+
+// K values [k, k + 8) of a row, in pieces of BYTES (load_bytes): a piece lies
+// within K or past it. What lies past K is read at a clamped address and cleared
+// by clear_past, which the caller runs when it uses the octet: a select beside
+// the load would wait for it. K >= 1.
+template <int BYTES, typename T>
 __device__ __forceinline__ void load_octet(Octet<T>& o, const T* __restrict__ row, int64_t k, int64_t K) {
-    if constexpr (VEC) {
-        const uint4* p = reinterpret_cast<const uint4*>(row + min(k, K - 8));
+    if constexpr (BYTES != kElementLoads) {
+        constexpr int n = BYTES / static_cast<int>(sizeof(T)), words = BYTES / 4;
 #pragma unroll
-        for (int i = 0; i < Octet<T>::kWords / 4; ++i) {
-            const uint4 v = p[i];
-            o.w[4 * i] = v.x, o.w[4 * i + 1] = v.y, o.w[4 * i + 2] = v.z, o.w[4 * i + 3] = v.w;
+        for (int i = 0; i < 8 / n; ++i) {
+            const T* p = row + min(k + i * n, K - n);
+            if constexpr (BYTES == 16) {
+                const uint4 v = *reinterpret_cast<const uint4*>(p);
+                o.w[i * words] = v.x, o.w[i * words + 1] = v.y, o.w[i * words + 2] = v.z, o.w[i * words + 3] = v.w;
+            } else {
+                const uint2 v = *reinterpret_cast<const uint2*>(p);
+                o.w[i * words] = v.x, o.w[i * words + 1] = v.y;
+            }
         }
     } else if constexpr (sizeof(T) == 4) {
 #pragma unroll
@@ -71,13 +85,36 @@ __device__ __forceinline__ void load_octet(Octet<T>& o, const T* __restrict__ ro
                      static_cast<uint32_t>(__builtin_bit_cast(uint16_t, row[min(k + 2 * i + 1, K - 1)])) << 16;
     }
 }
-template <bool VEC, typename T>
+// The same from a K-strided operand: value k of the column at p is p[k * ld].
+// tail (wave-uniform): the step reaches past K.
+template <typename T>
+__device__ __forceinline__ void load_octet_strided(Octet<T>& o, const T* __restrict__ p, int64_t ld, int64_t k, int64_t K,
+                                                   bool tail) {
+    T e[8];
+    if (tail) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) e[i] = p[min(k + i, K - 1) * ld];
+    } else {
+        const T* q = p + k * ld;
+#pragma unroll
+        for (int i = 0; i < 8; ++i, q += ld) e[i] = *q;
+    }
+#pragma unroll
+    for (int i = 0; i < Octet<T>::kWords; ++i) {
+        if constexpr (sizeof(T) == 4) o.w[i] = __float_as_uint(e[i]);
+        else
+            o.w[i] = __builtin_bit_cast(uint16_t, e[2 * i]) |
+                     static_cast<uint32_t>(__builtin_bit_cast(uint16_t, e[2 * i + 1])) << 16;
+    }
+}
+template <typename T>
 __device__ __forceinline__ void clear_past(Octet<T>& o, int64_t k, int64_t K) {
     constexpr int kPerWord = 4 / static_cast<int>(sizeof(T));
 #pragma unroll
     for (int i = 0; i < Octet<T>::kWords; ++i) {
-        if (VEC ? k >= K : k + i * kPerWord >= K) o.w[i] = 0;
-        else if (!VEC && kPerWord == 2 && k + i * 2 + 1 >= K) o.w[i] &= 0xffffu;
+        const bool out = k + i * kPerWord >= K;
+        if (kPerWord == 2) o.w[i] &= out ? 0u : k + i * 2 + 1 >= K ? 0xffffu : 0xffffffffu;
+        else o.w[i] = out ? 0u : o.w[i];
     }
 }
 
@@ -107,8 +144,12 @@ __device__ __forceinline__ uint4 take_plane(float (&f)[8]) {
 // split (eight MFMAs a wave and step otherwise), else 32. An LDS row is BK
 // 16-bit values of one plane; 16-byte group g of row r sits at group
 // g ^ swizzle(r), so that the sixteen rows read by sixteen consecutive lanes
-// fill 256 distinct bytes of banks.
-template <typename TA, typename TB, int BM, int BN>
+// fill 256 distinct bytes of banks. A_STRIDED / B_STRIDED: the operand is stored
+// K-major ([K, rows]); its octets are gathered by eight loads, each coalesced
+// over the rows of consecutive lanes.
+// DEPTH: K steps whose operands are on their way in registers; more than one where
+// a launch has too few tiles to hide the loads behind other workgroups.
+template <typename TA, typename TB, int BM, int BN, bool A_STRIDED = false, bool B_STRIDED = false, int DEPTH = 1>
 struct Tile {
     static constexpr int NA = planes<TA, TB>(), NB = planes<TB, TA>();
     static constexpr bool kNative = NA == 1 && NB == 1;
@@ -117,6 +158,7 @@ struct Tile {
     static constexpr int kGroups = BK / 8;
     static constexpr int MT = BM / 64, NT = BN / 64;  // 32 x 32 tiles of a wave
     static constexpr int kRowBytes = BK * 2;
+    static constexpr int kSets = kNative ? 2 : 1;  // fragment sets held by a wave
     static constexpr int kLdsBytes = (NA * BM + NB * BN) * kRowBytes;
     static constexpr int OA = BM * kGroups / kThreads, OB = BN * kGroups / kThreads;  // octets per thread
     static_assert(OA >= 1 && OB >= 1, "a thread stages at least one octet of each operand");
@@ -126,21 +168,34 @@ struct Tile {
 
     f32x16 acc[MT][NT];
 
+    // Octet i of the thread, of an operand of R rows: its row and K group. Eight
+    // or four consecutive threads share a row of a K-contiguous operand (its
+    // 16-byte pieces), consecutive threads take consecutive rows of a strided one.
+    template <int R, bool STRIDED>
+    __device__ static int octet_row(int i) {
+        return STRIDED ? (threadIdx.x + i * kThreads) % R : (threadIdx.x + i * kThreads) / kGroups;
+    }
+    template <int R, bool STRIDED>
+    __device__ static int octet_group(int i) {
+        return STRIDED ? (threadIdx.x + i * kThreads) / R : threadIdx.x % kGroups;
+    }
+
     // a_row(r), b_row(r): pointers to row r of the block tile's operands, for
-    // rows this thread stages (already clamped to rows that exist).
+    // rows this thread stages (already clamped to rows that exist), read in pieces of
+    // A_BYTES and B_BYTES; a strided
+    // operand's row is the column whose value k lies at k * a_ld (b_ld).
     // b_first(t): the block tile's B row where this wave's n-tile t starts.
-    template <bool VEC, typename ARow, typename BRow, typename BFirst>
+    template <int A_BYTES, int B_BYTES, typename ARow, typename BRow, typename BFirst>
     __device__ __forceinline__ void run(char* lds, int64_t KA, int64_t KB, int64_t k_begin, int64_t k_end, ARow a_row,
-                                        BRow b_row, BFirst b_first) {
-        const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+                                        BRow b_row, BFirst b_first, int64_t a_ld = 1, int64_t b_ld = 1) {
+        const int lane = lane_id(), wave = threadIdx.x / kWave;
         const int wm = wave >> 1;
         const TA* ap[OA];
         const TB* bp[OB];
 #pragma unroll
-        for (int i = 0; i < OA; ++i) ap[i] = a_row((tid + i * kThreads) / kGroups);
+        for (int i = 0; i < OA; ++i) ap[i] = a_row(octet_row<BM, A_STRIDED>(i));
 #pragma unroll
-        for (int i = 0; i < OB; ++i) bp[i] = b_row((tid + i * kThreads) / kGroups);
-        const int g = tid % kGroups;  // kThreads is a multiple of kGroups: the same group in every octet
+        for (int i = 0; i < OB; ++i) bp[i] = b_row(octet_row<BN, B_STRIDED>(i));
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -148,43 +203,57 @@ struct Tile {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
         char* const lds_b = lds + NA * BM * kRowBytes;
-        Octet<TA> ao[OA];
-        Octet<TB> bo[OB];
-        auto load = [&](int64_t k0) {
+        Octet<TA> a_ring[DEPTH][OA];
+        Octet<TB> b_ring[DEPTH][OB];
+        auto load = [&](int64_t k0, Octet<TA> (&ao)[OA], Octet<TB> (&bo)[OB]) {
 #pragma unroll
-            for (int i = 0; i < OA; ++i) load_octet<VEC>(ao[i], ap[i], k0 + g * 8, KA);
+            for (int i = 0; i < OA; ++i) {
+                const int64_t k = k0 + octet_group<BM, A_STRIDED>(i) * 8;
+                if constexpr (A_STRIDED) load_octet_strided(ao[i], ap[i], a_ld, k, KA, k0 + BK > KA);
+                else load_octet<A_BYTES>(ao[i], ap[i], k, KA);
+            }
 #pragma unroll
-            for (int i = 0; i < OB; ++i) load_octet<VEC>(bo[i], bp[i], k0 + g * 8, KB);
+            for (int i = 0; i < OB; ++i) {
+                const int64_t k = k0 + octet_group<BN, B_STRIDED>(i) * 8;
+                if constexpr (B_STRIDED) load_octet_strided(bo[i], bp[i], b_ld, k, KB, k0 + BK > KB);
+                else load_octet<B_BYTES>(bo[i], bp[i], k, KB);
+            }
         };
-        load(k_begin);
-        for (int64_t k0 = k_begin; k0 < k_end; k0 += BK) {
+        auto step = [&](int64_t k0, Octet<TA> (&ao)[OA], Octet<TB> (&bo)[OB]) {
             lds_barrier();  // every wave is done with the previous step's planes
             if (k0 + BK > KA || k0 + BK > KB) {  // only the last step reaches past K
 #pragma unroll
-                for (int i = 0; i < OA; ++i) clear_past<VEC>(ao[i], k0 + g * 8, KA);
+                for (int i = 0; i < OA; ++i) clear_past(ao[i], k0 + octet_group<BM, A_STRIDED>(i) * 8, KA);
 #pragma unroll
-                for (int i = 0; i < OB; ++i) clear_past<VEC>(bo[i], k0 + g * 8, KB);
+                for (int i = 0; i < OB; ++i) clear_past(bo[i], k0 + octet_group<BN, B_STRIDED>(i) * 8, KB);
             }
-            stage<TA, NA, OA, BM>(lds, ao, g);
-            stage<TB, NB, OB, BN>(lds_b, bo, g);
-            if (k0 + BK < k_end) load(k0 + BK);
+            stage<TA, NA, OA, BM, A_STRIDED>(lds, ao);
+            stage<TB, NB, OB, BN, B_STRIDED>(lds_b, bo);
+            if (k0 + DEPTH * BK < k_end) load(k0 + DEPTH * BK, ao, bo);
             lds_barrier();
-#pragma unroll
-            for (int kk = 0; kk < BK / 16; ++kk) {
+            // the fragments of K group kk + 1 are read under the products of group kk
+            // where two sets fit the registers (one product each)
+            uint4 af[kSets][NA][MT], bf[kSets][NB][NT];
+            auto read = [&](int kk, int set) {
                 const int fg = kk * 2 + (lane >> 5);
-                uint4 af[NA][MT], bf[NB][NT];
 #pragma unroll
                 for (int p = 0; p < NA; ++p)
 #pragma unroll
                     for (int t = 0; t < MT; ++t)
-                        af[p][t] = *reinterpret_cast<const uint4*>(
+                        af[set][p][t] = *reinterpret_cast<const uint4*>(
                             lds + p * BM * kRowBytes + at(wm * (BM / 2) + t * 32 + (lane & 31), fg));
 #pragma unroll
                 for (int p = 0; p < NB; ++p)
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
-                        bf[p][t] = *reinterpret_cast<const uint4*>(lds_b + p * BN * kRowBytes +
-                                                                  at(b_first(t) + (lane & 31), fg));
+                        bf[set][p][t] = *reinterpret_cast<const uint4*>(lds_b + p * BN * kRowBytes +
+                                                                       at(b_first(t) + (lane & 31), fg));
+            };
+            read(0, 0);
+#pragma unroll
+            for (int kk = 0; kk < BK / 16; ++kk) {
+                const int set = kk % kSets;
+                if (kSets == 2 && kk + 1 < BK / 16) read(kk + 1, 1 - set);
                 // smallest products first
 #pragma unroll
                 for (int s = 2; s >= 0; --s)
@@ -198,24 +267,33 @@ struct Tile {
                             for (int j = 0; j < NT; ++j) {
                                 if constexpr (kHalf)
                                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                        __builtin_bit_cast(f16x8, bf[q][j]), __builtin_bit_cast(f16x8, af[p][i]),
-                                        acc[i][j], 0, 0, 0);
+                                        __builtin_bit_cast(f16x8, bf[set][q][j]),
+                                        __builtin_bit_cast(f16x8, af[set][p][i]), acc[i][j], 0, 0, 0);
                                 else
                                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                                        __builtin_bit_cast(bf16x8, bf[q][j]), __builtin_bit_cast(bf16x8, af[p][i]),
-                                        acc[i][j], 0, 0, 0);
+                                        __builtin_bit_cast(bf16x8, bf[set][q][j]),
+                                        __builtin_bit_cast(bf16x8, af[set][p][i]), acc[i][j], 0, 0, 0);
                             }
                     }
+                if (kSets == 1 && kk + 1 < BK / 16) read(kk + 1, 0);
             }
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+            if (k_begin + d * BK < k_end) load(k_begin + d * BK, a_ring[d], b_ring[d]);
+        for (int64_t k0 = k_begin; k0 < k_end; k0 += DEPTH * BK) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d)
+                if (k0 + d * BK < k_end) step(k0 + d * BK, a_ring[d], b_ring[d]);
         }
     }
 
   private:
-    template <typename T, int P, int O, int R>
-    __device__ static __forceinline__ void stage(char* lds, Octet<T> (&o)[O], int g) {
+    template <typename T, int P, int O, int R, bool STRIDED>
+    __device__ static __forceinline__ void stage(char* lds, Octet<T> (&o)[O]) {
 #pragma unroll
         for (int i = 0; i < O; ++i) {
-            const int off = at((threadIdx.x + i * kThreads) / kGroups, g);
+            const int off = at(octet_row<R, STRIDED>(i), octet_group<R, STRIDED>(i));
             if constexpr (P == 1) {
                 *reinterpret_cast<uint4*>(lds + off) = make_uint4(o[i].w[0], o[i].w[1], o[i].w[2], o[i].w[3]);
             } else {
@@ -235,10 +313,85 @@ __device__ __forceinline__ int acc_column(int v) { return 8 * (v / 4) + 4 * (lan
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) < __builtin_inff(); }
 
-// start + sum_k a[k] b[k] as one fp32 multiply-add chain.
+// Runs fix(j, v) for every output of this lane that is not finite, after its
+// stores have left: a rolled loop over a bit mask, so that the rare case costs the
+// kernel no registers.
+template <int J, typename Fix>
+__device__ __forceinline__ void fix_not_finite(const float (&o)[J][16], Fix fix) {
+    static_assert(J * 16 <= 64, "one bit per output");
+    uint64_t mask = 0;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mask |= finite(o[j][v]) ? 0ull : 1ull << (j * 16 + v);
+    if (__builtin_expect(__ballot(mask != 0) == 0, 1)) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    while (mask) {
+        const int b = __builtin_ctzll(mask);
+        mask &= mask - 1;
+        fix(b / 16, b % 16);
+    }
+}
+
+// Stores a wave's 32 x (32 J) outputs as full rows: o[j][v] is row lane % 32,
+// column 32 j + acc_column(v) of the wave's block, whose first element goes to
+// out[0] (rows ld apart). They pass through the wave's own LDS region of
+// store_bytes<T, J>() and leave in 16-byte pieces of whole rows (without it every
+// store would touch 32 rows). rows, cols: how many of them exist. VEC: rows of
+// out start 16-byte aligned and cols is a multiple of 8; otherwise the pieces are
+// stored element by element. The caller has joined the workgroup's waves after
+// the tile's last LDS reads.
+template <typename T, int J>
+constexpr int store_bytes() {
+    return 32 * (32 * J * static_cast<int>(sizeof(T)) + 16);
+}
+template <typename T, int J>
+__device__ __forceinline__ void store_rows(char* region, const float (&o)[J][16], T* __restrict__ out, int64_t ld,
+                                           int64_t rows, int64_t cols, bool vec) {
+    constexpr int kRow = 32 * J * static_cast<int>(sizeof(T)) + 16, kPieces = (kRow - 16) / 16;
+    constexpr int kPer = 16 / static_cast<int>(sizeof(T));
+    const int lane = lane_id();
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            union {
+                T e[4];
+                uint32_t w[sizeof(T)];
+            } u;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) u.e[q] = from_f32<T>(o[j][v + q]);
+            char* at = region + (lane & 31) * kRow + (j * 32 + acc_column(v)) * static_cast<int>(sizeof(T));
+            if constexpr (sizeof(T) == 4) *reinterpret_cast<uint4*>(at) = make_uint4(u.w[0], u.w[1], u.w[2], u.w[3]);
+            else *reinterpret_cast<uint2*>(at) = make_uint2(u.w[0], u.w[1]);
+        }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own region: in order, no barrier
+#pragma unroll
+    for (int i = 0; i < 32 * kPieces / kWave; ++i) {
+        const int piece = i * kWave + lane, r = piece / kPieces, c = piece % kPieces * kPer;
+        union {
+            uint4 raw;
+            T e[kPer];
+        } u;
+        u.raw = *reinterpret_cast<const uint4*>(region + r * kRow + c * static_cast<int>(sizeof(T)));
+        if (r >= rows) continue;
+        T* p = out + r * ld + c;
+        if (vec) {
+            if (c < cols) *reinterpret_cast<uint4*>(p) = u.raw;
+        } else {
+#pragma unroll
+            for (int q = 0; q < kPer; ++q)
+                if (c + q < cols) p[q] = u.e[q];
+        }
+    }
+    asm volatile("" ::: "memory");
+}
+
+// start + sum_k a[k a_ld] b[k b_ld] as one fp32 multiply-add chain.
 template <typename TA, typename TB>
-__device__ __noinline__ float scalar_dot(const TA* a, const TB* b, int64_t K, float start) {
-    for (int64_t k = 0; k < K; ++k) start = __builtin_fmaf(to_f32(a[k]), to_f32(b[k]), start);
+__device__ __noinline__ float scalar_dot(const TA* a, const TB* b, int64_t K, float start, int64_t a_ld = 1,
+                                         int64_t b_ld = 1) {
+    for (int64_t k = 0; k < K; ++k) start = __builtin_fmaf(to_f32(a[k * a_ld]), to_f32(b[k * b_ld]), start);
     return start;
 }
 

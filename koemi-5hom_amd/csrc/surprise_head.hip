@@ -1,0 +1,493 @@
+// Causal surprise from the prior states: the content head's product with the row
+// scoring in its epilogue, and the backward of both.
+//
+// Reference: src/koemi/cuda_kernels/think/surprise_kernel.cu:194-328 (an fp32
+// library product, a row kernel over its logits, and in the backward the
+// product again, a row kernel writing the logits' gradient and two more library
+// products). Here the logits never reach memory: a workgroup holds 64 rows x 256
+// vocabulary columns in its accumulators, scores them there and keeps (max, sum
+// of exponentials, negative log-likelihood) per row for the backward, whose
+// first kernel forms the logits again and writes their gradient G (fp32). The
+// weight gradients contract G with the states and the weights, with G split into
+// three bf16 planes that sum to it exactly (split_gemm.hpp): bf16 and fp16
+// states and weights are never widened in memory, and every product is as exact
+// as the fp32 one it replaces.
+#include "column_sum.hpp"
+#include "common.hpp"
+#include "detmath.hpp"
+#include "split_gemm.hpp"
+
+#include <algorithm>
+
+namespace koemi {
+namespace {
+
+using split_gemm::kElementLoads;
+using split_gemm::kThreads;
+
+constexpr int kRows = 64;  // rows of a head tile
+// Vocabulary columns of a head tile: 256, so that a byte vocabulary is scored in
+// one, or 64 where the 256-column tiles would leave most CUs idle, with four K steps
+// of loads in flight since no second workgroup hides them (256 rows x
+// 1024, fp32: 66 -> 26 us; a tile step costs its latency there).
+constexpr int kWide = 256, kNarrow = 64;
+constexpr int64_t kWideTiles = 128;
+
+template <typename T, int BN>
+using HeadTile = split_gemm::Tile<T, T, kRows, BN, false, false, BN == kNarrow ? 4 : 1>;
+inline int head_columns(int64_t rows, int64_t V) {
+    return (rows + kRows - 1) / kRows * ((V + kWide - 1) / kWide) < kWideTiles ? kNarrow : kWide;
+}
+
+// The logits of the workgroup's rows and vocabulary columns [v0, v0 + BN), in
+// the accumulators: lane l of wave (wm, wn) holds row 32 wm + l % 32, columns
+// BN / 2 wn + 32 j + acc_column(v). Columns past V repeat column V - 1.
+template <int BYTES, int BN, typename T>
+__device__ __forceinline__ void head_logits(HeadTile<T, BN>& tile, char* lds, const T* __restrict__ prior,
+                                            const T* __restrict__ weight, int64_t row0, int64_t v0, int64_t rows,
+                                            int64_t D, int64_t V) {
+    const int wn = threadIdx.x / kWave & 1;
+    tile.template run<BYTES, BYTES>(
+        lds, D, D, 0, (D + HeadTile<T, BN>::BK - 1) / HeadTile<T, BN>::BK * HeadTile<T, BN>::BK,
+        [&](int r) { return prior + min(row0 + r, rows - 1) * D; },
+        [&](int r) { return weight + min(v0 + r, V - 1) * D; }, [&](int t) { return wn * (BN / 2) + t * 32; });
+    if constexpr (!HeadTile<T, BN>::kNative) {
+        // a row or column with an infinity or a NaN: the plain chain's result
+        const int wm = threadIdx.x / kWave >> 1;
+        const int64_t row = min(row0 + wm * 32 + (lane_id() & 31), rows - 1);
+#pragma unroll
+        for (int j = 0; j < HeadTile<T, BN>::NT; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (!split_gemm::finite(tile.acc[0][j][v]))
+                    tile.acc[0][j][v] = split_gemm::scalar_dot(
+                        prior + row * D, weight + min(v0 + wn * (BN / 2) + j * 32 + split_gemm::acc_column(v), V - 1) * D, D,
+                        0.0f);
+    }
+}
+
+// The score of a row from its logits' maximum, sum of exponentials and target
+// logit (surprise_kernel.cu:84-134).
+template <typename T>
+__device__ __forceinline__ void finish_row(float m, float sum, float target, bool in, bool live, float log_vocab,
+                                           int64_t row, int64_t rows, T* __restrict__ out, float* __restrict__ stats) {
+#pragma clang fp contract(off)
+    const float nll = (detmath::det_logf(sum) + m) - target;
+    float s = 0.0f;
+    if (live) s = in ? 1.0f - detmath::det_expf(-nll / log_vocab) : __builtin_nanf("");
+    out[row] = from_f32<T>(s);
+    stats[row] = m;
+    stats[rows + row] = sum;
+    stats[2 * rows + row] = nll;
+}
+
+// Scores: one workgroup per 64 rows and 256 columns. A vocabulary of one tile is
+// finished here; with more, the tiles' (maximum, sum, target logit) go to `part`
+// [tiles, 3, rows] and surprise_head_finish_kernel joins them. Bound by its one round
+// of tiles (the states from HBM, the weights from L2); [32768, 512] bf16,
+// vocabulary 256: 22 us, against two casts (21), the library's fp32 product (70)
+// and the row kernel (9).
+template <typename T, int BN, int BYTES>
+__global__ __launch_bounds__(kThreads, 2) void surprise_head_forward_kernel(
+    const T* __restrict__ prior, const T* __restrict__ weight, const T* __restrict__ bias,
+    const int64_t* __restrict__ targets, const uint8_t* __restrict__ valid, T* __restrict__ out,
+    float* __restrict__ stats, float* __restrict__ part, int64_t rows, int64_t D, int64_t V, int64_t v_tiles,
+    float log_vocab) {
+#pragma clang fp contract(off)
+    using Tile = HeadTile<T, BN>;
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
+    __shared__ __attribute__((aligned(16))) float bias_sh[BN];
+    __shared__ float red[2][kRows], sums[2][kRows], target_sh[kRows];
+    const int tid = threadIdx.x, wave = tid / kWave, wm = wave >> 1, wn = wave & 1;
+    const int r = wm * 32 + (lane_id() & 31);
+    const int64_t row0 = blockIdx.x / v_tiles * kRows, tile_v = blockIdx.x % v_tiles, v0 = tile_v * BN;
+    const int64_t row = min(row0 + r, rows - 1);
+    const int64_t t = targets[row];
+    const int c0 = wn * (BN / 2) + 4 * (lane_id() >> 5);
+    if (tid < BN) bias_sh[tid] = to_f32(bias[min(v0 + tid, V - 1)]);
+    if (tid < kRows) target_sh[tid] = 0.0f;
+    Tile tile;
+    head_logits<BYTES, BN>(tile, lds, prior, weight, row0, v0, rows, D, V);  // barriers inside: the biases are visible
+    // columns from this lane's first one: the tile's valid ones and the target
+    const int here = static_cast<int>(min(V - v0, static_cast<int64_t>(BN))) - c0;
+    const int hit = t >= v0 && t < v0 + BN ? static_cast<int>(t - v0) - c0 : -1;
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int j = 0; j < Tile::NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int c = j * 32 + 8 * (v / 4) + v % 4;
+            const float z = tile.acc[0][j][v] + bias_sh[c0 + c];
+            if (c == hit) target_sh[r] = z;
+            tile.acc[0][j][v] = c < here ? z : -__builtin_inff();
+            m = fmaxf(m, tile.acc[0][j][v]);
+        }
+    m = fmaxf(m, __shfl_xor(m, 32, kWave));
+    red[wn][r] = m;  // both halves of the wave hold the row's value
+    __syncthreads();
+    m = fmaxf(red[0][r], red[1][r]);
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Tile::NT; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const float e = detmath::det_expf_nonpos(tile.acc[0][j][v] - m);
+            if (j * 32 + 8 * (v / 4) + v % 4 < here) sum = sum + e;
+        }
+    sum = sum + __shfl_xor(sum, 32, kWave);
+    sums[wn][r] = sum;
+    __syncthreads();
+    if (wn != 0 || lane_id() >= 32 || row0 + r >= rows) return;
+    sum = sums[0][r] + sums[1][r];
+    if (v_tiles == 1) {
+        finish_row(m, sum, target_sh[r], t >= 0 && t < V, valid[row] != 0, log_vocab, row, rows, out, stats);
+    } else {
+        float* p = part + tile_v * 3 * rows + row;
+        p[0] = m;
+        p[rows] = sum;
+        p[2 * rows] = target_sh[r];  // 0 in every tile but the target's
+    }
+}
+
+// Joins the vocabulary tiles of surprise_head_forward_kernel, a thread per row.
+template <typename T>
+__global__ void surprise_head_finish_kernel(const float* __restrict__ part, const int64_t* __restrict__ targets,
+                                            const uint8_t* __restrict__ valid, T* __restrict__ out,
+                                            float* __restrict__ stats, int64_t rows, int64_t V, int64_t v_tiles,
+                                            int columns, float log_vocab) {
+#pragma clang fp contract(off)
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (row >= rows) return;
+    const float* p = part + row;
+    const int64_t t = targets[row];
+    float m = -__builtin_inff(), sum = 0.0f;
+    for (int64_t i = 0; i < v_tiles; ++i) m = fmaxf(m, p[i * 3 * rows]);
+    for (int64_t i = 0; i < v_tiles; ++i) {
+        const float mi = p[i * 3 * rows], si = p[(i * 3 + 1) * rows];
+        // a tile of minus infinities alone holds a NaN sum and adds nothing to finite ones
+        if (mi > -__builtin_inff() || !(m > -__builtin_inff())) sum = sum + si * detmath::det_expf_nonpos(mi - m);
+    }
+    const bool in = t >= 0 && t < V;
+    finish_row(m, sum, in ? p[(t / columns * 3 + 2) * rows] : 0.0f, in, valid[row] != 0, log_vocab, row, rows, out, stats);
+}
+
+// d score / d logits (surprise_kernel.cu:136-192), G [rows, V] fp32:
+//   G_j = g exp(-nll / ln V) / ln V (softmax_j - [j == target]),
+// zero for invalid rows, and the workgroup's 64-row column sums of it (the
+// bias gradient's partial rows). At the sizes above 28 us, against the product
+// (70), the row kernel (37) and the column sum (27).
+template <typename T, int BN, int BYTES>
+__global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_logits_kernel(
+    const T* __restrict__ prior, const T* __restrict__ weight, const T* __restrict__ bias,
+    const int64_t* __restrict__ targets, const uint8_t* __restrict__ valid, const T* __restrict__ grad,
+    const float* __restrict__ stats, float* __restrict__ G, float* __restrict__ bias_partial, int64_t rows, int64_t D,
+    int64_t V, int64_t v_tiles, float log_vocab) {
+#pragma clang fp contract(off)
+    using Tile = HeadTile<T, BN>;
+    constexpr int J = Tile::NT < 2 ? 1 : 2;
+    constexpr int kRegion = split_gemm::store_bytes<float, J>();
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes > 4 * kRegion ? Tile::kLdsBytes : 4 * kRegion];
+    __shared__ __attribute__((aligned(16))) float bias_sh[BN];
+    __shared__ float column_sh[2][BN];
+    const int tid = threadIdx.x, wave = tid / kWave, wm = wave >> 1, wn = wave & 1;
+    const int r = wm * 32 + (lane_id() & 31);
+    const int64_t block = blockIdx.x / v_tiles, row0 = block * kRows, v0 = blockIdx.x % v_tiles * BN;
+    const int64_t row = min(row0 + r, rows - 1);
+    const int64_t t = targets[row];
+    const bool live = row0 + r < rows && valid[row] && t >= 0 && t < V;
+    const float m = stats[row], inv_sum = 1.0f / stats[rows + row];
+    const float gnll = to_f32(grad[row]) * detmath::det_expf(-stats[2 * rows + row] / log_vocab) / log_vocab;
+    const int c0 = wn * (BN / 2) + 4 * (lane_id() >> 5);
+    Tile tile;
+    if (tid < BN) bias_sh[tid] = to_f32(bias[min(v0 + tid, V - 1)]);
+    head_logits<BYTES, BN>(tile, lds, prior, weight, row0, v0, rows, D, V);
+    split_gemm::lds_barrier();  // G passes through LDS
+    const int hit = t >= v0 && t < v0 + BN ? static_cast<int>(t - v0) - c0 : -1;
+#pragma unroll
+    for (int j = 0; j < Tile::NT; j += J) {
+        float o[J][16];
+#pragma unroll
+        for (int h = 0; h < J; ++h)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int c = (j + h) * 32 + 8 * (v / 4) + v % 4;
+                const float p = detmath::det_expf_nonpos((tile.acc[0][j + h][v] + bias_sh[c0 + c]) - m) * inv_sum;
+                o[h][v] = live ? gnll * (p - (c == hit ? 1.0f : 0.0f)) : 0.0f;
+            }
+        const int64_t first = v0 + wn * (BN / 2) + j * 32;
+        split_gemm::store_rows<float, J>(lds + wave * kRegion, o, G + (row0 + wm * 32) * V + first, V,
+                                         rows - row0 - wm * 32, V - first, V % 8 == 0);
+        // lane l sums column l of the 32 rows the region still holds
+        if (lane_id() < 32 * J) {
+            const float* column = reinterpret_cast<const float*>(lds + wave * kRegion) + lane_id();
+            float acc = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 32; ++i) acc += column[i * (kRegion / 32 / 4)];
+            column_sh[wm][wn * (BN / 2) + j * 32 + lane_id()] = acc;
+        }
+        asm volatile("" ::: "memory");  // the region is rewritten by the next columns
+    }
+    __syncthreads();
+    if (tid < BN && v0 + tid < V)
+        bias_partial[block * V + v0 + tid] = column_sh[0][tid] + column_sh[1][tid];
+}
+
+// grad_prior [rows, D] = G [rows, V] W [V, D]. Bound by its few K steps (eight at a
+// vocabulary of 256) and the splits beside them. At the sizes above 50 us, against
+// 77 for the library's fp32 product and 11 for the cast of its result.
+template <typename T, int B, int BYTES>
+__global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
+    const float* __restrict__ G, const T* __restrict__ weight, T* __restrict__ grad_prior, int64_t rows, int64_t D,
+    int64_t V, int64_t d_tiles, int vec_out) {
+    constexpr int BM = B, BN = B;
+    using Tile = split_gemm::Tile<float, T, BM, BN, false, true, B == 64 ? 4 : 1>;
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
+    const int64_t row0 = blockIdx.x / d_tiles * BM, d0 = blockIdx.x % d_tiles * BN;
+    const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
+    Tile tile;
+    tile.template run<BYTES, kElementLoads>(
+        lds, V, V, 0, (V + Tile::BK - 1) / Tile::BK * Tile::BK,
+        [&](int r) { return G + min(row0 + r, rows - 1) * V; }, [&](int r) { return weight + min(d0 + r, D - 1); },
+        [&](int t) { return wn * (BN / 2) + t * 32; }, 1, D);
+    split_gemm::lds_barrier();  // the output rows pass through LDS
+    constexpr int J = Tile::NT < 2 ? 1 : 2;
+    constexpr int kRegion = split_gemm::store_bytes<T, J>();
+    static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
+#pragma unroll
+    for (int i = 0; i < Tile::MT; ++i) {
+        const int64_t block_row = row0 + wm * (BM / 2) + i * 32;
+#pragma unroll
+        for (int j0 = 0; j0 < Tile::NT; j0 += J) {
+            const int64_t first = d0 + wn * (BN / 2) + j0 * 32;
+            float o[J][16];
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[j][v] = tile.acc[i][j0 + j][v];
+            T* out = grad_prior + block_row * D + first;
+            split_gemm::store_rows<T, J>(lds + wave * kRegion, o, out, D, rows - block_row, D - first, vec_out);
+            split_gemm::fix_not_finite(o, [&](int j, int v) {
+                const int r = lane_id() & 31, c = j * 32 + split_gemm::acc_column(v);
+                if (block_row + r < rows && first + c < D)
+                    out[r * D + c] = from_f32<T>(
+                        split_gemm::scalar_dot(G + (block_row + r) * V, weight + first + c, V, 0.0f, 1, D));
+            });
+        }
+    }
+}
+
+// Partial sums of grad_weight [V, D] = G^T [V, rows] prior [rows, D] over the
+// rows [chunk * chunk_rows, + chunk_rows): a vocabulary this small has few
+// tiles, so the rows are split until the chip is full. At the sizes above 53 us (+ 7 for
+// the sum of the chunks), against 406 for the library's fp32 product on few tiles.
+template <typename T>
+__global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
+    const float* __restrict__ G, const T* __restrict__ prior, float* __restrict__ partial, int64_t rows, int64_t D,
+    int64_t V, int64_t d_tiles, int64_t v_tiles, int64_t chunk_rows) {
+    constexpr int BM = 128, BN = 128;
+    using Tile = split_gemm::Tile<float, T, BM, BN, true, true>;
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
+    const int64_t chunk = blockIdx.x / (d_tiles * v_tiles), tile_id = blockIdx.x % (d_tiles * v_tiles);
+    const int64_t v0 = tile_id / d_tiles * BM, d0 = tile_id % d_tiles * BN;
+    const int64_t k0 = chunk * chunk_rows, k1 = min(rows, k0 + chunk_rows);  // chunk_rows is a multiple of BK
+    const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
+    Tile tile;
+    tile.template run<kElementLoads, kElementLoads>(
+        lds, rows, rows, k0, k1, [&](int r) { return G + min(v0 + r, V - 1); },
+        [&](int r) { return prior + min(d0 + r, D - 1); }, [&](int t) { return wn * 64 + t * 32; }, V, D);
+    split_gemm::lds_barrier();  // the output rows pass through LDS
+    constexpr int kRegion = split_gemm::store_bytes<float, 1>();
+    static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
+#pragma unroll
+    for (int i = 0; i < Tile::MT; ++i) {
+        const int64_t block_v = v0 + wm * (BM / 2) + i * 32;
+#pragma unroll
+        for (int j = 0; j < Tile::NT; ++j) {
+            const int64_t first = d0 + wn * 64 + j * 32;
+            float o[1][16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[0][e] = tile.acc[i][j][e];
+            float* out = partial + (chunk * V + block_v) * D + first;
+            split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, D, V - block_v, D - first, D % 8 == 0);
+            split_gemm::fix_not_finite(o, [&](int, int e) {
+                const int r = lane_id() & 31, c = split_gemm::acc_column(e);
+                if (block_v + r < V && first + c < D)
+                    out[r * D + c] = split_gemm::scalar_dot(G + k0 * V + block_v + r, prior + k0 * D + first + c, k1 - k0,
+                                                            0.0f, V, D);
+            });
+        }
+    }
+}
+
+// Workspace of the backward: G, the weight gradient's chunks, the bias
+// gradient's partial rows.
+struct HeadWorkspace {
+    int64_t chunks, chunk_rows, blocks;
+    size_t partial_off, bias_off, total;
+};
+inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
+constexpr int64_t kWeightTiles = 512;              // two workgroups per CU (256: 73 us, 512: 53)
+constexpr int64_t kPartialFloats = int64_t(1) << 24;  // 64 MiB of partial sums at most
+
+inline HeadWorkspace head_workspace(int64_t rows, int64_t D, int64_t V) {
+    HeadWorkspace w;
+    const int64_t tiles = (V + 127) / 128 * ((D + 127) / 128);
+    int64_t chunks = kWeightTiles / tiles;
+    if (chunks > (rows + 127) / 128) chunks = (rows + 127) / 128;  // at least four K steps each
+    if (chunks > kPartialFloats / (V * D)) chunks = kPartialFloats / (V * D);
+    if (chunks < 1) chunks = 1;
+    w.chunk_rows = ((rows + chunks - 1) / chunks + 31) / 32 * 32;
+    w.chunks = (rows + w.chunk_rows - 1) / w.chunk_rows;
+    w.blocks = (rows + kRows - 1) / kRows;
+    w.partial_off = align256(static_cast<size_t>(rows) * V * sizeof(float));
+    w.bias_off = w.partial_off + align256(static_cast<size_t>(w.chunks) * V * D * sizeof(float));
+    w.total = w.bias_off + static_cast<size_t>(w.blocks) * V * sizeof(float);
+    return w;
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// run(kernel) with the columns and loads of a head tile.
+#define KOEMI_HEAD_KERNEL(run, kernel, T, columns, bytes)                                               \
+    ((columns) == kWide ? ((bytes) == 16 ? run(kernel<T, kWide, 16>)                                    \
+                           : (bytes) == 8 ? run(kernel<T, kWide, 8>) : run(kernel<T, kWide, 0>))        \
+                        : ((bytes) == 16 ? run(kernel<T, kNarrow, 16>)                                  \
+                           : (bytes) == 8 ? run(kernel<T, kNarrow, 8>) : run(kernel<T, kNarrow, 0>)))
+
+template <typename T>
+int head_forward(const void* prior, const void* weight, const void* bias, const int64_t* targets, const uint8_t* valid,
+                 void* out, float* stats, float* part, int64_t rows, int64_t D, int64_t V, float log_vocab,
+                 hipStream_t s) {
+    const int columns = head_columns(rows, V);
+    const int bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
+    const int64_t v_tiles = (V + columns - 1) / columns;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rows + kRows - 1) / kRows * v_tiles)), dim3(kThreads), 0, s,
+                           static_cast<const T*>(prior), static_cast<const T*>(weight), static_cast<const T*>(bias),
+                           targets, valid, static_cast<T*>(out), stats, part, rows, D, V, v_tiles, log_vocab);
+        return check_launch("koemi_surprise_head_forward");
+    };
+    const int st = KOEMI_HEAD_KERNEL(run, surprise_head_forward_kernel, T, columns, bytes);
+    if (st != KOEMI_OK || v_tiles == 1) return st;
+    hipLaunchKernelGGL(surprise_head_finish_kernel<T>, dim3(grid_for(rows, 256)), dim3(256), 0, s, part, targets, valid,
+                       static_cast<T*>(out), stats, rows, V, v_tiles, columns, log_vocab);
+    return check_launch("koemi_surprise_head_forward(finish)");
+}
+
+template <typename T>
+int head_backward(const void* prior, const void* weight, const void* bias, const int64_t* targets, const uint8_t* valid,
+                  const float* stats, const void* grad, void* grad_prior, void* grad_weight, void* grad_bias,
+                  int64_t rows, int64_t D, int64_t V, float log_vocab, const HeadWorkspace& ws, char* base,
+                  hipStream_t s) {
+    float* G = reinterpret_cast<float*>(base);
+    float* partial = reinterpret_cast<float*>(base + ws.partial_off);
+    float* bias_partial = reinterpret_cast<float*>(base + ws.bias_off);
+    const T* p = static_cast<const T*>(prior);
+    const T* w = static_cast<const T*>(weight);
+    const int64_t d_tiles = (D + 127) / 128, v_tiles = (V + 127) / 128;
+    const int columns = head_columns(rows, V);
+    const int head_bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
+    const int64_t head_tiles = (V + columns - 1) / columns;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ws.blocks * head_tiles)), dim3(kThreads), 0, s, p, w,
+                           static_cast<const T*>(bias), targets, valid, static_cast<const T*>(grad), stats, G,
+                           bias_partial, rows, D, V, head_tiles, log_vocab);
+        return check_launch("koemi_surprise_head_backward(logits)");
+    };
+    int st = KOEMI_HEAD_KERNEL(run, surprise_head_grad_logits_kernel, T, columns, head_bytes);
+    if (st != KOEMI_OK) return st;
+    const int bytes = split_gemm::load_bytes<float>(G, V);
+    // 128 x 128 tiles, or 64 x 64 ones with four K steps of loads in flight where the
+    // larger would give fewer than one to each CU (4000 rows x 300, vocabulary 1000,
+    // fp32: 67 -> 39 us)
+    const int64_t b = (rows + 127) / 128 * d_tiles < 256 ? 64 : 128;
+    const int64_t prior_tiles = (D + b - 1) / b;
+    const auto prior_run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rows + b - 1) / b * prior_tiles)), dim3(kThreads), 0, s, G,
+                           w, static_cast<T*>(grad_prior), rows, D, V, prior_tiles,
+                           static_cast<int>(D % 8 == 0 && aligned16(grad_prior)));
+        return check_launch("koemi_surprise_head_backward(prior)");
+    };
+    st = b == 128 ? (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, 128, 16>)
+                     : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, 128, 8>)
+                                  : prior_run(surprise_head_grad_prior_kernel<T, 128, 0>))
+                  : (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, 64, 16>)
+                     : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, 64, 8>)
+                                  : prior_run(surprise_head_grad_prior_kernel<T, 64, 0>));
+    if (st != KOEMI_OK) return st;
+    hipLaunchKernelGGL(surprise_head_grad_weight_kernel<T>, dim3(static_cast<unsigned>(ws.chunks * d_tiles * v_tiles)),
+                       dim3(kThreads), 0, s, G, p, partial, rows, D, V, d_tiles, v_tiles, ws.chunk_rows);
+    st = check_launch("koemi_surprise_head_backward(weight)");
+    if (st != KOEMI_OK) return st;
+    launch_column_sum(partial, static_cast<T*>(grad_weight), ws.chunks, V * D, s);
+    st = check_launch("koemi_surprise_head_backward(weight sum)");
+    if (st != KOEMI_OK) return st;
+    launch_column_sum(bias_partial, static_cast<T*>(grad_bias), ws.blocks, V, s);
+    return check_launch("koemi_surprise_head_backward(bias sum)");
+}
+
+int check_head(int64_t rows, int64_t D, int64_t V, int dtype) {
+    if (rows < 1 || D < 1 || V < 2) return fail(KOEMI_ERR_INVALID, "the surprise head needs rows, width >= 1 and vocab >= 2");
+    if (!float_dtype(dtype)) return fail(KOEMI_ERR_UNSUPPORTED, "the surprise head does not support dtype %s", dtype_name(dtype));
+    if ((rows + 63) / 64 * ((V + 63) / 64) > 0x7fffffffLL || (rows + 127) / 128 * ((D + 127) / 128) > 0x7fffffffLL ||
+        (V + 127) / 128 * ((D + 127) / 128) > 0x7fffffffLL || V > 0x7fffffffLL / 8 || D > 0x7fffffffLL / 8)
+        return fail(KOEMI_ERR_UNSUPPORTED, "the surprise head's sizes are too large");
+    return KOEMI_OK;
+}
+
+}  // namespace
+}  // namespace koemi
+
+using namespace koemi;
+
+extern "C" size_t koemi_surprise_head_forward_workspace_bytes(int64_t rows, int64_t vocab) {
+    if (rows < 1 || vocab < 2) return 0;
+    const int columns = head_columns(rows, vocab);
+    if (vocab <= columns) return 0;
+    return static_cast<size_t>((vocab + columns - 1) / columns) * 3 * static_cast<size_t>(rows) * sizeof(float);
+}
+
+extern "C" int koemi_surprise_head_forward(const void* prior, const void* weight, const void* bias,
+                                           const int64_t* target_ids, const uint8_t* valid_mask, void* surprise,
+                                           float* stats, int64_t rows, int64_t width, int64_t vocab, float log_vocab,
+                                           int dtype, void* workspace, size_t workspace_bytes, koemi_stream_t stream) {
+    const int st = check_head(rows, width, vocab, dtype);
+    if (st != KOEMI_OK) return st;
+    if (!prior || !weight || !bias || !target_ids || !valid_mask || !surprise || !stats)
+        return fail(KOEMI_ERR_INVALID, "the surprise head received a null pointer");
+    const size_t need = koemi_surprise_head_forward_workspace_bytes(rows, vocab);
+    if (workspace_bytes < need || (need > 0 && !workspace))
+        return fail(KOEMI_ERR_INVALID, "surprise head workspace too small: need %zu bytes", need);
+    const auto run = [&](auto tag) {
+        return head_forward<decltype(tag)>(prior, weight, bias, target_ids, valid_mask, surprise, stats,
+                                           static_cast<float*>(workspace), rows, width, vocab, log_vocab,
+                                           as_stream(stream));
+    };
+    return dtype == KOEMI_F32 ? run(float{}) : dtype == KOEMI_F16 ? run(f16{}) : run(bf16{});
+}
+
+extern "C" size_t koemi_surprise_head_backward_workspace_bytes(int64_t rows, int64_t width, int64_t vocab) {
+    if (rows < 1 || width < 1 || vocab < 2) return 0;
+    return head_workspace(rows, width, vocab).total;
+}
+
+extern "C" int koemi_surprise_head_backward(const void* prior, const void* weight, const void* bias,
+                                            const int64_t* target_ids, const uint8_t* valid_mask, const float* stats,
+                                            const void* grad_surprise, void* grad_prior, void* grad_weight,
+                                            void* grad_bias, int64_t rows, int64_t width, int64_t vocab, float log_vocab,
+                                            int dtype, void* workspace, size_t workspace_bytes, koemi_stream_t stream) {
+    const int st = check_head(rows, width, vocab, dtype);
+    if (st != KOEMI_OK) return st;
+    if (!prior || !weight || !bias || !target_ids || !valid_mask || !stats || !grad_surprise || !grad_prior ||
+        !grad_weight || !grad_bias)
+        return fail(KOEMI_ERR_INVALID, "the surprise head received a null pointer");
+    const HeadWorkspace ws = head_workspace(rows, width, vocab);
+    if (!workspace || workspace_bytes < ws.total)
+        return fail(KOEMI_ERR_INVALID, "surprise head workspace too small: need %zu bytes", ws.total);
+    const auto run = [&](auto tag) {
+        return head_backward<decltype(tag)>(prior, weight, bias, target_ids, valid_mask, stats, grad_surprise, grad_prior,
+                                            grad_weight, grad_bias, rows, width, vocab, log_vocab, ws,
+                                            static_cast<char*>(workspace), as_stream(stream));
+    };
+    return dtype == KOEMI_F32 ? run(float{}) : dtype == KOEMI_F16 ? run(f16{}) : run(bf16{});
+}

@@ -30,6 +30,7 @@ SOURCES = (
     "affine_scan.hip",
     "rmsnorm_silu.hip",
     "surprise.hip",
+    "surprise_head.hip",
     "moe_route.hip",
     "moe_permute.hip",
     "moe_grouped_mlp.hip",

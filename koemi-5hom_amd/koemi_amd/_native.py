@@ -66,6 +66,14 @@ _SIGNATURES: dict[str, tuple[Any, tuple[Any, ...]]] = {
         (_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int, _P, c_size_t, _P),
     ),
     "koemi_surprise_rows_forward": (c_int, (_P, _P, _P, _P, _P, c_int64, c_int64, c_float, c_int, _P)),
+    "koemi_surprise_head_forward": (
+        c_int, (_P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_float, c_int, _P, c_size_t, _P)),
+    "koemi_surprise_head_forward_workspace_bytes": (c_size_t, (c_int64, c_int64)),
+    "koemi_surprise_head_backward_workspace_bytes": (c_size_t, (c_int64, c_int64, c_int64)),
+    "koemi_surprise_head_backward": (
+        c_int,
+        (_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_float, c_int, _P, c_size_t, _P),
+    ),
     "koemi_surprise_rows_backward": (
         c_int,
         (_P, _P, _P, _P, _P, _P, c_int64, c_int64, c_float, c_int, _P),

@@ -2,9 +2,9 @@
 
 ``causal_surprise`` and ``benchmark_causal_surprise`` mirror
 ``src/koemi/cuda_kernels/think/surprise.py`` (signature, exceptions, messages,
-autograd contract). As in the reference (surprise_kernel.cu:194-261) the
-content-head logits come from a plain fp32 GEMM (here ``torch.mm``, i.e.
-hipBLASLt) and the per-row work runs in ``csrc/surprise.hip``.
+autograd contract) on ``csrc/surprise_head.hip``: the content head's product
+with the row scoring in its epilogue, where the reference
+(surprise_kernel.cu:194-328) writes fp32 logits and runs a row kernel.
 
 Build-side fronts (keyword-only extensions, no reference counterpart):
 
@@ -121,29 +121,60 @@ def _rows_backward(
     return grad_logits
 
 
+def _head_forward(prior: Tensor, weight: Tensor, bias: Tensor, targets: Tensor, valid: Tensor) -> tuple[Tensor, Tensor]:
+    """Scores [B, L] and the rows' [3, B L] statistics for the backward, the logits kept on chip."""
+
+    batch, sequence, width = prior.shape
+    rows, vocab = batch * sequence, weight.shape[0]
+    out = torch.empty((batch, sequence), device=prior.device, dtype=prior.dtype)
+    stats = torch.empty((3, rows), device=prior.device, dtype=torch.float32)
+    need = _native.query("koemi_surprise_head_forward_workspace_bytes", rows, vocab)
+    workspace = torch.empty((need,), device=prior.device, dtype=torch.uint8) if need else None
+    with torch.cuda.device(prior.device):
+        _native.call("koemi_surprise_head_forward", prior.data_ptr(), weight.data_ptr(), bias.data_ptr(),
+                     targets.data_ptr(), valid.data_ptr(), out.data_ptr(), stats.data_ptr(), rows, width, vocab,
+                     _log_vocab(vocab), _native.dtype_code(prior.dtype), _native.ptr(workspace), need,
+                     _native.stream_of(prior.device))
+    return out, stats
+
+
+def _head_backward(prior: Tensor, weight: Tensor, bias: Tensor, targets: Tensor, valid: Tensor, stats: Tensor,
+                   gradient: Tensor) -> tuple[Tensor, Tensor, Tensor]:
+    batch, sequence, width = prior.shape
+    rows, vocab = batch * sequence, weight.shape[0]
+    grads = tuple(torch.empty_like(t) for t in (prior, weight, bias))
+    need = _native.query("koemi_surprise_head_backward_workspace_bytes", rows, width, vocab)
+    workspace = torch.empty((need,), device=prior.device, dtype=torch.uint8)
+    with torch.cuda.device(prior.device):
+        _native.call("koemi_surprise_head_backward", prior.data_ptr(), weight.data_ptr(), bias.data_ptr(),
+                     targets.data_ptr(), valid.data_ptr(), stats.data_ptr(), gradient.data_ptr(),
+                     *(t.data_ptr() for t in grads), rows, width, vocab, _log_vocab(vocab),
+                     _native.dtype_code(prior.dtype), workspace.data_ptr(), need, _native.stream_of(prior.device))
+    return grads
+
+
 class _CausalSurpriseFunction(torch.autograd.Function):
     @staticmethod
     def forward(context, prior_states, content_weight, content_bias, target_ids, valid_mask):  # type: ignore[override]
         _load()
         inputs = tuple(t.contiguous() for t in (prior_states, content_weight, content_bias, target_ids, valid_mask))
-        prior, weight, bias, targets, valid = inputs
-        batch, sequence, width = prior.shape
-        prior_float = prior.view(batch * sequence, width).float()
-        logits = torch.mm(prior_float, weight.float().t())
-        surprise = _rows_forward(logits, bias, targets.view(-1), valid.view(-1), prior.dtype)
-        context.save_for_backward(*inputs)
-        return surprise.view(batch, sequence)
+        surprise, stats = _head_forward(*inputs)
+        context.save_for_backward(*inputs, stats)
+        return surprise
 
     @staticmethod
     def backward(context, gradient):  # type: ignore[override]
-        prior, weight, bias, targets, valid = context.saved_tensors
+        prior, weight, bias, targets, valid, stats = context.saved_tensors
+        gradient = gradient.contiguous().view(-1).to(prior.dtype)
+        if not torch.is_grad_enabled():
+            return (*_head_backward(prior, weight, bias, targets, valid, stats, gradient), None, None)
+        # create_graph: the products as differentiable torch operations (as the
+        # reference's backward forms them, surprise_kernel.cu:263-328)
         batch, sequence, width = prior.shape
         prior_float = prior.view(batch * sequence, width).float()
         weight_float = weight.float()
         logits = torch.mm(prior_float, weight_float.t())
-        grad_logits = _rows_backward(
-            logits, bias, targets.view(-1), valid.view(-1), gradient.contiguous().view(-1).to(prior.dtype)
-        )
+        grad_logits = _rows_backward(logits, bias, targets.view(-1), valid.view(-1), gradient)
         gradient_prior = torch.mm(grad_logits, weight_float).view(prior.shape)
         gradient_weight = torch.mm(grad_logits.t(), prior_float)
         gradient_bias = grad_logits.sum(0)

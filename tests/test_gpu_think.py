@@ -201,3 +201,89 @@ def test_fixed_threshold_admission_is_strict(device):
     big_valid = (torch.rand((3, 1000), generator=g) < 0.8).to(device)
     assert torch.equal(think.admission_above(big, big_valid, 0.5),
                        think.salience_admission(big, big_valid, threshold=0.5)[0])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,length,width,vocab", [
+    (1, 1, 1, 2), (3, 21, 8, 19), (1, 64, 64, 256), (5, 13, 72, 257), (2, 64, 300, 255), (1, 129, 136, 520),
+    (4, 300, 128, 256), (3, 700, 40, 130), (2, 65, 512, 1000), (9, 600, 264, 64),
+])
+def test_causal_surprise_head_of_every_tile_shape(device, dtype, batch, length, width, vocab):
+    """Scores and gradients at the edges of the head's tiles (64 rows, 256 columns, 128 columns of the
+    weight gradients, row chunks, unaligned widths) against float64 autograd.
+
+    With u = 2^-24: a logit's fp32 sum errs by dz = 4 sqrt(D) u sum |terms| (Higham's sqrt(n) model with a
+    factor of 4), the row's maximum over columns; a score by (2 dz + 16 u (1 + |lse|)) / ln V; G by |g| / ln V
+    times (p (4 dz + 32 u (1 + |lse|)) + 16 u |p - [target]|); the gradients by that through the other factor and
+    their own fp32 sums, then half an ulp of the output's type."""
+
+    g = torch.Generator().manual_seed(batch * 1000003 + length * 1009 + width + vocab)
+    prior = (0.5 * torch.randn((batch, length, width), generator=g)).to(dtype)
+    weight = (2.0 / math.sqrt(width) * torch.randn((vocab, width), generator=g)).to(dtype)
+    bias = (0.1 * torch.randn((vocab,), generator=g)).to(dtype)
+    targets = torch.randint(0, vocab, (batch, length), generator=g)
+    valid = torch.rand((batch, length), generator=g) < 0.85
+    up = torch.randn((batch, length), generator=g).to(dtype)
+    leaves = [t.to(device).requires_grad_() for t in (prior, weight, bias)]
+    score = think.causal_surprise(*leaves, targets.to(device), valid.to(device))
+    grads = torch.autograd.grad(score, leaves, up.to(device), retain_graph=True)
+    p, w, b = (t.double().requires_grad_() for t in (prior, weight, bias))
+    z = p @ w.t() + b
+    lse = torch.logsumexp(z, -1)
+    nll = lse - z.gather(-1, targets[..., None])[..., 0]
+    want = torch.where(valid, 1 - torch.exp(-nll / math.log(vocab)), 0.0)
+    want_grads = torch.autograd.grad(want, (p, w, b), up.double())
+    u, ln = 2.0**-24, math.log(vocab)
+    half_ulp = {torch.float32: u, torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[dtype]
+    rows = batch * length
+    p, w, b, z, lse = p.detach().view(rows, width), w.detach(), b.detach(), z.detach().view(rows, vocab), lse.detach().view(rows, 1)
+    dz = (4 * math.sqrt(width) * u * (p.abs() @ w.abs().t() + b.abs())).amax(-1, keepdim=True) + 16 * u * (1 + lse.abs())
+    soft = torch.softmax(z, -1)
+    hot = torch.nn.functional.one_hot(targets.view(-1), vocab).double()
+    gnll = (up.double().view(-1, 1) * torch.exp(-nll.detach().view(-1, 1) / ln) / ln) * valid.view(-1, 1)
+    G = gnll * (soft - hot)
+    dG = gnll.abs() * (soft * 4 * dz + 2 * dz / ln * (soft - hot).abs() + 16 * u * (soft - hot).abs())
+    tiny = 2.0**-25 if dtype == torch.float16 else 1e-37
+    checks = [
+        (score, want, (2 * dz / ln).view(batch, length) * valid),
+        (grads[0], want_grads[0], (dG @ w.abs() + 4 * math.sqrt(vocab) * u * (G.abs() @ w.abs())).view(prior.shape)),
+        (grads[1], want_grads[1], dG.t() @ p.abs() + 4 * math.sqrt(rows) * u * (G.abs().t() @ p.abs())),
+        (grads[2], want_grads[2], dG.sum(0) + 4 * math.sqrt(rows) * u * G.abs().sum(0)),
+    ]
+    for got, ref, bound in checks:
+        err = (got.detach().double().cpu() - ref.detach()).abs()
+        bound = bound + half_ulp * ref.detach().abs() + tiny
+        assert bool((err <= bound).all()), float((err / bound).max())
+    with_graph = torch.autograd.grad(score, leaves, up.to(device), create_graph=True)
+    for got, ref, bound in zip(with_graph, want_grads, (c[2] for c in checks[1:])):
+        bound = bound + half_ulp * ref.abs() + tiny
+        assert bool(((got.detach().double().cpu() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_causal_surprise_contains_what_is_not_finite(device, dtype):
+    """A row of states with infinities or NaN leaves every other row's score and gradient unchanged, and so
+    does an invalid row or (unchecked) a target out of range; the out-of-range row scores NaN with no gradient."""
+
+    g = torch.Generator().manual_seed(5)
+    prior = (0.5 * torch.randn((2, 70, 96), generator=g)).to(dtype).to(device)
+    weight = (0.2 * torch.randn((300, 96), generator=g)).to(dtype).to(device)
+    bias = torch.zeros((300,), dtype=dtype, device=device)
+    targets = torch.randint(0, 300, (2, 70), generator=g).to(device)
+    valid = torch.ones((2, 70), dtype=torch.bool, device=device)
+    up = torch.ones((2, 70), dtype=dtype, device=device)
+    def run(prior, targets):
+        leaf = prior.clone().requires_grad_()
+        score = think.causal_surprise(leaf, weight, bias, targets, valid, validate_targets=False)
+        return score.detach(), torch.autograd.grad(score, leaf, up)[0]
+    clean, clean_grad = run(prior, targets)
+    bad, bad_targets = prior.clone(), targets.clone()
+    bad[0, 3, 7], bad[1, 40, 0], bad[1, 69, 95] = float("inf"), float("nan"), -float("inf")
+    bad_targets[0, 10], bad_targets[1, 1] = 300, -1
+    score, grad = run(bad, bad_targets)
+    touched = torch.zeros((2, 70), dtype=torch.bool, device=device)
+    for i, j in ((0, 3), (1, 40), (1, 69), (0, 10), (1, 1)):
+        touched[i, j] = True
+    assert torch.equal(score[~touched], clean[~touched]) and torch.equal(grad[~touched], clean_grad[~touched])
+    assert bool(torch.isnan(score[touched]).all())
+    assert not grad[0, 10].any() and not grad[1, 1].any()
