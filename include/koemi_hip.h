@@ -224,6 +224,12 @@ int koemi_moe_router_balance_loss(const float* probability_mass, const float* as
 int koemi_moe_check_assignments(const void* assignments, int assignment_dtype,
                                 const uint8_t* valid_mask, int32_t* flags, int64_t tokens,
                                 int64_t top_k, int64_t expert_count, koemi_stream_t stream);
+/* Checks of sorted pairs (moe/__init__.py:293-301, 345-353), ORed into flags[0]
+ * (zeroed by the caller): 1 the last of offset_count offsets outside [0, pairs],
+ * 2 an id among the valid pairs outside [0, limit) (looked at only without 1),
+ * 4 offsets that decrease or start below 0. */
+int koemi_moe_check_segments(const int64_t* ids, const int64_t* offsets, int32_t* flags, int64_t pairs,
+                             int64_t offset_count, int64_t limit, koemi_stream_t stream);
 
 /* Per-expert activation counts (model/network.py:48-70):
  * counts[e] = #{(t, s): valid[t] && assignments[t, s] == e}. counts int64 [E]

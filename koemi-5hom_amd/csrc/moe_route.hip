@@ -274,6 +274,28 @@ __global__ void zero_i64_kernel(int64_t* __restrict__ p, int64_t n) {
     if (i < n) p[i] = 0;
 }
 
+// The fronts' checks of sorted pairs (moe/__init__.py:293-301, 345-353) as bits of
+// *flags: 1 the last offset outside [0, pairs], 2 an id of a valid pair outside
+// [0, limit), 4 offsets that decrease or start below 0. One launch and one
+// read-back for what ran as eight small kernels and three read-backs (61 us of a
+// checked expert call on the host; 18 us so).
+__global__ __launch_bounds__(256) void check_segments_kernel(const int64_t* __restrict__ ids,
+                                                             const int64_t* __restrict__ offsets,
+                                                             int32_t* __restrict__ flags, int64_t pairs,
+                                                             int64_t offset_count, int64_t limit) {
+    const int64_t last = offsets[offset_count - 1];
+    const bool outside = last < 0 || last > pairs;
+    int bits = outside ? 1 : 0;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (!outside)
+        for (int64_t i = first; i < last; i += stride)
+            if (ids[i] < 0 || ids[i] >= limit) bits |= 2;
+    for (int64_t i = first; i < offset_count; i += stride)
+        if (offsets[i] < (i ? offsets[i - 1] : 0)) bits |= 4;
+    if (bits) atomicOr(flags, bits);
+}
+
 }  // namespace
 }  // namespace koemi
 
@@ -408,6 +430,17 @@ extern "C" int koemi_moe_check_assignments(const void* assignments, int assignme
         hipLaunchKernelGGL(check_assignments_kernel<int64_t>, grid, block, 0, s, static_cast<const int64_t*>(assignments),
                            valid_mask, flags, tokens, top_k, expert_count);
     return check_launch("koemi_moe_check_assignments");
+}
+
+extern "C" int koemi_moe_check_segments(const int64_t* ids, const int64_t* offsets, int32_t* flags, int64_t pairs,
+                                        int64_t offset_count, int64_t limit, koemi_stream_t stream) {
+    if (pairs < 0 || offset_count < 1 || limit < 0) return fail(KOEMI_ERR_INVALID, "invalid segment check sizes");
+    if (!offsets || !flags || (pairs > 0 && !ids)) return fail(KOEMI_ERR_INVALID, "segment check received a null pointer");
+    const int64_t items = pairs > offset_count ? pairs : offset_count;
+    const int64_t blocks = (items + 1023) / 1024;
+    hipLaunchKernelGGL(check_segments_kernel, dim3(static_cast<unsigned>(blocks < 256 ? blocks : 256)), dim3(256), 0,
+                       as_stream(stream), ids, offsets, flags, pairs, offset_count, limit);
+    return check_launch("koemi_moe_check_segments");
 }
 
 extern "C" int koemi_moe_expert_counts(const void* assignments, int assignment_dtype,

@@ -219,6 +219,7 @@ _SIGNATURES: dict[str, tuple[Any, tuple[Any, ...]]] = {
         c_int,
         (_P, c_int, _P, c_int, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int64, c_int64, c_int64, _P, c_size_t, _P),
     ),
+    "koemi_moe_check_segments": (c_int, (_P, _P, _P, c_int64, c_int64, c_int64, _P)),
     "koemi_moe_grouped_mlp_workspace_bytes": (c_size_t, (c_int64, c_int64, c_int64, c_int64, c_int)),
     "koemi_moe_grouped_mlp": (
         c_int,
@@ -271,6 +272,10 @@ def library_built() -> bool:
     return LIBRARY_PATH.is_file()
 
 
+def library_loaded() -> bool:
+    return _LIBRARY is not None
+
+
 def load_library() -> ctypes.CDLL:
     """Load libkoemi_hip.so once per process and bind every declared entry point."""
 
@@ -315,10 +320,33 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
     return tensor.data_ptr()
 
 
+# The raw handle without building a Stream object (2 us a call); torch.cuda.current_stream's where it is absent.
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(device: torch.device) -> int:
     """Raw hipStream_t of torch's current stream on `device`."""
 
+    if _RAW_STREAM is not None and device.index is not None:
+        return _RAW_STREAM(device.index)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+class _NoGuard:
+    def __enter__(self) -> None:
+        return None
+
+    def __exit__(self, *args: Any) -> None:
+        return None
+
+
+_NO_GUARD = _NoGuard()
+
+
+def device_guard(device: torch.device) -> Any:
+    """``torch.cuda.device(device)``, or nothing where that device is already current."""
+
+    return _NO_GUARD if device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def ptr_array(tensors: list[torch.Tensor | None]) -> ctypes.Array:
@@ -328,17 +356,26 @@ def ptr_array(tensors: list[torch.Tensor | None]) -> ctypes.Array:
     return (c_void_p * len(tensors))(*(ptr(t) for t in tensors))
 
 
+_FUNCTIONS: dict[str, Any] = {}
+
+
+def _function(name: str) -> Any:
+    function = _FUNCTIONS.get(name)
+    if function is None:
+        function = _FUNCTIONS[name] = getattr(load_library(), name)
+    return function
+
+
 def call(name: str, *args: Any) -> None:
     """Invoke an entry point and raise NativeCallError on a non-zero status."""
 
-    lib = load_library()
-    status = getattr(lib, name)(*args)
+    status = _function(name)(*args)
     if status != OK:
-        message = (lib.koemi_last_error() or b"").decode("utf-8", "replace")
+        message = (load_library().koemi_last_error() or b"").decode("utf-8", "replace")
         raise NativeCallError(name, status, message)
 
 
 def query(name: str, *args: Any) -> int:
     """Invoke a size query entry point."""
 
-    return int(getattr(load_library(), name)(*args))
+    return int(_function(name)(*args))

@@ -36,7 +36,7 @@ def rmsnorm_silu_forward(input_tensor: Tensor, weight: Tensor, eps: float) -> li
     inverse_rms = torch.empty((input_tensor.shape[0],), device=input_tensor.device, dtype=torch.float32)
     if input_tensor.shape[0] == 0:
         return [output, inverse_rms]
-    with torch.cuda.device(input_tensor.device):
+    with _native.device_guard(input_tensor.device):
         _native.call(
             "koemi_rmsnorm_silu_forward",
             input_tensor.data_ptr(),
@@ -68,7 +68,7 @@ def rmsnorm_silu_backward(
     gradient_weight = torch.empty_like(weight)
     workspace_bytes = _native.query("koemi_rmsnorm_silu_backward_workspace_bytes", rows, hidden)
     workspace = torch.empty((max(workspace_bytes, 1),), device=input_tensor.device, dtype=torch.uint8)
-    with torch.cuda.device(input_tensor.device):
+    with _native.device_guard(input_tensor.device):
         _native.call(
             "koemi_rmsnorm_silu_backward",
             gradient_output.data_ptr(),

@@ -120,7 +120,7 @@ def scan_forward(retention: Tensor, increment: Tensor, initial: Tensor) -> Tenso
         return states
     batch, sequence, features = _geometry(increment)
     broadcast = retention.numel() == batch * sequence
-    with torch.cuda.device(increment.device):
+    with _native.device_guard(increment.device):
         _native.call(
             "koemi_affine_scan_forward",
             retention.data_ptr(),
@@ -150,7 +150,7 @@ def scan_backward(
         return gradient_retention, gradient_increment, gradient_initial
     batch, sequence, features = _geometry(states)
     broadcast = retention.numel() == batch * sequence
-    with torch.cuda.device(states.device):
+    with _native.device_guard(states.device):
         _native.call(
             "koemi_affine_scan_backward",
             retention.data_ptr(),

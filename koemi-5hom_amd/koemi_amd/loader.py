@@ -95,6 +95,8 @@ def cuda_extension_available() -> bool:
 def require_library() -> None:
     """Load the kernel library or raise the loader's typed errors."""
 
+    if _native.library_loaded() and torch.cuda.is_available():
+        return
     status = detect_cuda_toolchain()
     if not status.ready:
         raise CudaExtensionUnavailableError(f"GPU kernel library is unavailable: {status.reason}.")

@@ -112,7 +112,7 @@ def _assignment_flags(assignments: Tensor, valid_mask: Tensor, expert_count: int
 
     flags = torch.zeros((2,), device=assignments.device, dtype=torch.int32)
     tokens, top_k = assignments.shape
-    with torch.cuda.device(assignments.device):
+    with _native.device_guard(assignments.device):
         _native.call(
             "koemi_moe_check_assignments",
             assignments.data_ptr(),
@@ -126,6 +126,19 @@ def _assignment_flags(assignments: Tensor, valid_mask: Tensor, expert_count: int
         )
     out_of_range, duplicate = flags.tolist()
     return bool(out_of_range), bool(duplicate)
+
+
+def _segment_flags(ids: Tensor, segment_offsets: Tensor, limit: int) -> tuple[bool, bool, bool]:
+    """(the last offset outside [0, pairs], an id of a valid pair outside [0, limit), the offsets not
+    non-decreasing from at least 0), from one device check and one read-back. The ids are looked at only where
+    the last offset is inside."""
+
+    flags = torch.zeros((1,), device=ids.device, dtype=torch.int32)
+    with _native.device_guard(ids.device):
+        _native.call("koemi_moe_check_segments", ids.data_ptr(), segment_offsets.data_ptr(), flags.data_ptr(),
+                     ids.shape[0], segment_offsets.shape[0], limit, _native.stream_of(ids.device))
+    word = flags.item()
+    return bool(word & 1), bool(word & 2), bool(word & 4)
 
 
 def route_topk_valid(
@@ -165,7 +178,7 @@ def route_topk_valid(
     # the duplicate check's flag only when it is read (validate)
     duplicate = torch.zeros((1,), device=token_ids.device, dtype=torch.int32) if validate else None
     if count:
-        with torch.cuda.device(token_ids.device):
+        with _native.device_guard(token_ids.device):
             _native.call(
                 "koemi_moe_route_hash",
                 token_ids.data_ptr(),
@@ -210,7 +223,7 @@ def route_topk_modulo(token_ids: Tensor, valid_mask: Tensor, *, expert_count: in
     assignments = torch.empty((count, top_k), device=token_ids.device, dtype=torch.int64)
     if count:
         token_ids, valid_mask = token_ids.contiguous(), valid_mask.contiguous()
-        with torch.cuda.device(token_ids.device):
+        with _native.device_guard(token_ids.device):
             _native.call("koemi_moe_route_modulo", token_ids.data_ptr(), valid_mask.data_ptr(),
                          _native.dtype_code(token_ids.dtype), assignments.data_ptr(), count, expert_count, top_k,
                          _native.stream_of(token_ids.device))
@@ -249,7 +262,7 @@ class RouterStatistics:
             raise CudaMoeValidationError("probability_mass and assignment_counts must be [expert_count]")
         _require_library()
         loss = torch.empty((), device=mass.device, dtype=torch.float32)
-        with torch.cuda.device(mass.device):
+        with _native.device_guard(mass.device):
             _native.call("koemi_moe_router_balance_loss", mass.data_ptr(), counts.data_ptr(), valid.data_ptr(),
                          mass.numel(), loss.data_ptr(), _native.stream_of(mass.device))
         return loss
@@ -305,7 +318,7 @@ def route_topk_learned(router_logits: Tensor, valid_mask: Tensor, *, top_k: int,
         need = _native.query("koemi_moe_route_learned_stats_workspace_bytes", count, expert_count)
         workspace = torch.empty((max(need, 1),), device=device, dtype=torch.uint8)
         logits_c, valid_c = router_logits.contiguous(), valid_mask.contiguous()
-        with torch.cuda.device(device):
+        with _native.device_guard(device):
             _native.call("koemi_moe_route_learned_stats", logits_c.data_ptr(),
                          valid_c.data_ptr(), assignments.data_ptr(), weights.data_ptr(),
                          mass.data_ptr(), counts.data_ptr(), valid_count.data_ptr(), loss.data_ptr(), count,
@@ -313,7 +326,7 @@ def route_topk_learned(router_logits: Tensor, valid_mask: Tensor, *, top_k: int,
         statistics = RouterStatistics(mass, counts, valid_count, loss)
         return assignments.reshape(shape), weights.reshape(shape), statistics
     if count:
-        with torch.cuda.device(router_logits.device):
+        with _native.device_guard(router_logits.device):
             _native.call(
                 "koemi_moe_route_learned",
                 router_logits.data_ptr(),
@@ -343,7 +356,7 @@ def expert_activation_counts(assignments: Tensor, valid_mask: Tensor, *, expert_
     _require_library()
     top_k = int(assignments.shape[-1])
     counts = torch.empty((expert_count,), device=assignments.device, dtype=torch.int64)
-    with torch.cuda.device(assignments.device):
+    with _native.device_guard(assignments.device):
         _native.call(
             "koemi_moe_expert_counts",
             assignments.data_ptr(),
@@ -425,7 +438,7 @@ def permute_topk(
         raise CudaMoeValidationError("context dimensions must be positive")
     workspace_bytes = _native.query("koemi_moe_permute_workspace_bytes", tokens, top_k, expert_count)
     workspace = torch.empty((workspace_bytes,), device=device, dtype=torch.uint8)
-    with torch.cuda.device(device):
+    with _native.device_guard(device):
         _native.call(
             "koemi_moe_permute",
             flat.data_ptr(),
@@ -520,16 +533,12 @@ def grouped_expert_mlp_inference(
     _require_library()
     pairs = int(sorted_context.shape[0])
     if validate:
-        offsets = segment_offsets.tolist()
-        valid_pair_count = int(offsets[-1])
-        if valid_pair_count < 0 or valid_pair_count > pairs:
+        outside, bad, unordered = _segment_flags(sorted_experts, segment_offsets, expert_count)
+        if outside:
             raise CudaMoeValidationError("segment_offsets final value is outside pair_count")
-        if valid_pair_count:
-            selected = sorted_experts[:valid_pair_count]
-            bad = torch.stack(((selected < 0).any(), (selected >= expert_count).any())).tolist()
-            if any(bad):
-                raise CudaMoeValidationError("sorted expert ids are outside the expert catalog")
-        if any(b < a for a, b in zip(offsets, offsets[1:])) or offsets[0] < 0:
+        if bad:
+            raise CudaMoeValidationError("sorted expert ids are outside the expert catalog")
+        if unordered:
             raise CudaMoeValidationError("segment_offsets must be non-decreasing")
     output = torch.empty_like(sorted_context)
     if pairs == 0:
@@ -545,7 +554,7 @@ def grouped_expert_mlp_inference(
         _native.dtype_code(sorted_context.dtype),
     )
     workspace = torch.empty((workspace_bytes,), device=sorted_context.device, dtype=torch.uint8)
-    with torch.cuda.device(sorted_context.device):
+    with _native.device_guard(sorted_context.device):
         _native.call(
             "koemi_moe_grouped_mlp",
             x.data_ptr(),
@@ -590,7 +599,7 @@ def permute_indices(assignments: Tensor, valid_mask: Tensor, *, expert_count: in
     pair_positions = torch.empty((pairs,), device=device, dtype=torch.int64)
     need = _native.query("koemi_moe_permute_workspace_bytes", tokens, top_k, expert_count)
     workspace = torch.empty((need,), device=device, dtype=torch.uint8)
-    with torch.cuda.device(device):
+    with _native.device_guard(device):
         _native.call("koemi_moe_permute_indices", assignments.contiguous().data_ptr(),
                      _native.dtype_code(assignments.dtype), valid_mask.contiguous().data_ptr(),
                      _native.ptr(pair_weights.contiguous() if pair_weights is not None else None),
@@ -624,7 +633,7 @@ def permute_hash_indices(token_ids: Tensor, previous_token_ids: Tensor, valid_ma
     pair_positions = torch.empty((pairs,), device=device, dtype=torch.int64)
     need = _native.query("koemi_moe_permute_workspace_bytes", tokens, top_k, expert_count)
     workspace = torch.empty((need,), device=device, dtype=torch.uint8)
-    with torch.cuda.device(device):
+    with _native.device_guard(device):
         _native.call("koemi_moe_permute_hash_indices", ids.contiguous().data_ptr(), prev.contiguous().data_ptr(),
                      _native.dtype_code(ids.dtype), valid_mask.reshape(-1).contiguous().data_ptr(),
                      sorted_rows.data_ptr(), sorted_experts.data_ptr(), segment_offsets.data_ptr(),
@@ -673,7 +682,7 @@ def grouped_expert_mlp_indexed(
     workspace_bytes = _native.query("koemi_moe_grouped_mlp_workspace_bytes", pairs, input_width, hidden_width,
                                     expert_count, _native.dtype_code(torch.bfloat16))
     workspace = torch.empty((workspace_bytes,), device=context.device, dtype=torch.uint8)
-    with torch.cuda.device(context.device):
+    with _native.device_guard(context.device):
         _native.call("koemi_moe_grouped_mlp_indexed", x.data_ptr(), int(x.shape[0]), sorted_rows.data_ptr(),
                      segment_offsets.data_ptr(), *(w.data_ptr() for w in weights), output.data_ptr(), pairs,
                      input_width, hidden_width, expert_count, workspace.data_ptr(), workspace_bytes,
@@ -700,7 +709,7 @@ def weights_to_fragments(weights: Tensor) -> Tensor:
     _require_library()
     src = _aligned(weights.contiguous())
     out = torch.empty_like(src)
-    with torch.cuda.device(weights.device):
+    with _native.device_guard(weights.device):
         _native.call("koemi_moe_weights_to_fragments", src.data_ptr(), out.data_ptr(), matrices, rows, cols,
                      _native.stream_of(weights.device))
     return out
@@ -743,7 +752,7 @@ def grouped_expert_mlp_fragments(
     workspace_bytes = _native.query("koemi_moe_grouped_mlp_workspace_bytes", pairs, input_width, hidden_width,
                                     expert_count, _native.dtype_code(torch.bfloat16))
     workspace = torch.empty((workspace_bytes,), device=context.device, dtype=torch.uint8)
-    with torch.cuda.device(context.device):
+    with _native.device_guard(context.device):
         _native.call("koemi_moe_grouped_mlp_fragments", x.data_ptr(), int(x.shape[0]), sorted_rows.data_ptr(),
                      segment_offsets.data_ptr(), *(w.data_ptr() for w in weights), output.data_ptr(), pairs,
                      input_width, hidden_width, expert_count, workspace.data_ptr(), workspace_bytes,
@@ -792,20 +801,17 @@ def combine_topk(
     _require_library()
     pairs = int(expert_outputs.shape[0])
     if validate:
-        valid_pair_count = int(segment_offsets[-1].item())
-        if valid_pair_count < 0 or valid_pair_count > pairs:
+        outside, bad, _ = _segment_flags(sorted_rows, segment_offsets, token_count)
+        if outside:
             raise CudaMoeValidationError("segment_offsets final value is outside pair_count")
-        if valid_pair_count:
-            selected = sorted_rows[:valid_pair_count]
-            bad = torch.stack(((selected < 0).any(), (selected >= token_count).any())).tolist()
-            if any(bad):
-                raise CudaMoeValidationError("sorted rows are outside token_count")
+        if bad:
+            raise CudaMoeValidationError("sorted rows are outside token_count")
     width = int(expert_outputs.shape[1])
     y = _aligned(expert_outputs)
     combined = torch.empty((token_count, width), device=expert_outputs.device, dtype=expert_outputs.dtype)
     workspace_bytes = _native.query("koemi_moe_combine_workspace_bytes", token_count, top_k)
     workspace = torch.empty((workspace_bytes,), device=expert_outputs.device, dtype=torch.uint8)
-    with torch.cuda.device(expert_outputs.device):
+    with _native.device_guard(expert_outputs.device):
         _native.call(
             "koemi_moe_combine",
             y.data_ptr(),

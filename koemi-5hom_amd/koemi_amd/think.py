@@ -79,7 +79,7 @@ def _rows_forward(logits: Tensor, bias: Tensor | None, targets: Tensor, valid: T
     out = torch.empty((rows,), device=logits.device, dtype=out_dtype)
     if rows == 0:
         return out
-    with torch.cuda.device(logits.device):
+    with _native.device_guard(logits.device):
         _native.call(
             "koemi_surprise_rows_forward",
             logits.data_ptr(),
@@ -103,7 +103,7 @@ def _rows_backward(
     grad_logits = torch.empty_like(logits)
     if rows == 0:
         return grad_logits
-    with torch.cuda.device(logits.device):
+    with _native.device_guard(logits.device):
         _native.call(
             "koemi_surprise_rows_backward",
             logits.data_ptr(),
@@ -130,7 +130,7 @@ def _head_forward(prior: Tensor, weight: Tensor, bias: Tensor, targets: Tensor, 
     stats = torch.empty((3, rows), device=prior.device, dtype=torch.float32)
     need = _native.query("koemi_surprise_head_forward_workspace_bytes", rows, vocab)
     workspace = torch.empty((need,), device=prior.device, dtype=torch.uint8) if need else None
-    with torch.cuda.device(prior.device):
+    with _native.device_guard(prior.device):
         _native.call("koemi_surprise_head_forward", prior.data_ptr(), weight.data_ptr(), bias.data_ptr(),
                      targets.data_ptr(), valid.data_ptr(), out.data_ptr(), stats.data_ptr(), rows, width, vocab,
                      _log_vocab(vocab), _native.dtype_code(prior.dtype), _native.ptr(workspace), need,
@@ -145,7 +145,7 @@ def _head_backward(prior: Tensor, weight: Tensor, bias: Tensor, targets: Tensor,
     grads = tuple(torch.empty_like(t) for t in (prior, weight, bias))
     need = _native.query("koemi_surprise_head_backward_workspace_bytes", rows, width, vocab)
     workspace = torch.empty((need,), device=prior.device, dtype=torch.uint8)
-    with torch.cuda.device(prior.device):
+    with _native.device_guard(prior.device):
         _native.call("koemi_surprise_head_backward", prior.data_ptr(), weight.data_ptr(), bias.data_ptr(),
                      targets.data_ptr(), valid.data_ptr(), stats.data_ptr(), gradient.data_ptr(),
                      *(t.data_ptr() for t in grads), rows, width, vocab, _log_vocab(vocab),
@@ -433,7 +433,7 @@ def salience_admission(
     count = scores.numel()
     admission = torch.empty((count,), device=scores.device, dtype=torch.bool)
     tau = torch.empty((), device=scores.device, dtype=torch.float32)
-    with torch.cuda.device(scores.device):
+    with _native.device_guard(scores.device):
         stream = _native.stream_of(scores.device)
         if threshold is not None:
             if isinstance(threshold, bool) or not isinstance(threshold, (int, float)):

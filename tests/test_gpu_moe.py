@@ -605,3 +605,24 @@ def test_grouped_mlp_any_shape_subnormals_and_infinities(device, dtype):
     rows = [r for r in range(70, 110) if r != 100]
     assert torch.equal(got[rows], clean.cpu()[rows])
     assert not torch.isfinite(got[100]).all() or dtype == torch.float16
+
+
+@pytest.mark.parametrize("pairs, offsets, limit, changes", [
+    (0, [0], 0, {}), (0, [0, 0], 1, {}), (5, [0, 2, 5], 3, {}), (5, [0, 2, 6], 3, {}), (5, [0, 2, -1], 3, {}),
+    (5, [0, 3, 2, 5], 3, {}), (5, [-1, 3, 5], 3, {}), (5, [0, 2, 4], 3, {4: 9}), (5, [0, 2, 4], 3, {3: 9}),
+    (5, [0, 2, 4], 3, {0: -1}), (9000, [0, 4000, 9000], 7, {8999: 7}), (300000, [0, 100, 299999], 7, {299999: 7}),
+    (300000, [0, 100, 300000], 7, {299999: 7}), (5, [0] * 3000 + [-2] + [5], 3, {}),
+])
+def test_segment_check_equals_the_torch_expressions(device, pairs, offsets, limit, changes):
+    """The one-launch check of sorted pairs against the expressions of the reference's fronts."""
+
+    ids = torch.arange(pairs, dtype=torch.int64) % max(limit, 1)
+    for index, value in changes.items():
+        ids[index] = value
+    valid = offsets[-1]
+    outside = valid < 0 or valid > pairs
+    selected = ids[:0] if outside else ids[:valid]
+    bad = bool(((selected < 0) | (selected >= limit)).any())
+    unordered = any(b < a for a, b in zip(offsets, offsets[1:])) or offsets[0] < 0
+    got = moe._segment_flags(ids.to(device), torch.tensor(offsets, device=device), limit)
+    assert got == (outside, bad, unordered)
