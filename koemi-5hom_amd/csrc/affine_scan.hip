@@ -37,42 +37,30 @@ constexpr int kScanSteps = KOEMI_SCAN_STEPS;        // S: serial steps per wave 
 constexpr int kScanSegments = KOEMI_SCAN_SEGMENTS;  // NSEG: waves per workgroup
 
 // Loads are unconditional (the position is clamped into the sequence) and the
-// identity element is selected afterwards: loads under divergent branches would
-// force the compiler to wait for every outstanding load, including the prefetch
-// of the next chunk.
-template <typename T, typename A, int S, bool BCAST>
-__device__ __forceinline__ void scan_load(const T* __restrict__ a_col, const T* __restrict__ b_col,
-                                          int64_t a_stride, int64_t F, int64_t L, int64_t t_first,
-                                          bool col_ok, A (&ra)[S], A (&rb)[S]) {
-    T va[S], vb[S];
-#pragma unroll
-    for (int i = 0; i < S; ++i) {
-        const int64_t t = t_first + i;
-        const int64_t tc = t < L ? t : L - 1;
-        va[i] = a_col[tc * a_stride];
-        vb[i] = b_col[tc * F];
-    }
-#pragma unroll
-    for (int i = 0; i < S; ++i) {
-        const bool ok = col_ok && t_first + i < L;
-        ra[i] = ok ? static_cast<A>(va[i]) : A(1);
-        rb[i] = ok ? static_cast<A>(vb[i]) : A(0);
-    }
-}
-
-template <typename T, int S, int NSEG, bool BCAST>
+// identity element is selected when the chunk is scanned: loads under divergent
+// branches, or selects beside them, would wait for every outstanding load,
+// including the prefetch of the next chunk.
+//
+// LPC > 1 splits each wave into LPC groups of 64 / LPC lanes, each a segment of its
+// own: a workgroup owns 64 / LPC columns and NSEG * LPC segments, so a batch of few
+// columns runs on LPC times the workgroups with LPC times fewer chunks to walk (a
+// chunk costs its latency there). Segments are composed in the same order: the
+// same bits for any LPC. (Two columns per lane, with twice the lane groups, measured
+// the same within 5% where the chip is full and 1.2 to 1.5 times slower where it is
+// not.)
+template <typename T, int S, int NSEG, bool BCAST, int LPC>
 __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
     const T* __restrict__ a, const T* __restrict__ b, const T* __restrict__ h0, T* __restrict__ h,
     int64_t L, int64_t F, int64_t col_tiles) {
     using A = typename AccOf<T>::type;
-    constexpr int CH = S * NSEG;
-    __shared__ A seg_p[NSEG][kWave];
-    __shared__ A seg_b[NSEG][kWave];
+    constexpr int TW = kWave / LPC, NS = NSEG * LPC, CH = S * NS;
+    __shared__ A seg_p[NS][TW];
+    __shared__ A seg_b[NS][TW];
 
-    const int lane = lane_id();
-    const int seg = static_cast<int>(threadIdx.x) / kWave;
+    const int lane = lane_id() % TW;
+    const int seg = static_cast<int>(threadIdx.x) / TW;
     const int64_t bi = static_cast<int64_t>(blockIdx.x) / col_tiles;
-    const int64_t f = (static_cast<int64_t>(blockIdx.x) % col_tiles) * kWave + lane;
+    const int64_t f = (static_cast<int64_t>(blockIdx.x) % col_tiles) * TW + lane;
     const bool col_ok = f < F;
     const int64_t fc = col_ok ? f : 0;
 
@@ -83,15 +71,31 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
 
     A carry = col_ok ? static_cast<A>(h0[bi * F + fc]) : A(0);
 
-    // Scan one chunk held in (ra, rb), starting at t0, and write its states.
-    auto process = [&](A (&ra)[S], A (&rb)[S], int64_t t0) {
+    struct Raw {
+        T a[S], b[S];
+    };
+    auto fetch = [&](int64_t t_first, Raw& raw) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const int64_t t = t_first + i;
+            const int64_t tc = t < L ? t : L - 1;
+            raw.a[i] = a_col[tc * a_stride];
+            raw.b[i] = b_col[tc * F];
+        }
+    };
+    // Scan one chunk, starting at t0, and write its states.
+    auto process = [&](const Raw& raw, int64_t t0) {
         const int64_t t_seg = t0 + static_cast<int64_t>(seg) * S;
+        A ra[S], rb[S];
         // Segment-local inclusive scan from a zero state: (prod a, local h).
         A p = A(1), q = A(0);
 #pragma unroll
         for (int i = 0; i < S; ++i) {
-            q = ra[i] * q + rb[i];
-            p = p * ra[i];
+            const bool ok = col_ok && t_seg + i < L;
+            const A av = ok ? static_cast<A>(raw.a[i]) : A(1);
+            const A bv = ok ? static_cast<A>(raw.b[i]) : A(0);
+            q = av * q + bv;
+            p = p * av;
             ra[i] = p;
             rb[i] = q;
         }
@@ -100,8 +104,8 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
         __syncthreads();
         // Compose the carried state through the segments before this one.
         A c = carry, c_in = carry;
-#pragma unroll
-        for (int j = 0; j < NSEG; ++j) {
+#pragma unroll 8  // all of them at once would hold every segment's transfer in registers
+        for (int j = 0; j < NS; ++j) {
             if (j == seg) c_in = c;
             c = seg_p[j][lane] * c + seg_b[j][lane];
         }
@@ -118,15 +122,15 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
 
     // Two register buffers, alternated by a two-chunk loop body, so that the
     // next chunk's loads are always in flight while the current one is scanned.
-    A xa[S], xb[S], ya[S], yb[S];
+    Raw x, y;
     const int64_t seg_off = static_cast<int64_t>(seg) * S;
-    scan_load<T, A, S, BCAST>(a_col, b_col, a_stride, F, L, seg_off, col_ok, xa, xb);
+    fetch(seg_off, x);
     for (int64_t t0 = 0; t0 < L; t0 += 2 * CH) {
-        scan_load<T, A, S, BCAST>(a_col, b_col, a_stride, F, L, t0 + CH + seg_off, col_ok, ya, yb);
-        process(xa, xb, t0);
+        fetch(t0 + CH + seg_off, y);
+        process(x, t0);
         if (t0 + CH >= L) break;
-        scan_load<T, A, S, BCAST>(a_col, b_col, a_stride, F, L, t0 + 2 * CH + seg_off, col_ok, xa, xb);
-        process(ya, yb, t0 + CH);
+        fetch(t0 + 2 * CH + seg_off, x);
+        process(y, t0 + CH);
     }
 }
 
@@ -506,57 +510,59 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_wide_kernel(
 // Reverse-time adjoint of the scan (dense/affine_scan.cu:58-106):
 //   g_t = dh_t + a_{t+1} g_{t+1},  db_t = g_t,  da_t = g_t h_{t-1},  dh0 = a_0 g_0.
 // In reversed time u = L-1-t this is a forward scan with coefficient a_{t+1}
-// and increment dh_t, so it reuses the same two-level structure.
-template <typename T, int S, int NSEG, bool BCAST>
+// and increment dh_t, so it reuses the same two-level structure, lane groups
+// included, and keeps the next chunk's loads in flight as they come from memory
+// (they are widened when their chunk is scanned).
+template <typename T, int S, int NSEG, bool BCAST, int LPC>
 __global__ __launch_bounds__(kWave * NSEG) void scan_backward_kernel(
     const T* __restrict__ a, const T* __restrict__ h0, const T* __restrict__ h,
     const T* __restrict__ dh, T* __restrict__ da, T* __restrict__ db, T* __restrict__ dh0,
     int64_t L, int64_t F, int64_t col_tiles) {
     using A = typename AccOf<T>::type;
-    constexpr int CH = S * NSEG;
-    __shared__ A seg_p[NSEG][kWave];
-    __shared__ A seg_b[NSEG][kWave];
+    constexpr int TW = kWave / LPC, NS = NSEG * LPC, CH = S * NS;
+    __shared__ A seg_p[NS][TW];
+    __shared__ A seg_b[NS][TW];
 
-    const int lane = lane_id();
-    const int seg = static_cast<int>(threadIdx.x) / kWave;
+    const int lane = lane_id() % TW;
+    const int seg = static_cast<int>(threadIdx.x) / TW;
     const int64_t bi = static_cast<int64_t>(blockIdx.x) / col_tiles;
-    const int64_t f = (static_cast<int64_t>(blockIdx.x) % col_tiles) * kWave + lane;
+    const int64_t f = (static_cast<int64_t>(blockIdx.x) % col_tiles) * TW + lane;
     const bool col_ok = f < F;
     const int64_t fc = col_ok ? f : 0;
 
     const T* a_col = BCAST ? a + bi * L : a + bi * L * F + fc;
     const int64_t a_stride = BCAST ? 1 : F;
     const int64_t base = bi * L * F + fc;
-    const A h_init = col_ok ? static_cast<A>(h0[bi * F + fc]) : A(0);
+    const T h_init = h0[bi * F + fc];
 
     A carry = A(0);
-    for (int64_t u0 = 0; u0 < L; u0 += CH) {
-        const int64_t u_seg = u0 + static_cast<int64_t>(seg) * S;
-        A ra[S], rb[S], hp[S];
-        T va[S], vg[S], vh[S];
+    struct Raw {
+        T a[S], g[S], h[S];
+    };
+    auto fetch = [&](int64_t u_seg, Raw& raw) {
 #pragma unroll
-        for (int i = 0; i < S; ++i) {  // unconditional, clamped loads (see scan_load)
+        for (int i = 0; i < S; ++i) {
             const int64_t t = L - 1 - (u_seg + i);
             const int64_t tc = t < 0 ? 0 : t;
             const int64_t ta = tc + 1 < L ? tc + 1 : L - 1;
             const int64_t tp = tc > 0 ? tc - 1 : 0;
-            va[i] = a_col[ta * a_stride];
-            vg[i] = dh[base + tc * F];
-            vh[i] = h[base + tp * F];
+            raw.a[i] = a_col[ta * a_stride];
+            raw.g[i] = dh[base + tc * F];
+            raw.h[i] = h[base + tp * F];
         }
+    };
+    auto process = [&](const Raw& raw, int64_t u0) {
+        const int64_t u_seg = u0 + static_cast<int64_t>(seg) * S;
+        A ra[S], rb[S];
+        A p = A(1), q = A(0);
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const int64_t t = L - 1 - (u_seg + i);
             const bool ok = col_ok && t >= 0;
-            ra[i] = (ok && t + 1 < L) ? static_cast<A>(va[i]) : A(1);
-            rb[i] = ok ? static_cast<A>(vg[i]) : A(0);
-            hp[i] = ok ? (t > 0 ? static_cast<A>(vh[i]) : h_init) : A(0);
-        }
-        A p = A(1), q = A(0);
-#pragma unroll
-        for (int i = 0; i < S; ++i) {
-            q = ra[i] * q + rb[i];
-            p = p * ra[i];
+            const A av = (ok && t + 1 < L) ? static_cast<A>(raw.a[i]) : A(1);
+            const A gv = ok ? static_cast<A>(raw.g[i]) : A(0);
+            q = av * q + gv;
+            p = p * av;
             ra[i] = p;
             rb[i] = q;
         }
@@ -564,8 +570,8 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_backward_kernel(
         seg_b[seg][lane] = q;
         __syncthreads();
         A c = carry, c_in = carry;
-#pragma unroll
-        for (int j = 0; j < NSEG; ++j) {
+#pragma unroll 8
+        for (int j = 0; j < NS; ++j) {
             if (j == seg) c_in = c;
             c = seg_p[j][lane] * c + seg_b[j][lane];
         }
@@ -574,14 +580,24 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_backward_kernel(
 #pragma unroll
             for (int i = 0; i < S; ++i) {
                 const int64_t t = L - 1 - (u_seg + i);
+                const A g = ra[i] * c_in + rb[i];
                 if (t >= 0) {
-                    const A g = ra[i] * c_in + rb[i];
                     db[base + t * F] = static_cast<T>(g);
-                    da[base + t * F] = static_cast<T>(g * hp[i]);
+                    da[base + t * F] = static_cast<T>(g * static_cast<A>(t > 0 ? raw.h[i] : h_init));
                 }
             }
         }
         __syncthreads();
+    };
+    const int64_t seg_off = static_cast<int64_t>(seg) * S;
+    Raw x, y;
+    fetch(seg_off, x);
+    for (int64_t u0 = 0; u0 < L; u0 += 2 * CH) {
+        fetch(u0 + CH + seg_off, y);
+        process(x, u0);
+        if (u0 + CH >= L) break;
+        fetch(u0 + 2 * CH + seg_off, x);
+        process(y, u0 + CH);
     }
     if (col_ok && seg == 0) {
         dh0[bi * F + fc] = static_cast<T>(static_cast<A>(a_col[0]) * carry);
@@ -591,6 +607,20 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_backward_kernel(
 #ifndef KOEMI_SCAN_VEC
 #define KOEMI_SCAN_VEC 2
 #endif
+
+// Lane groups of the general kernels: more of them while the column strips leave
+// CUs without a workgroup and a chunk is still shorter than the sequence. Forward +
+// backward, us: [4, 1024, 256] fp32 21 + 35 at one group, 13 + 17 at eight; [1, 4096,
+// 300] 70 + 137 and 31 + 46; [8, 2048, 1024] 56 + 105 at one (the backward without
+// the prefetch), 50 + 67 at two, but 67 + 108 at four: past one workgroup per CU the
+// narrower strips only cost.
+inline int lane_groups(int64_t B, int64_t L, int64_t F) {
+    int lpc = 1;
+    while (lpc < 8 && B * ((F + kWave / lpc - 1) / (kWave / lpc)) < 256 &&
+           static_cast<int64_t>(kScanSteps) * kScanSegments * lpc < L)
+        lpc *= 2;
+    return lpc;
+}
 
 template <typename T, bool BCAST>
 int launch_forward(const void* a, const void* b, const void* h0, void* h, int64_t B, int64_t L,
@@ -619,30 +649,41 @@ int launch_forward(const void* a, const void* b, const void* h0, void* h, int64_
             return check_launch("koemi_affine_scan_forward");
         }
     }
-    const int64_t col_tiles = (F + kWave - 1) / kWave;
-    const int64_t blocks = B * col_tiles;
-    if (blocks > 0x7fffffff) return fail(KOEMI_ERR_UNSUPPORTED, "affine scan grid too large");
-    hipLaunchKernelGGL((scan_forward_kernel<T, kScanSteps, kScanSegments, BCAST>),
-                       dim3(static_cast<unsigned>(blocks)), dim3(kWave * kScanSegments), 0, stream,
-                       static_cast<const T*>(a), static_cast<const T*>(b),
-                       static_cast<const T*>(h0), static_cast<T*>(h), L, F, col_tiles);
-    return check_launch("koemi_affine_scan_forward");
+    const auto run = [&](auto kernel, int64_t columns) {
+        const int64_t col_tiles = (F + columns - 1) / columns;
+        if (B * col_tiles > 0x7fffffff) return fail(KOEMI_ERR_UNSUPPORTED, "affine scan grid too large");
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(B * col_tiles)), dim3(kWave * kScanSegments), 0, stream,
+                           static_cast<const T*>(a), static_cast<const T*>(b), static_cast<const T*>(h0),
+                           static_cast<T*>(h), L, F, col_tiles);
+        return check_launch("koemi_affine_scan_forward");
+    };
+    switch (lane_groups(B, L, F)) {
+        case 1: return run(scan_forward_kernel<T, kScanSteps, kScanSegments, BCAST, 1>, kWave);
+        case 2: return run(scan_forward_kernel<T, kScanSteps, kScanSegments, BCAST, 2>, kWave / 2);
+        case 4: return run(scan_forward_kernel<T, kScanSteps, kScanSegments, BCAST, 4>, kWave / 4);
+        default: return run(scan_forward_kernel<T, kScanSteps, kScanSegments, BCAST, 8>, kWave / 8);
+    }
 }
 
 template <typename T, bool BCAST>
 int launch_backward(const void* a, const void* h0, const void* h, const void* dh, void* da,
                     void* db, void* dh0, int64_t B, int64_t L, int64_t F, hipStream_t stream) {
-    const int64_t col_tiles = (F + kWave - 1) / kWave;
-    const int64_t blocks = B * col_tiles;
-    if (blocks > 0x7fffffff) return fail(KOEMI_ERR_UNSUPPORTED, "affine scan grid too large");
-    hipLaunchKernelGGL((scan_backward_kernel<T, kScanSteps, kScanSegments, BCAST>),
-                       dim3(static_cast<unsigned>(blocks)), dim3(kWave * kScanSegments), 0, stream,
-                       static_cast<const T*>(a), static_cast<const T*>(h0),
-                       static_cast<const T*>(h), static_cast<const T*>(dh), static_cast<T*>(da),
-                       static_cast<T*>(db), static_cast<T*>(dh0), L, F, col_tiles);
-    return check_launch("koemi_affine_scan_backward");
+    const auto run = [&](auto kernel, int64_t columns) {
+        const int64_t col_tiles = (F + columns - 1) / columns;
+        if (B * col_tiles > 0x7fffffff) return fail(KOEMI_ERR_UNSUPPORTED, "affine scan grid too large");
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(B * col_tiles)), dim3(kWave * kScanSegments), 0, stream,
+                           static_cast<const T*>(a), static_cast<const T*>(h0), static_cast<const T*>(h),
+                           static_cast<const T*>(dh), static_cast<T*>(da), static_cast<T*>(db), static_cast<T*>(dh0), L,
+                           F, col_tiles);
+        return check_launch("koemi_affine_scan_backward");
+    };
+    switch (lane_groups(B, L, F)) {
+        case 1: return run(scan_backward_kernel<T, kScanSteps, kScanSegments, BCAST, 1>, kWave);
+        case 2: return run(scan_backward_kernel<T, kScanSteps, kScanSegments, BCAST, 2>, kWave / 2);
+        case 4: return run(scan_backward_kernel<T, kScanSteps, kScanSegments, BCAST, 4>, kWave / 4);
+        default: return run(scan_backward_kernel<T, kScanSteps, kScanSegments, BCAST, 8>, kWave / 8);
+    }
 }
-
 int check_scan_args(const void* a, const void* b, const void* h0, const void* h, int64_t B,
                     int64_t L, int64_t F, int dtype) {
     if (B < 0 || L < 0 || F < 0) return fail(KOEMI_ERR_INVALID, "affine scan sizes must be non-negative");

@@ -145,9 +145,9 @@ def scan_backward(
     _load()
     gradient_retention = torch.empty_like(states)
     gradient_increment = torch.empty_like(states)
-    gradient_initial = torch.zeros_like(initial)
     if states.numel() == 0:
-        return gradient_retention, gradient_increment, gradient_initial
+        return gradient_retention, gradient_increment, torch.zeros_like(initial)
+    gradient_initial = torch.empty_like(initial)
     batch, sequence, features = _geometry(states)
     broadcast = retention.numel() == batch * sequence
     with _native.device_guard(states.device):

@@ -10,6 +10,7 @@ the max abs / rel errors are printed.
 from __future__ import annotations
 
 import json
+import math
 from pathlib import Path
 
 import numpy as np
@@ -144,3 +145,34 @@ def test_config3_full_against_the_oracle(device):
     # chunk 64 through the model-path seam gives the same states
     chunked = cuda_scan.cuda_affine_scan(c.retention[:2].to(device), c.increment[:2].to(device), chunk_size=c.chunk)
     np.testing.assert_array_equal(chunked.cpu().numpy(), got[:2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("broadcast", [False, True])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 64, 7), (2, 65, 9), (1, 129, 33), (5, 257, 17), (2, 513, 64), (1, 1100, 200),
+                                   (70, 200, 100), (300, 130, 5)])
+def test_lane_groups(device, dtype, broadcast, shape):
+    """Forward and gradients where the columns are few (one to eight lane groups per wave, chunks longer
+    than, equal to and shorter than the sequence) against the sequential recurrence in float64.
+    fp32 within 1e-5 (tests/cuda/test_dense_cuda.py:78), float64 1e-12; 16-bit results within their rounding
+    of the states (half an ulp) and of the products formed from the rounded states."""
+
+    b, l, f = shape
+    g = torch.Generator().manual_seed(b * 101 + l * 7 + f)
+    a = torch.sigmoid(torch.randn((b, l, 1 if broadcast else f), generator=g) + 1.0).to(dtype)
+    x = (0.5 * torch.randn((b, l, f), generator=g)).to(dtype)
+    h0 = torch.randn((b, f), generator=g).to(dtype)
+    up = torch.randn((b, l, f), generator=g).to(dtype)
+    leaves = [t.to(device).requires_grad_() for t in (a, x, h0)]
+    states = dense_affine_scan(*leaves)
+    grads = torch.autograd.grad(states, leaves, up.to(device))
+    a64, x64, h64 = (t.double().requires_grad_() for t in (a, x, h0))
+    want = sequential_torch(a64, x64, h64)
+    want_grads = torch.autograd.grad(want, (a64, x64, h64), up.double())
+    tol = {torch.float32: 1e-5, torch.float64: 1e-12, torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[dtype]
+    for got, ref in zip((states, *grads), (want, *want_grads)):
+        got, ref = got.detach().double().cpu(), ref.detach()
+        scale = 1.0 + ref.abs().max()
+        if broadcast and ref is want_grads[0]:
+            scale = scale * math.sqrt(f)  # a sum over the features of rounded products
+        assert bool(((got - ref).abs() <= tol * (ref.abs() + scale)).all())
