@@ -8,14 +8,17 @@
 //   b = (1 - a) * tanh(u W_c^T + b_c)
 //   invalid positions (valid mask given and false): a = 1, b = 0
 //
-// The two width x width products are plain GEMMs and run on rocBLAS (fp32
-// accumulation, fp32 results in the workspace); one HIP kernel then applies
+// The two width x width products leave fp32 results in the workspace: fp32 inputs
+// on the matrix cores as split bf16 planes (split_gemm.hpp; fp32 accumulation, the
+// products as exact as fp32 ones), 16-bit ones and a few rows as plain GEMMs on rocBLAS. One HIP
+// kernel then applies
 // the biases, the bounded sigmoid, tanh and the mask and writes a and b in the
 // input dtype, reading each fp32 product once (16-byte loads, four columns per
 // thread). koemi_recurrent_scan (fp32) hands the two products straight to the
 // affine-scan kernel, which applies the same expressions in registers, so a
 // and b never reach memory.
 #include "common.hpp"
+#include "split_gemm.hpp"
 
 #include <rocblas/rocblas.h>
 
@@ -58,11 +61,7 @@ __global__ __launch_bounds__(256) void gates_epilogue_kernel(
 }
 
 rocblas_datatype gates_blas_type(int dtype) {
-    switch (dtype) {
-        case KOEMI_F16: return rocblas_datatype_f16_r;
-        case KOEMI_BF16: return rocblas_datatype_bf16_r;
-        default: return rocblas_datatype_f32_r;
-    }
+    return dtype == KOEMI_F16 ? rocblas_datatype_f16_r : dtype == KOEMI_BF16 ? rocblas_datatype_bf16_r : rocblas_datatype_f32_r;
 }
 
 size_t gates_workspace(int64_t rows, int64_t D) {
@@ -70,10 +69,91 @@ size_t gates_workspace(int64_t rows, int64_t D) {
     return 2 * one;
 }
 
-// zr = u W_r^T, zc = u W_c^T (row-major [rows, D], fp32) on rocBLAS: in its
+// zr = u W_r^T, zc = u W_c^T for fp32: B x B tiles, a tile's columns all of one
+// product. Workgroup b runs on XCD b % 8; an XCD takes a contiguous range of tiles,
+// four row blocks at a time over every column, so that its L2 serves the rows and
+// weights that concurrently running tiles share. Bound by the matrix cores (six
+// bf16 products an fp32 one) and the splits beside them: [16384, 1024] with its scan
+// 387 us against 559 with rocBLAS's fp32 products (about 325 us of it, 210 TFLOP/s,
+// 1.27 PFLOP/s counting six), its error against float64 4.5e-7 against 5.1e-7.
+template <int B, int BYTES>
+__global__ __launch_bounds__(split_gemm::kThreads, 2) void gate_products_kernel(
+    const float* __restrict__ u, const float* __restrict__ wr, const float* __restrict__ wc, float* __restrict__ zr,
+    float* __restrict__ zc, int64_t rows, int64_t D, uint32_t row_tiles, uint32_t half_tiles) {
+    using Tile = split_gemm::Tile<float, float, B, B, false, false, B == 64 ? 4 : 1>;
+    constexpr int kRegion = split_gemm::store_bytes<float, 1>();
+    static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
+    constexpr uint32_t kGroup = 4;
+    const uint32_t columns = 2 * half_tiles, tiles = row_tiles * columns, per_xcd = (tiles + 7) / 8;
+    if ((blockIdx.x >> 3) >= per_xcd) return;
+    const uint32_t logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (logical >= tiles) return;
+    const uint32_t first = logical / (kGroup * columns) * kGroup;
+    const uint32_t group = min(kGroup, row_tiles - first), within = logical % (kGroup * columns);
+    const uint32_t column = within / group;
+    const int64_t row0 = static_cast<int64_t>(first + within % group) * B;
+    const int64_t n0 = static_cast<int64_t>(column % half_tiles) * B;
+    const float* w = column < half_tiles ? wr : wc;
+    float* z = column < half_tiles ? zr : zc;
+    const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
+    Tile tile;
+    tile.template run<BYTES, BYTES>(
+        lds, D, D, 0, (D + Tile::BK - 1) / Tile::BK * Tile::BK, [&](int r) { return u + min(row0 + r, rows - 1) * D; },
+        [&](int r) { return w + min(n0 + r, D - 1) * D; }, [&](int t) { return wn * (B / 2) + t * 32; });
+    split_gemm::lds_barrier();  // the output rows pass through LDS
+#pragma unroll
+    for (int i = 0; i < Tile::MT; ++i) {
+        const int64_t block_row = row0 + wm * (B / 2) + i * 32;
+#pragma unroll
+        for (int j = 0; j < Tile::NT; ++j) {
+            const int64_t c0 = n0 + wn * (B / 2) + j * 32;
+            float o[1][16];
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[0][v] = tile.acc[i][j][v];
+            float* out = z + block_row * D + c0;
+            split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, D, rows - block_row, D - c0, D % 8 == 0);
+            split_gemm::fix_not_finite(o, [&](int, int v) {
+                const int r = lane_id() & 31, c = split_gemm::acc_column(v);
+                if (block_row + r < rows && c0 + c < D)
+                    out[r * D + c] = split_gemm::scalar_dot(u + (block_row + r) * D, w + (c0 + c) * D, D, 0.0f);
+            });
+        }
+    }
+}
+
+int gate_products_f32(const float* u, const float* wr, const float* wc, float* zr, float* zc, int64_t rows, int64_t D,
+                      hipStream_t s) {
+    // 64 x 64 tiles with four K steps of loads in flight where the 128 x 128 ones would
+    // give fewer than one to each CU (168 rows x 512 with its scan: 28 -> 19 us)
+    const int64_t b = (rows + 127) / 128 * 2 * ((D + 127) / 128) < 256 ? 64 : 128;
+    const int64_t row_tiles = (rows + b - 1) / b, half_tiles = (D + b - 1) / b;
+    const int64_t blocks = (row_tiles * half_tiles * 2 + 7) / 8 * 8;
+    if (blocks > 0x7fffffffLL) return fail(KOEMI_ERR_UNSUPPORTED, "recurrent gates sizes exceed the grid");
+    // D is a multiple of 4, so rows start 16-byte aligned where the bases do; a base
+    // from a C caller may not
+    const auto bytes = [&](const void* p) { return split_gemm::load_bytes<float>(p, D); };
+    const bool wide = bytes(u) == 16 && bytes(wr) == 16 && bytes(wc) == 16;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(split_gemm::kThreads), 0, s, u, wr, wc, zr,
+                           zc, rows, D, static_cast<uint32_t>(row_tiles), static_cast<uint32_t>(half_tiles));
+        return check_launch("recurrent gates (products)");
+    };
+    if (b == 128) return wide ? run(gate_products_kernel<128, 16>) : run(gate_products_kernel<128, 0>);
+    return wide ? run(gate_products_kernel<64, 16>) : run(gate_products_kernel<64, 0>);
+}
+
+// zr = u W_r^T, zc = u W_c^T (row-major [rows, D], fp32); 16-bit inputs and a few rows on rocBLAS: in its
 // column-major terms Z' (D x rows) = W'^T (D x D) . u' (D x rows).
 int gate_products(const void* input, const void* retention_weight, const void* candidate_weight, float* zr,
                   float* zc, int64_t rows, int64_t width, int dtype, hipStream_t s) {
+    // a few rows of a wide product leave most CUs idle for a long walk over K: there
+    // rocBLAS's smaller tiles are as fast (32 rows x 1024: 28 us with the scan, 30 on
+    // these tiles; 168 x 512: 28 and 21)
+    const bool few = (rows + 63) / 64 * 2 * ((width + 63) / 64) < 64 && width > 768;
+    if (dtype == KOEMI_F32 && !few)
+        return gate_products_f32(static_cast<const float*>(input), static_cast<const float*>(retention_weight),
+                                 static_cast<const float*>(candidate_weight), zr, zc, rows, width, s);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fail(KOEMI_ERR_LAUNCH, "recurrent gates: no device");
     std::lock_guard<std::mutex> lock(g_blas_mutex);

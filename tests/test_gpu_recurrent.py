@@ -373,3 +373,38 @@ def test_recurrent_gates_reject_bad_inputs(device):
         recurrent.recurrent_gates(u, wr[:4], br, wc, bc)
     with pytest.raises(dense.DenseCudaValidationError, match="valid_mask"):
         recurrent.recurrent_gates(u, wr, br, wc, bc, valid[:, :2])
+
+
+@pytest.mark.parametrize("rows, width", [(1, 4), (63, 60), (65, 64), (130, 132), (300, 516), (64, 1028), (70, 1028), (5000, 128), (4100, 260)])
+def test_fp32_gate_products_of_every_tile_shape(device, rows, width):
+    """The fp32 gates at the edges of the products' tiles (64 and 128 rows and columns, K remainders, the
+    library's few rows of a wide product) against float64, with rows that hold infinities and NaN.
+
+    dz = 4 sqrt(D) 2^-24 sum |terms| for a pre-activation's fp32 sum; the sigmoid and tanh add 1.5e-7 and
+    2.5e-7 (absolute), their slopes are at most 1/4 and 1, and a few roundings of values up to 1 are 2^-22."""
+
+    g = torch.Generator().manual_seed(rows * 31 + width)
+    u = torch.randn((rows, width), generator=g)
+    wr, wc = (torch.randn((width, width), generator=g) / width**0.5 for _ in range(2))
+    br, bc = (0.1 * torch.randn((width,), generator=g) for _ in range(2))
+    got = recurrent.recurrent_gates(*(t.to(device) for t in (u, wr, br, wc, bc)))
+    zr, zc = (u.double() @ w.double().t() + b.double() for w, b in ((wr, br), (wc, bc)))
+    a = 2.0**-8 + (1 - 2.0**-7) * torch.sigmoid(zr)
+    want = (a, (1 - a) * torch.tanh(zc))
+    dr, dc = (4 * width**0.5 * 2.0**-24 * (u.double().abs() @ w.double().abs().t() + b.double().abs()) for w, b in ((wr, br), (wc, bc)))
+    bounds = (dr / 4 + 1.5e-7 + 2.0**-22, dr / 4 + dc + 4e-7 + 2.0**-22)
+    for have, ref, bound in zip(got, want, bounds):
+        err = (have.double().cpu() - ref).abs()
+        assert bool((err <= bound).all()), float((err / bound).max())
+    bad = u.clone()
+    bad[0, 0] = float("inf")
+    bad[rows // 2, width - 1] = float("nan") if rows > 1 else float("inf")
+    touched = {0, rows // 2}
+    out = recurrent.recurrent_gates(*(t.to(device) for t in (bad, wr, br, wc, bc)))
+    keep = [r for r in range(rows) if r not in touched]
+    for have, clean in zip(out, got):
+        assert torch.equal(have[keep], clean[keep])
+    if rows > 1:  # an infinite input saturates the gates by the sign of its weight; NaN stays NaN
+        assert torch.isnan(out[0][rows // 2]).all()
+        sign = wr[:, 0].to(device) > 0
+        assert torch.equal(out[0][0], torch.where(sign, 1 - 2.0**-8, 2.0**-8).float())
