@@ -7,7 +7,7 @@
 // sliding window, novelty = clamp(1 - largest, 0, 1), 1 with no eligible
 // slot) and KoemiModel.refine_memory (network.py:714-721: memory value =
 // fast + sigmoid(W_g [working; fast; refine; local] + b_g) * refine), torch
-// composites in the reference. Both are row-local; one wave per query (the
+// composites in the reference. Both are row-local; one wave per run of queries (the
 // novelty's at most `window` dot products over the width) or per position
 // (the gate's dot product over four widths, then the mix).
 #include "common.hpp"
@@ -67,6 +67,107 @@ __global__ __launch_bounds__(256) void local_novelty_kernel(
     if (lane == 0) novelty[job] = any ? fminf(fmaxf(1.0f - best, 0.0f), 1.0f) : 1.0f;
 }
 
+// N values per lane (a power of two) summed over the wave, in N + 5 - log2 N
+// exchanges instead of 6 N: each halving step sends the half of the values that the
+// partner keeps. Lane l ends with the sum of value l / (64 / N).
+template <int N>
+__device__ __forceinline__ float wave_sum_each(float (&v)[N]) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int n = N / 2, off = 32; n > 0; n >>= 1, off >>= 1) {
+        const bool upper = lane & off;
+#pragma unroll
+        for (int i = 0; i < n; ++i) {
+            const float send = upper ? v[i] : v[i + n];
+            v[i] = (upper ? v[i + n] : v[i]) + __shfl_xor(send, off, kWave);
+        }
+    }
+    float s = v[0];
+#pragma unroll
+    for (int off = kWave / N / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
+    return s;
+}
+
+// Columns [8 lane + 512 g, + 8) of a row, g < NG (zeros past D, a multiple of 8).
+template <int NG, typename T>
+__device__ __forceinline__ void load_columns(const T* __restrict__ row, int64_t D, float (&x)[NG][8]) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int64_t c = 512 * g + 8 * lane_id();
+        const int64_t cc = min(c, D - 8);
+        const float4 a = load4(row + cc), b = load4(row + cc + 4);
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[g][i] = c < D ? v[i] : 0.0f;
+    }
+}
+
+// The novelty of kNoveltyRun consecutive queries of a window row per wave: the
+// queries stay in registers and every key of their joint window is read (and its
+// norm formed) once, the next key's loads under this one's products. Bound by the
+// latency of that walk (window + 3 keys); [64, 128, 1024] at a window of 16, bf16
+// keys: 33 us (52 at runs of eight, 32 at two), against 112 for a wave per query that
+// reads its 16 keys alone.
+constexpr int kNoveltyRun = 4;
+template <typename KT, int NG>
+__global__ __launch_bounds__(256, 2) void local_novelty_run_kernel(
+    const float* __restrict__ carried_keys, const uint8_t* __restrict__ carried_valid, const KT* __restrict__ keys,
+    int64_t key_stride, const uint8_t* __restrict__ key_valid, const float* __restrict__ queries, int64_t q_stride,
+    float* __restrict__ novelty, int64_t rows, int64_t C, int64_t L, int64_t D, int64_t window) {
+    const int64_t runs = (L + kNoveltyRun - 1) / kNoveltyRun;
+    const int64_t job = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;  // (row, run)
+    if (job >= rows * runs) return;
+    const int64_t r = job / runs, t0 = (job - r * runs) * kNoveltyRun;
+    float q[kNoveltyRun][NG][8], sums[kNoveltyRun];
+#pragma unroll
+    for (int j = 0; j < kNoveltyRun; ++j) {
+        load_columns<NG>(queries + (r * L + min(t0 + j, L - 1)) * q_stride, D, q[j]);
+        sums[j] = 0.0f;
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sums[j] = fmaf(q[j][g][i], q[j][g][i], sums[j]);
+    }
+    const float qn = fmaxf(sqrtf(wave_sum_each(sums)), 1e-12f);  // of this lane's query
+    const int64_t t = t0 + lane_id() / (kWave / kNoveltyRun), own = C + t;
+    const int64_t first = max(C + t0 - window, int64_t(0));
+    const int64_t last = C + min(t0 + kNoveltyRun, L) - 1;  // one past the last query's slots
+    auto load_key = [&](int64_t s, float (&k)[NG][8]) {
+        if (s < C) load_columns<NG>(carried_keys + (r * C + s) * D, D, k);
+        else load_columns<NG>(keys + (r * L + (s - C)) * key_stride, D, k);
+    };
+    float best = -INFINITY;
+    bool any = false;
+    float k[NG][8], next[NG][8];
+    if (first < last) load_key(first, next);
+    for (int64_t s = first; s < last; ++s) {  // wave-uniform
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) k[g][i] = next[g][i];
+        load_key(min(s + 1, last - 1), next);
+        if (!(s < C ? carried_valid[r * C + s] : key_valid[r * L + (s - C)])) continue;
+        float kk = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kNoveltyRun; ++j) sums[j] = 0.0f;
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                kk = fmaf(k[g][i], k[g][i], kk);
+#pragma unroll
+                for (int j = 0; j < kNoveltyRun; ++j) sums[j] = fmaf(k[g][i], q[j][g][i], sums[j]);
+            }
+        const float dot = wave_sum_each(sums);
+        kk = wave_sum(kk);
+        if (s < own && s >= own - window) {
+            best = fmaxf(best, dot / (fmaxf(sqrtf(kk), 1e-12f) * qn));
+            any = true;
+        }
+    }
+    if (lane_id() % (kWave / kNoveltyRun) == 0 && t < L) novelty[r * L + t] = any ? fminf(fmaxf(1.0f - best, 0.0f), 1.0f) : 1.0f;
+}
+
 // Position p: pre = sum_k x_k w_k + b over x = [working; fast; refine;
 // local] (LOW: every x_k and w_k rounded to bf16, fp32 accumulation, the sum
 // rounded to bf16 after the bias: nn.Linear under bf16 autocast), g =
@@ -124,6 +225,29 @@ extern "C" int koemi_local_novelty(const float* carried_keys, const uint8_t* car
     if ((jobs + 3) / 4 > 0x7fffffffLL) return fail(KOEMI_ERR_UNSUPPORTED, "local novelty grid too large");
     const dim3 grid(static_cast<unsigned>((jobs + 3) / 4));
     hipStream_t s = as_stream(stream);
+    // Runs of queries where a row fits the registers and every row starts aligned to its
+    // loads (16 bytes of fp32, 8 of bf16); a wave per query otherwise, and for the few
+    // queries of a short window.
+    const auto aligned = [](const void* p, int64_t stride, int64_t size, int64_t to) {
+        return p == nullptr || (reinterpret_cast<uintptr_t>(p) % to == 0 && stride * size % to == 0);
+    };
+    const int64_t key_size = key_dtype == KOEMI_BF16 ? 2 : 4;
+    if (length >= 4 && width % 8 == 0 && width <= 1024 && aligned(carried_keys, width, 4, 16) &&
+        aligned(queries, query_row_stride, 4, 16) && aligned(keys, key_row_stride, key_size, 4 * key_size)) {
+        const int64_t run_jobs = rows * ((length + kNoveltyRun - 1) / kNoveltyRun);
+        const auto run = [&](auto kernel, const auto* typed_keys) {
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((run_jobs + 3) / 4)), dim3(256), 0, s, carried_keys,
+                               carried_valid, typed_keys, key_row_stride, key_valid, queries, query_row_stride, novelty,
+                               rows, capacity, length, width, window);
+            return check_launch("koemi_local_novelty");
+        };
+        if (key_dtype == KOEMI_BF16) {
+            const bf16* k16 = static_cast<const bf16*>(keys);
+            return width <= 512 ? run(local_novelty_run_kernel<bf16, 1>, k16) : run(local_novelty_run_kernel<bf16, 2>, k16);
+        }
+        const float* k32 = static_cast<const float*>(keys);
+        return width <= 512 ? run(local_novelty_run_kernel<float, 1>, k32) : run(local_novelty_run_kernel<float, 2>, k32);
+    }
     if (key_dtype == KOEMI_BF16)
         hipLaunchKernelGGL(local_novelty_kernel<bf16>, grid, dim3(256), 0, s, carried_keys, carried_valid,
                            static_cast<const bf16*>(keys), key_row_stride, key_valid, queries, query_row_stride, novelty,

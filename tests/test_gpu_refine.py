@@ -41,6 +41,10 @@ PAD = herm.PAD_TOKEN_ID
 @pytest.mark.parametrize("rows, cap, length, d, window, key_bf16", [
     (5, 4, 11, 16, 4, False), (3, 16, 40, 64, 16, True), (2, 16, 128, 1024, 16, True), (4, 3, 2, 20, 6, False),
     (3, 0, 9, 8, 3, False),
+    # runs of four queries: one short of, equal to and past a run, widths at a register group's edge and past
+    # the layout, no carried slots, a window longer than the row
+    (3, 16, 7, 504, 16, True), (3, 16, 8, 512, 16, False), (4, 5, 17, 520, 9, True), (2, 0, 33, 1024, 40, True),
+    (2, 16, 13, 1032, 16, True), (2, 3, 5, 12, 4, True), (5, 4, 4, 24, 3, True), (5, 4, 3, 24, 3, True),
 ])
 def test_local_novelty_matches_the_oracle(device, rows, cap, length, d, window, key_bf16):
     rng = np.random.default_rng(rows * 100 + length)
