@@ -30,7 +30,7 @@
 // window's own terms of the final state (fp32 MFMA, K = slots);
 // assoc_window_read_kernel the reads: the causal influence rows of 64 queries
 // (fp32 MFMA, K = features) in LDS, then influence x values plus the carried
-// basis term on MFMA, the denominators as wave reductions. The projection may
+// basis term on MFMA, the denominators by four lanes a row. The projection may
 // be fp32 or bf16 (the GEMM's own output dtype); everything after the load is
 // fp32.
 #include "common.hpp"
@@ -196,9 +196,11 @@ __global__ __launch_bounds__(256) void assoc_prep_kernel(
 // weights: terms[d][m] = sum_s fwt_s tanh(v_s[d]) kf_s[m] on fp32 MFMA (A =
 // the weighted values, 32 columns of a wave's half, B = the key features,
 // K = slots, the slots split in two halves over wave pairs and added through
-// LDS), normalizer terms sum_s fwt_s kf_s[m] by a wave reduction. FINAL
+// LDS), normalizer terms sum_s fwt_s kf_s[m] by groups of lanes. FINAL
 // writes the next state e^{c_{L-1}} state + terms (the fmaf the carry kernel
 // applies between windows); otherwise the terms. Grid (rows, ceil(D / 64)).
+// Latency bounds it (64 slots to a wave's K loop), so eight steps' values are
+// in flight ahead of their use.
 template <int MAXM, bool FINAL, typename PT, bool TANH = true>
 __global__ __launch_bounds__(256) void assoc_delta_kernel(
     const PT* __restrict__ proj, int64_t stride, int64_t value_off, AssocPrep prep,
@@ -213,29 +215,39 @@ __global__ __launch_bounds__(256) void assoc_delta_kernel(
     const int64_t c0 = static_cast<int64_t>(blockIdx.y) * 64;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     const int h = lane >> 5, r32 = lane & 31;
-    for (int s = tid; s < L; s += 256) fwt[s] = prep.fwt[b * L + s];
-    for (int i = tid; i < L * MAXM; i += 256) kf[(i / MAXM) * QP + i % MAXM] = prep.kf[b * L * MAXM + i];
-    __syncthreads();
     const int half = ((L + 1) / 2 + 1) & ~1;
     const int db = wave & 1, kh = wave >> 1;
     const int s_lo = kh * half, s_hi = min(L, s_lo + half);
     const int64_t dv = c0 + db * 32 + r32;
     const PT* vcol = proj + b * L * stride + value_off + (dv < D ? dv : D - 1);
+    // eight steps' values in flight, the first eight from before the staging
+    PT xn[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) xn[q] = vcol[min(s_lo + 2 * q + h, L - 1) * stride];
+    for (int s = tid; s < L; s += 256) fwt[s] = prep.fwt[b * L + s];
+    for (int i = tid; i < L * MAXM / 4; i += 256) {
+        const float4 v = reinterpret_cast<const float4*>(prep.kf + b * L * MAXM)[i];
+        float* dst = kf + (4 * i / MAXM) * QP + 4 * i % MAXM;
+        dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+    }
+    __syncthreads();
     const float fon = r32 < MAXM ? 1.0f : 0.0f;
     const int mf = min(r32, MAXM - 1);
     f32x16 acc = {};
-    for (int s = s_lo; s < s_hi; s += 8) {  // four steps' operands loaded together
-        float x[4], a[4], bf[4];
+    for (int s = s_lo; s < s_hi; s += 16) {
+        float x[8];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = to_f32(vcol[min(s + 2 * q + h, L - 1) * stride]);
+        for (int q = 0; q < 8; ++q) x[q] = to_f32(xn[q]);
+        if (s + 16 < s_hi) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int sl = s + 2 * q + h, slc = min(sl, L - 1);
-            a[q] = sl < s_hi ? fwt[slc] * (TANH ? fast_tanh(x[q]) : x[q]) : 0.0f;
-            bf[q] = kf[slc * QP + mf] * fon;
+            for (int q = 0; q < 8; ++q) xn[q] = vcol[min(s + 16 + 2 * q + h, L - 1) * stride];
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = mfma2(a[q], bf[q], acc);
+        for (int q = 0; q < 8; ++q) {
+            const int sl = s + 2 * q + h, slc = min(sl, L - 1);
+            const float a = sl < s_hi ? fwt[slc] * (TANH ? fast_tanh(x[q]) : x[q]) : 0.0f;
+            acc = mfma2(a, kf[slc * QP + mf] * fon, acc);
+        }
     }
     if (kh == 1) {
 #pragma unroll
@@ -255,12 +267,15 @@ __global__ __launch_bounds__(256) void assoc_delta_kernel(
         }
     }
     if (blockIdx.y == 0 && wave == 3) {
-        for (int m = 0; m < M; ++m) {
-            float sum = 0.0f;
-            for (int s = lane; s < L; s += kWave) sum = fmaf(fwt[s], kf[s * QP + m], sum);
-            sum = wave_sum_xor(sum);
-            if (lane == 0) next_normalizer[b * M + m] = FINAL ? fmaf(keep, normalizer[b * M + m], sum) : sum;
-        }
+        constexpr int kLanes = kWave / MAXM;  // neighbours that share a feature, each with every kLanes-th slot
+        const int m = lane / kLanes;
+        float sum = 0.0f;
+#pragma unroll 8
+        for (int s = lane % kLanes; s < L; s += kLanes) sum = fmaf(fwt[s], kf[s * QP + m], sum);
+#pragma unroll
+        for (int off = kLanes / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+        if (lane % kLanes == 0 && m < M)
+            next_normalizer[b * M + m] = FINAL ? fmaf(keep, normalizer[b * M + m], sum) : sum;
     }
 }
 
@@ -270,11 +285,18 @@ __global__ __launch_bounds__(256) void assoc_delta_kernel(
 // forms the influence of slot s on query t,
 //   e^{prior_t - c_s} (q_t . f_s) weight_s  (s < t, else 0),
 // on fp32 MFMA (32 x 32 blocks, K = features) into LDS, and the denominators
-// den_t = sum_s influence + e^{prior_t} (q_t . normalizer) by wave
-// reductions. Then per column tile each wave forms a 32 x 32 block of
+// den_t = sum_s influence + e^{prior_t} (q_t . normalizer) by four lanes a row. Then per column tile each wave forms a 32 x 32 block of
 // sum_s influence tanh(v_s[d]) + e^{prior_t} (q_t . basis_d) on MFMA (A from
 // LDS, B the value columns straight from memory, eight steps' loads in flight
 // ahead of their use), and writes read = den/(den + 2^-8) num/(den + 2^-8).
+//
+// Latency bounds it: about three workgroups share a CU and each is a chain of
+// staging, influence, denominators and K steps. Staging in 16-byte pieces, the
+// denominators of all rows at once (a wave reduction per row is a chain of six
+// exchanges, 16 rows in turn), the basis loaded ahead of the K steps in 16-byte pieces
+// (its rows lie M floats apart: one float at a time touches a line per lane) and
+// the queries with the most slots first: 48 -> 37 us for 64 windows of 128 x
+// 1024 in bf16, 46 -> 35 us for the refine reads.
 constexpr int kReadTiles = 4;
 constexpr int kReadRows = 64;
 inline size_t read_lds(int64_t L, int64_t M) {
@@ -284,10 +306,10 @@ inline size_t read_lds(int64_t L, int64_t M) {
 }
 
 template <int MAXM, typename PT, typename OutT, bool VEC4, bool TANH = true>
-__global__ __launch_bounds__(256) void assoc_window_read_kernel(
+__global__ __launch_bounds__(256, 3) void assoc_window_read_kernel(
     const PT* __restrict__ proj, int64_t stride, int64_t value_off, AssocPrep prep,
     const float* __restrict__ basis, const float* __restrict__ normalizer, OutT* __restrict__ out, int64_t ostride,
-    int L, int64_t D, int M) {
+    int L, int64_t D, int M, bool basis4) {
     extern __shared__ float sh[];
     constexpr int QP = MAXM + 1;
     const int Lq = (L + 31) & ~31;
@@ -302,7 +324,8 @@ __global__ __launch_bounds__(256) void assoc_window_read_kernel(
     const int64_t b = blockIdx.x;
     const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     const int h = lane >> 5, r32 = lane & 31;
-    const int t0 = static_cast<int>(blockIdx.z) * kReadRows;
+    // the last queries first: they have the most slots to read
+    const int t0 = static_cast<int>(gridDim.z - 1 - blockIdx.z) * kReadRows;
     const int rows = min(kReadRows, L - t0);
     const int s_cnt = t0 + rows;  // slots that can reach these queries (s < t <= t0 + rows - 1)
     // bf16 path: this lane's value columns, and the loads of its first eight
@@ -327,10 +350,23 @@ __global__ __launch_bounds__(256) void assoc_window_read_kernel(
             for (int u = 0; u < 8; ++u) bn[u] = load2(vrows + v_dq + min(2 * u + h, L - 1) * stride);
         }
     }
-    for (int i = tid; i < s_cnt * MAXM; i += 256) f_sh[(i % MAXM) * IP + i / MAXM] = prep.kf[b * L * MAXM + i];
-    for (int i = tid; i < kReadRows * MAXM; i += 256) {
-        const int r = i / MAXM;
-        q_sh[r * QP + i % MAXM] = r < rows ? prep.qf[(b * L + t0) * MAXM + i] : 0.0f;
+    // four neighbouring lanes per query form its denominator below
+    const int den_row = tid >> 2, den_part = tid & 3;
+    float nrm[MAXM / 4];
+#pragma unroll
+    for (int j = 0; j < MAXM / 4; ++j) nrm[j] = normalizer[b * M + min(4 * j + den_part, M - 1)];
+    for (int i = tid; i < s_cnt * MAXM / 4; i += 256) {
+        const float4 v = reinterpret_cast<const float4*>(prep.kf + b * L * MAXM)[i];
+        float* dst = f_sh + (4 * i % MAXM) * IP + 4 * i / MAXM;
+        dst[0] = v.x, dst[IP] = v.y, dst[2 * IP] = v.z, dst[3 * IP] = v.w;
+    }
+#pragma unroll
+    for (int i = tid; i < kReadRows * MAXM / 4; i += 256) {
+        const int r = 4 * i / MAXM;
+        const float4 v = reinterpret_cast<const float4*>(prep.qf + (b * L + t0) * MAXM)[r < rows ? i : 0];
+        float* dst = q_sh + r * QP + 4 * i % MAXM;
+        const bool on = r < rows;
+        dst[0] = on ? v.x : 0.0f, dst[1] = on ? v.y : 0.0f, dst[2] = on ? v.z : 0.0f, dst[3] = on ? v.w : 0.0f;
     }
     for (int s2 = tid; s2 < s_cnt; s2 += 256) {
         cum[s2] = prep.cum[b * L + s2];
@@ -356,14 +392,22 @@ __global__ __launch_bounds__(256) void assoc_window_read_kernel(
         }
     }
     __syncthreads();
-    for (int rr = 0; rr < kReadRows / 4; ++rr) {
-        const int r = wave * (kReadRows / 4) + rr;
-        float sum = 0.0f;
-        for (int s = lane; s < s_cnt; s += kWave) sum += infl[r * IP + s];
-        float nq = lane < M ? q_sh[r * QP + lane] * normalizer[b * M + lane] : 0.0f;
-        sum = wave_sum_xor(sum);
-        nq = wave_sum_xor(nq);
-        if (lane == 0) den[r] = sum + fast_exp(pr[r]) * nq;
+    {
+        // the blocks' slots past s_cnt hold zeros
+        const float* row = infl + den_row * IP + den_part * 8 * nsb;
+        float sum0 = 0.0f, sum1 = 0.0f;
+        for (int j = 0; j < 8 * nsb; j += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) sum0 += row[j + u], sum1 += row[j + u + 1];
+        }
+        float nq = 0.0f;
+#pragma unroll
+        for (int j = 0; j < MAXM / 4; ++j)  // q_sh is zero past M
+            nq += 4 * j + den_part < M ? q_sh[den_row * QP + 4 * j + den_part] * nrm[j] : 0.0f;
+        float sum = sum0 + sum1;
+        sum += __shfl_xor(sum, 1, kWave), nq += __shfl_xor(nq, 1, kWave);
+        sum += __shfl_xor(sum, 2, kWave), nq += __shfl_xor(nq, 2, kWave);
+        if (den_part == 0) den[den_row] = sum + fast_exp(pr[den_row]) * nq;
     }
     __syncthreads();
 
@@ -388,6 +432,26 @@ __global__ __launch_bounds__(256) void assoc_window_read_kernel(
         for (int m = 0; m < 2; ++m)
 #pragma unroll
             for (int c = 0; c < 2; ++c) acc[m][c] = f32x16{};
+        // the carried basis of this lane's columns: its half of the features
+        float bs[2][MAXM / 2];
+        const auto load_basis = [&] {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float* col = basis + (b * D + v_dq + c) * M;
+                if (basis4) {
+#pragma unroll
+                    for (int kk = 0; kk < MAXM / 2; kk += 4) {
+                        const float4 v = *reinterpret_cast<const float4*>(col + h * (MAXM / 2) + kk);
+                        bs[c][kk] = v.x, bs[c][kk + 1] = v.y, bs[c][kk + 2] = v.z, bs[c][kk + 3] = v.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int kk = 0; kk < MAXM / 2; ++kk) bs[c][kk] = col[min(h * (MAXM / 2) + kk, M - 1)];
+                }
+            }
+        };
+        // ahead of the products where that leaves three waves to a SIMD
+        if constexpr (MAXM <= 16) load_basis();
         for (int s = 0; s < kfull; s += 16) {
             float2 bc[8];
 #pragma unroll
@@ -410,17 +474,17 @@ __global__ __launch_bounds__(256) void assoc_window_read_kernel(
                 acc[1][1] = mfma2(a1, ty, acc[1][1]);
             }
         }
+        if constexpr (MAXM > 16) load_basis();
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
             const float ep = fast_exp(pr[m * 32 + r32]);
 #pragma unroll
             for (int kk = 0; kk < MAXM / 2; ++kk) {
-                const int mm = 2 * kk + h;
+                const int mm = h * (MAXM / 2) + kk;
                 const float on = mm < M ? 1.0f : 0.0f;
                 const float aq = ep * q_sh[(m * 32 + r32) * QP + mm];
 #pragma unroll
-                for (int c = 0; c < 2; ++c)
-                    acc[m][c] = mfma2(aq, basis[(b * D + min(v_dq + c, D - 1)) * M + min(mm, M - 1)] * on, acc[m][c]);
+                for (int c = 0; c < 2; ++c) acc[m][c] = mfma2(aq, bs[c][kk] * on, acc[m][c]);
             }
         }
         if (cok) {
@@ -550,9 +614,10 @@ int launch_window_read(const PT* proj, int64_t stride, int64_t value_off, const 
     // multiple of four elements (aligned 4-element loads and stores)
     const bool vec4 = D % 4 == 0 && stride % 4 == 0 && value_off % 4 == 0 && ostride % 4 == 0 &&
                       reinterpret_cast<uintptr_t>(proj) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    const bool basis4 = M == MAXM && reinterpret_cast<uintptr_t>(basis) % 16 == 0;
     auto launch = [&](auto kernel, auto* o) {
         hipLaunchKernelGGL(kernel, grid, dim3(256), read_lds(L, M), s, proj, stride, value_off, prep, basis,
-                           normalizer, o, ostride, L, D, M);
+                           normalizer, o, ostride, L, D, M, basis4);
     };
     if (out_dtype == KOEMI_BF16) {
         if (vec4) launch(assoc_window_read_kernel<MAXM, PT, bf16, true, TANH>, static_cast<bf16*>(out));

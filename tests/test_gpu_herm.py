@@ -305,6 +305,25 @@ def test_associative_reads_into_a_bf16_block_and_from_bf16_projections(device, l
         assert torch.equal(wide[..., 2 * d:], rw.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("length, m", [(65, 16), (130, 16), (96, 32), (33, 13)])
+def test_associative_reads_of_a_basis_at_any_alignment(device, length, m):
+    """Every feature count that fills its registers reads a 16-byte aligned
+    basis four features at a time, any other basis one by one: the same values
+    in the same order, so the same bits."""
+    b, d = 2, 68
+    g = torch.Generator(device=device).manual_seed(length + m)
+    proj = torch.randn((b, length, (3 * d + 2 * m + 2 + 3) // 4 * 4), generator=g, device=device)
+    surprise = torch.rand((b, length), generator=g, device=device)
+    valid = torch.rand((b, length), generator=g, device=device) < 0.8
+    basis = torch.randn((b, d, m), generator=g, device=device)
+    norm = torch.rand((b, m), generator=g, device=device)
+    moved = torch.empty(basis.numel() + 1, device=device)[1:].view(b, d, m).copy_(basis)
+    assert basis.data_ptr() % 16 == 0 and moved.data_ptr() % 16 != 0
+    want = herm.associative_scan_read(proj, surprise, valid, basis, norm, width=d, features=m)
+    got = herm.associative_scan_read(proj, surprise, valid, moved, norm, width=d, features=m)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
 @pytest.mark.parametrize("b, length", [(3, 130), (64, 1)])
 def test_shifted_surprise_equals_the_row_kernel_on_shifted_logits(device, b, length):
     """koemi_herm_surprise_shifted scores row t on the logits of row t - 1
