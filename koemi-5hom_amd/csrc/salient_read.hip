@@ -772,6 +772,11 @@ namespace {
 //     issued together.
 // Needs width % 4 == 0, 16-byte aligned rows and at most kWinMaxSlots
 // candidate slots per block; other shapes take the kernels above.
+// A block is a chain of latencies with two workgroups to a CU, so loads are what
+// is kept in flight: raw words of both row kinds through one address form, the
+// next slot tile's keys and the next chunk's queries under the products, all
+// eight queries of a wave in one softmax. 64 windows of 128 x 1024 (bf16 rows in
+// place): the local read 55 -> 40 us, the salient read 51 -> 47 us.
 constexpr int kWinQ = 32;
 constexpr int kWinMaxSlots = 152;   // salient blocks: LDS 4 x 32 x 153 fp32 partial scores (78 KiB)
 constexpr int kWinLocalSlots = 64;  // local blocks: 4 x 32 x 65 (33 KiB)
@@ -796,26 +801,15 @@ __device__ __forceinline__ void split3(const float (&x)[8], bf16x8& hi, bf16x8& 
     }
 }
 
-// eight values from column col (a multiple of 8) of a row, zeros past D (a
-// multiple of 8)
-__device__ __forceinline__ void load8(const float* row, int64_t col, int64_t D, float (&x)[8]) {
-    if (col < D) {
-        const float4 a = *reinterpret_cast<const float4*>(row + col);
-        const float4 b = *reinterpret_cast<const float4*>(row + col + 4);
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-    } else {
+// eight values of a row from its raw words: fp32 (a, b), or bf16 (a); zeros where
+// the columns lie past the width
+__device__ __forceinline__ void widen8(uint4 a, uint4 b, bool fp32, bool within, float (&x)[8]) {
+    const uint32_t wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = 0.0f;
-    }
-}
-__device__ __forceinline__ void load8(const bf16* row, int64_t col, int64_t D, float (&x)[8]) {
-    if (col < D) {
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + col);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = static_cast<float>(v[i]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = 0.0f;
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t low = i % 2 == 0 ? wa[i / 2] << 16 : wa[i / 2] & 0xffff0000u;
+        const uint32_t w = fp32 ? (i < 4 ? wa[i] : wb[i - 4]) : low;
+        x[i] = __uint_as_float(within ? w : 0u);
     }
 }
 
@@ -828,13 +822,13 @@ __device__ inline f32x16 mfma_f32_32x32x2(float a, float b, f32x16 c) {
 // and values are rows `kstride` elements apart of type KT (fp32, or the bf16
 // columns of the block's projection read in place, widened exactly).
 template <bool LOCAL, int MAXS, typename OutT, typename KT>
-__global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
+__global__ __launch_bounds__(256, 2) void window_read_kernel(
     const float* __restrict__ ck, const float* __restrict__ cv, const uint8_t* __restrict__ cvalid,
     const KT* __restrict__ k, const KT* __restrict__ v, int64_t kstride, const uint8_t* __restrict__ flags,
     const float* __restrict__ q, OutT* __restrict__ out, int64_t ostride, int S, int L, int64_t D, int window,
     float scale) {
     constexpr int NST = (MAXS + 31) / 32;  // slot tiles
-    constexpr int NJ = (MAXS + kWave - 1) / kWave;
+    constexpr int NJ = (MAXS + 7) / 8;  // listed slots of a query to one of its eight lanes
     __shared__ int list[MAXS];
     __shared__ int wave_cnt[4], wave_carried[4];
     __shared__ float sc[4][kWinQ][MAXS + 1];
@@ -875,12 +869,20 @@ __global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
     }
     const int nst = (n + 31) / 32;
     // Rows of listed slots: carried rows (fp32, D apart) or window rows (KT,
-    // kstride apart). Loads of a group of listed slots [i_lo, i_hi] take one
-    // path when the group is all carried or all window (uniform: nc splits
-    // the list), a per-lane choice only in the group that straddles nc.
-    auto carried_row = [&](const float* base_rows, int s) { return base_rows + (row * S + s) * D; };
-    auto window_row = [&](const KT* base_rows, int s) { return base_rows + (row * L + (s - S)) * kstride; };
-    auto group_kind = [&](int i_lo, int i_hi) { return i_lo >= nc ? 1 : (min(i_hi, n - 1) < nc ? 0 : 2); };
+    // kstride apart). A lane keeps its row's address and element size, and loads
+    // raw words that are widened where they are used: one address form for either
+    // kind, so every load of a step is issued together whatever the group holds (a
+    // branch per row widens inside it and waits for each load in turn).
+    auto group_kind = [&](int i_lo, int i_hi) {  // 0 all carried, 1 all window, 2 both (uniform: nc splits the list)
+        if constexpr (std::is_same<KT, float>::value) return 0;  // fp32 rows of either kind
+        else return i_lo >= nc ? 1 : (min(i_hi, n - 1) < nc ? 0 : 2);
+    };
+    auto is_fp32 = [&](int i) { return std::is_same<KT, float>::value || min(i, n - 1) < nc; };
+    auto row_of = [&](const float* carried_rows, const KT* window_rows, int i) {
+        const int sl = list[min(i, n - 1)];
+        return sl < S ? reinterpret_cast<const char*>(carried_rows + (row * S + sl) * D)
+                      : reinterpret_cast<const char*>(window_rows + (row * L + (sl - S)) * kstride);
+    };
     // scores
     {
         const float* qrow = q + (row * L + t0 + min(r, nq - 1)) * D;
@@ -894,80 +896,89 @@ __global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
         // slots). The local read runs on bf16 MFMA with the queries split in
         // three (split3: exact products), three products per k step for bf16
         // window rows (keys read in place), six for fp32 rows; the salient read
-        // (mostly carried slots) on fp32 MFMA, one product per column.
+        // (mostly carried slots) on fp32 MFMA, one product per column. The keys of
+        // the next slot tile and the queries of the next chunk are in flight under
+        // the products. What lies past D is read at column 0 and cleared.
         const int64_t chunks = (D + 63) / 64;
+        uint4 qn[4][2], kn[4][2];
+        auto column = [&](int64_t ch, int j) { return 64 * ch + 16 * j + 8 * h; };
+        auto fetch_queries = [&](int64_t ch) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t col = column(ch, j);
+                const uint4* p = reinterpret_cast<const uint4*>(qrow + (col < D ? col : 0));
+                qn[j][0] = p[0], qn[j][1] = p[1];
+            }
+        };
+        auto fetch_keys = [&](int64_t ch, int st) {
+            const char* p = row_of(ck, k, st * 32 + r);
+            const bool four = is_fp32(st * 32 + r), words = group_kind(st * 32, st * 32 + 31) != 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t col = column(ch, j);
+                const char* e = p + (col < D ? col : 0) * (four ? 4 : 2);
+                kn[j][0] = *reinterpret_cast<const uint4*>(e);
+                if (words) kn[j][1] = *reinterpret_cast<const uint4*>(e + (four ? 16 : 0));
+            }
+        };
+        if (wave < chunks) {
+            if constexpr (LOCAL) fetch_queries(wave);
+            fetch_keys(wave, 0);
+        }
         for (int64_t ch = wave; ch < chunks; ch += 4) {
-            if constexpr (LOCAL) {
-                // the queries as three bf16 parts (their sum is the query exactly)
-                bf16x8 qh[4], qm[4], ql[4];
+            bf16x8 qh[4], qm[4], ql[4];  // local: the queries as three bf16 parts (their sum is the query exactly)
+            float qx[4][8];              // salient (its five slot tiles a chunk leave no registers to fetch ahead)
+            if constexpr (!LOCAL) fetch_queries(ch);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float x[8];
-                    load8(qrow, 64 * ch + 16 * j + 8 * h, D, x);
-                    split3(x, qh[j], qm[j], ql[j]);
-                }
+            for (int j = 0; j < 4; ++j) {
+                widen8(qn[j][0], qn[j][1], true, column(ch, j) < D, qx[j]);
+                if constexpr (LOCAL) split3(qx[j], qh[j], qm[j], ql[j]);
+            }
+            if (LOCAL && ch + 4 < chunks) fetch_queries(ch + 4);
 #pragma unroll
-                for (int st = 0; st < NST; ++st) {
-                    if (st >= nst) break;
-                    const int ks = list[min(st * 32 + r, n - 1)];
-                    bool window_only = false;
-                    if constexpr (!std::is_same<KT, float>::value) window_only = group_kind(st * 32, st * 32 + 31) == 1;
-                    if (window_only) {
+            for (int st = 0; st < NST; ++st) {
+                if (st >= nst) break;
+                uint4 kc[4][2];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) kc[j][0] = kn[j][0], kc[j][1] = kn[j][1];
+                if (st + 1 < nst) fetch_keys(ch, st + 1);
+                else if (ch + 4 < chunks) fetch_keys(ch + 4, 0);
+                if constexpr (LOCAL) {
+                    if (group_kind(st * 32, st * 32 + 31) == 1) {
                         // bf16 keys: three products per k step
-                        const KT* krow = window_row(k, ks);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
-                            const int64_t col = 64 * ch + 16 * j + 8 * h;
-                            bf16x8 kb = {};
-                            if (col < D) kb = *reinterpret_cast<const bf16x8*>(krow + col);
+                            bf16x8 kb = __builtin_bit_cast(bf16x8, kc[j][0]);
+                            if (column(ch, j) >= D) kb = bf16x8{};
                             acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], kb, acc[st], 0, 0, 0);
                             acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qm[j], kb, acc[st], 0, 0, 0);
                             acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ql[j], kb, acc[st], 0, 0, 0);
                         }
-                    } else {
+                        continue;
+                    }
+                }
+                const bool four = is_fp32(st * 32 + r);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    float kx[8];
+                    widen8(kc[j][0], kc[j][1], four, column(ch, j) < D, kx);
+                    if constexpr (LOCAL) {
                         // fp32 keys (carried slots) split as well: six products
                         // per k step (the three dropped are below 2^-24 of the
                         // product; for bf16 keys the last three add exact zeros)
-                        float kx[4][8];
+                        bf16x8 kh, km, kl;
+                        split3(kx, kh, km, kl);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], kh, acc[st], 0, 0, 0);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qm[j], kh, acc[st], 0, 0, 0);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ql[j], kh, acc[st], 0, 0, 0);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], km, acc[st], 0, 0, 0);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qm[j], km, acc[st], 0, 0, 0);
+                        acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], kl, acc[st], 0, 0, 0);
+                    } else {
+                        // the salient read (mostly carried slots): fp32 MFMA, one product per column
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int64_t col = 64 * ch + 16 * j + 8 * h;
-                            if (ks < S) load8(carried_row(ck, ks), col, D, kx[j]);
-                            else load8(window_row(k, ks), col, D, kx[j]);
-                        }
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            bf16x8 kh, km, kl;
-                            split3(kx[j], kh, km, kl);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], kh, acc[st], 0, 0, 0);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qm[j], kh, acc[st], 0, 0, 0);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ql[j], kh, acc[st], 0, 0, 0);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], km, acc[st], 0, 0, 0);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qm[j], km, acc[st], 0, 0, 0);
-                            acc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qh[j], kl, acc[st], 0, 0, 0);
-                        }
+                        for (int m = 0; m < 8; ++m) acc[st] = mfma_f32_32x32x2(qx[j][m], kx[m], acc[st]);
                     }
-                }
-            } else {
-                // the salient read (mostly carried slots): fp32 MFMA, one product per column
-                float qx[4][8];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) load8(qrow, 64 * ch + 16 * j + 8 * h, D, qx[j]);
-#pragma unroll
-                for (int st = 0; st < NST; ++st) {
-                    if (st >= nst) break;
-                    const int ks = list[min(st * 32 + r, n - 1)];
-                    float kx[4][8];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int64_t col = 64 * ch + 16 * j + 8 * h;
-                        if (ks < S) load8(carried_row(ck, ks), col, D, kx[j]);
-                        else load8(window_row(k, ks), col, D, kx[j]);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-#pragma unroll
-                        for (int m = 0; m < 8; ++m) acc[st] = mfma_f32_32x32x2(qx[j][m], kx[j][m], acc[st]);
                 }
             }
         }
@@ -983,43 +994,46 @@ __global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
     }
     __syncthreads();
 
-    // softmax: wave w takes queries 8 w .. 8 w + 7; weights overwrite sc[0]
-    for (int qq = 0; qq < 8; ++qq) {
-        const int m = wave * 8 + qq;
+    // softmax: wave w takes queries 8 w .. 8 w + 7, eight lanes to a query (all
+    // queries at once: one by one, each wave reduction waits for the one before);
+    // weights overwrite sc[0]
+    {
+        const int m = wave * 8 + (lane >> 3);
         const int t = t0 + m;
+        const int per = (n + 7) / 8, first = (lane & 7) * per;
         float x[NJ];
-        bool ok[NJ];
+        uint32_t ok = 0;
         float mx = -INFINITY;
-        bool any = false;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int idx = j * kWave + lane;
-            x[j] = 0.0f;
-            ok[j] = false;
-            if (idx < n) {
-                const int sl = list[idx];
-                x[j] = (((sc[0][m][idx] + sc[1][m][idx]) + sc[2][m][idx]) + sc[3][m][idx]) * scale;
-                ok[j] = m < nq && sl < S + t && (!LOCAL || sl >= S + t - window);
-            }
-            if (ok[j]) {
-                any = true;
-                mx = fmaxf(mx, x[j]);
-            }
+            if (j >= per) break;
+            const int idx = min(first + j, n - 1);
+            const int sl = list[idx];
+            x[j] = (((sc[0][m][idx] + sc[1][m][idx]) + sc[2][m][idx]) + sc[3][m][idx]) * scale;
+            const bool use = first + j < n && m < nq && sl < S + t && (!LOCAL || sl >= S + t - window);
+            ok |= static_cast<uint32_t>(use) << j;
+            if (use) mx = fmaxf(mx, x[j]);
         }
-        mx = wave_max_xor(mx);
-        any = __any(any);
-        if (!any) mx = 0.0f;
+        uint32_t any = ok;
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+            any |= __shfl_xor(any, off, kWave);
+        }
+        if (any == 0) mx = 0.0f;
         float sum = 0.0f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            x[j] = ok[j] ? expf(x[j] - mx) : 0.0f;
+            if (j >= per) break;
+            x[j] = (ok >> j & 1u) != 0 ? expf(x[j] - mx) : 0.0f;
             sum += x[j];
         }
-        sum = wave_sum_xor(sum);
+#pragma unroll
+        for (int off = 1; off < 8; off <<= 1) sum += __shfl_xor(sum, off, kWave);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            const int idx = j * kWave + lane;
-            if (idx < n) sc[0][m][idx] = sum > 0.0f ? x[j] / sum : x[j];
+            if (j >= per) break;
+            if (first + j < n) sc[0][m][first + j] = sum > 0.0f ? x[j] / sum : x[j];
         }
     }
     __syncthreads();
@@ -1041,59 +1055,76 @@ __global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
         for (int cc = 0; cc < 4; ++cc)
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[cc][e] = 0.0f;
-        float4 bn[8];
+        uint4 bn[8];
         auto fetch = [&](int i0) {
-            auto fetch_with = [&](auto load_slot) {
+            const int kind = group_kind(i0, i0 + 15);
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int li = i0 + 8 * h + u;
-                    bn[u] = li < n ? load_slot(list[li]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int u = 0; u < 8; ++u) {
+                const int i = i0 + 8 * h + u;
+                const bool four = is_fp32(i);
+                const char* e = row_of(cv, v, i) + colc * (four ? 4 : 2);
+                if (kind == 0) {
+                    bn[u] = *reinterpret_cast<const uint4*>(e);
+                } else {
+                    const uint2 a = *reinterpret_cast<const uint2*>(e);
+                    bn[u].x = a.x, bn[u].y = a.y;
+                    if (kind == 2) {
+                        const uint2 b = *reinterpret_cast<const uint2*>(e + (four ? 8 : 0));
+                        bn[u].z = b.x, bn[u].w = b.y;
+                    }
                 }
-            };
-            if constexpr (std::is_same<KT, float>::value) {
-                fetch_with([&](int sl) { return load4((sl < S ? carried_row(cv, sl) : window_row(v, sl)) + colc); });
-            } else {
-                const int kind = group_kind(i0, i0 + 15);
-                if (kind == 0) fetch_with([&](int sl) { return load4(carried_row(cv, sl) + colc); });
-                else if (kind == 1) fetch_with([&](int sl) { return load4(window_row(v, sl) + colc); });
-                else
-                    fetch_with([&](int sl) {
-                        return sl < S ? load4(carried_row(cv, sl) + colc) : load4(window_row(v, sl) + colc);
-                    });
             }
         };
         fetch(0);
         // groups of 16 listed slots up to the last listed one (past it the
-        // weights are zero: those groups would add exact zeros)
+        // weights and the values are zero)
         for (int i0 = 0; i0 < n; i0 += 16) {
-            float4 bc[8];
+            uint4 bc[8];
             float wv[8];
+            const int kind = group_kind(i0, i0 + 15);
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 bc[u] = bn[u];
                 const int li = i0 + 8 * h + u;
-                wv[u] = li < n ? sc[0][r][li] : 0.0f;
+                const float w = sc[0][r][min(li, n - 1)];
+                wv[u] = li < n ? w : 0.0f;
+            }
+            if (i0 + 16 > n) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + 8 * h + u >= n) bc[u] = make_uint4(0, 0, 0, 0);
             }
             if (i0 + 16 < n) fetch(i0 + 16);
+            auto value = [&](int u, int cc) {  // column cc of row u: fp32, or bf16 widened
+                const uint4 w = bc[u];
+                const uint32_t word = cc == 0 ? w.x : cc == 1 ? w.y : cc == 2 ? w.z : w.w;
+                const uint32_t pair = cc < 2 ? w.x : w.y;
+                const bool four = kind == 0 || (kind == 2 && is_fp32(i0 + 8 * h + u));
+                return __uint_as_float(four ? word : cc % 2 == 0 ? pair << 16 : pair & 0xffff0000u);
+            };
             if constexpr (LOCAL) {
-                bool bf16_rows = false;
-                if constexpr (!std::is_same<KT, float>::value) bf16_rows = group_kind(i0, i0 + 15) == 1;
                 bf16x8 wh, wm, wl;
                 split3(wv, wh, wm, wl);
 #pragma unroll
                 for (int cc = 0; cc < 4; ++cc) {
-                    float vv[8];
+                    if (kind == 1) {
+                        uint4 packed;  // column cc of the eight rows: one half of a word each
+                        uint32_t* pw = reinterpret_cast<uint32_t*>(&packed);
+                        constexpr uint32_t kLow = 0x05040100u, kHigh = 0x07060302u;
 #pragma unroll
-                    for (int u = 0; u < 8; ++u)
-                        vv[u] = cc == 0 ? bc[u].x : cc == 1 ? bc[u].y : cc == 2 ? bc[u].z : bc[u].w;
-                    if (bf16_rows) {
-                        bf16x8 vb;  // exact: the rows hold bf16 values
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) vb[u] = static_cast<__bf16>(vv[u]);
+                        for (int u = 0; u < 4; ++u) {
+                            const uint32_t w0 = cc < 2 ? bc[2 * u].x : bc[2 * u].y;
+                            const uint32_t w1 = cc < 2 ? bc[2 * u + 1].x : bc[2 * u + 1].y;
+                            pw[u] = __builtin_amdgcn_perm(w1, w0, cc % 2 == 0 ? kLow : kHigh);
+                        }
+                        const bf16x8 vb = __builtin_bit_cast(bf16x8, packed);
                         o[cc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wh, vb, o[cc], 0, 0, 0);
                         o[cc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wm, vb, o[cc], 0, 0, 0);
                         o[cc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wl, vb, o[cc], 0, 0, 0);
                     } else {
+                        float vv[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) vv[u] = value(u, cc);
                         bf16x8 vh, vm, vl;
                         split3(vv, vh, vm, vl);
                         o[cc] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wh, vh, o[cc], 0, 0, 0);
@@ -1107,12 +1138,9 @@ __global__ __launch_bounds__(256, LOCAL ? 2 : 1) void window_read_kernel(
             } else {
                 // fp32 rows: one fp32 MFMA step per slot pair (slot 8 h + u of lane h)
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    o[0] = mfma_f32_32x32x2(wv[u], bc[u].x, o[0]);
-                    o[1] = mfma_f32_32x32x2(wv[u], bc[u].y, o[1]);
-                    o[2] = mfma_f32_32x32x2(wv[u], bc[u].z, o[2]);
-                    o[3] = mfma_f32_32x32x2(wv[u], bc[u].w, o[3]);
-                }
+                for (int u = 0; u < 8; ++u)
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc) o[cc] = mfma_f32_32x32x2(wv[u], value(u, cc), o[cc]);
             }
         }
         if (cok) {

@@ -171,6 +171,44 @@ def test_reads_of_bf16_projection_columns_equal_the_widened_reads(device, window
     assert torch.equal(got2, got)
 
 
+@pytest.mark.parametrize("b, s, length, d, window, p", [
+    (2, 16, 40, 72, 16, 0.9),    # a slot tile and a value group that hold carried and window rows
+    (2, 16, 128, 200, 16, 1.0),  # carried rows end at a group's edge; window rows alone in later blocks
+    (3, 7, 33, 520, 0, 0.3),     # a second block of one query, a chunk of eight columns
+    (2, 24, 65, 136, 0, 1.0),    # every slot listed
+    (1, 16, 32, 8, 33, 0.1),     # few slots: lanes of the softmax without one
+    (2, 0, 31, 64, 16, 0.7),     # no ring: window rows alone
+])
+def test_fused_reads_of_bf16_rows_match_the_oracle(device, b, s, length, d, window, p):
+    """The one-launch read with the window's rows as bf16 columns read in
+    place, over the row kinds that a slot tile or a value group can hold."""
+    ck, cv, cvalid, k, v, flags, q = _read_case(5 * length + d, b, s, length, d, p, torch.float32)
+    projected = torch.cat([k, v, torch.zeros((b, length, 8))], dim=-1).to(torch.bfloat16).to(device)
+    case = (ck, cv, cvalid, projected[..., :d].float().cpu(), projected[..., d:2 * d].float().cpu(), flags, q)
+    out = torch.zeros((b, length, d), device=device)
+    on = lambda *ts: (x.to(device) for x in ts)
+    read = memory.read_local_window if window else memory.read_salient_window
+    read(*on(ck, cv, cvalid), projected[..., :d], projected[..., d:2 * d], *on(flags, q), out=out,
+         **({"window": window} if window else {}))
+    arrays = [x.numpy() for x in case]
+    want = oracle.read_local_window(*arrays, window) if window else oracle.read_salient_window(*arrays)
+    err = np.abs(out.cpu().numpy() - want)
+    vmax = max(float(cv.abs().max()) if s else 0.0, float(v.abs().max()))
+    print(f"bf16 rows s={s} L={length} d={d} window={window}: max_abs={err.max():.3e}", flush=True)
+    assert np.all(err <= 1e-4 * np.abs(want) + 1e-5 * vmax)
+
+
+def test_an_infinite_value_of_the_last_listed_slot_stays_infinite(device):
+    """Slots past the last listed one add nothing: one admitted entry with an
+    infinite value gives infinity to the queries that read it, not NaN."""
+    ck, cv, cvalid, k, v, adm, q = _read_case(9, 1, 0, 32, 16, 0.0, torch.float32)
+    adm[0, 3] = True
+    v[0, 3, 5] = float("inf")
+    got = memory.read_salient_window(*(x.to(device) for x in (ck, cv, cvalid, k, v, adm, q)))
+    assert torch.all(got[0, 4:, 5] == float("inf"))
+    assert torch.equal(got[0, 4:, 6].cpu(), v[0, 3, 6].expand(28))
+
+
 def test_read_salient_window_rejects_bad_inputs(device):
     ck, cv, cvalid, k, v, adm, q = (x.to(device) for x in _read_case(1, 2, 3, 5, 4, 0.5, torch.float32))
     with pytest.raises(think.CudaThinkValidationError, match="share a dtype"):
