@@ -267,11 +267,26 @@ __global__ __launch_bounds__(256) void assoc_delta_kernel(
         }
     }
     if (blockIdx.y == 0 && wave == 3) {
-        constexpr int kLanes = kWave / MAXM;  // neighbours that share a feature, each with every kLanes-th slot
+        // a feature to each group of kLanes neighbours, every one with the chains of MAXM
+        // residues of the slot: the sums are a wave reduction's, pair for pair (slots
+        // l, l + 64, .. in turn, then residues 32, 16, .. 1 apart)
+        constexpr int kLanes = kWave / MAXM;
         const int m = lane / kLanes;
-        float sum = 0.0f;
-#pragma unroll 8
-        for (int s = lane % kLanes; s < L; s += kLanes) sum = fmaf(fwt[s], kf[s * QP + m], sum);
+        float v[MAXM];
+#pragma unroll
+        for (int i = 0; i < MAXM; ++i) v[i] = 0.0f;
+        for (int s0 = lane % kLanes; s0 < L; s0 += kWave)
+#pragma unroll
+            for (int i = 0; i < MAXM; ++i) {
+                const int s = min(s0 + kLanes * i, L - 1);
+                const float next = fmaf(fwt[s], kf[s * QP + m], v[i]);
+                v[i] = s0 + kLanes * i < L ? next : v[i];
+            }
+#pragma unroll
+        for (int n = MAXM / 2; n > 0; n >>= 1)
+#pragma unroll
+            for (int i = 0; i < n; ++i) v[i] += v[i + n];
+        float sum = v[0];
 #pragma unroll
         for (int off = kLanes / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
         if (lane % kLanes == 0 && m < M)
@@ -295,8 +310,8 @@ __global__ __launch_bounds__(256) void assoc_delta_kernel(
 // denominators of all rows at once (a wave reduction per row is a chain of six
 // exchanges, 16 rows in turn), the basis loaded ahead of the K steps in 16-byte pieces
 // (its rows lie M floats apart: one float at a time touches a line per lane) and
-// the queries with the most slots first: 48 -> 37 us for 64 windows of 128 x
-// 1024 in bf16, 46 -> 35 us for the refine reads.
+// the queries with the most slots first: 47 -> 36 us for 64 windows of 128 x
+// 1024 in bf16, 44 -> 33 us for the refine reads.
 constexpr int kReadTiles = 4;
 constexpr int kReadRows = 64;
 inline size_t read_lds(int64_t L, int64_t M) {
@@ -393,20 +408,38 @@ __global__ __launch_bounds__(256, 3) void assoc_window_read_kernel(
     }
     __syncthreads();
     {
-        // the blocks' slots past s_cnt hold zeros
-        const float* row = infl + den_row * IP + den_part * 8 * nsb;
-        float sum0 = 0.0f, sum1 = 0.0f;
-        for (int j = 0; j < 8 * nsb; j += 8) {
+        // the sums are a wave reduction's over slots (features), pair for pair: a part
+        // holds the residues den_part + 4 i, the blocks' slots past s_cnt hold zeros
+        const float* row = infl + den_row * IP + den_part;
+        float v[16], nv[MAXM / 4];
+        float sum, nq;
+        {
+#pragma clang fp contract(off)
 #pragma unroll
-            for (int u = 0; u < 8; u += 2) sum0 += row[j + u], sum1 += row[j + u + 1];
+            for (int i = 0; i < 16; ++i) v[i] = 0.0f;
+            for (int j = 0; j < nsb; j += 2) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] += row[32 * j + 4 * i];
+                if (j + 1 < nsb) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[8 + i] += row[32 * j + 32 + 4 * i];
+                }
+            }
+#pragma unroll
+            for (int n = 8; n > 0; n >>= 1)
+#pragma unroll
+                for (int i = 0; i < n; ++i) v[i] += v[i + n];
+#pragma unroll
+            for (int j = 0; j < MAXM / 4; ++j)  // q_sh is zero past M
+                nv[j] = 4 * j + den_part < M ? q_sh[den_row * QP + 4 * j + den_part] * nrm[j] : 0.0f;
+#pragma unroll
+            for (int n = MAXM / 8; n > 0; n >>= 1)
+#pragma unroll
+                for (int j = 0; j < n; ++j) nv[j] += nv[j + n];
+            sum = v[0], nq = nv[0];
+            sum += __shfl_xor(sum, 2, kWave), nq += __shfl_xor(nq, 2, kWave);
+            sum += __shfl_xor(sum, 1, kWave), nq += __shfl_xor(nq, 1, kWave);
         }
-        float nq = 0.0f;
-#pragma unroll
-        for (int j = 0; j < MAXM / 4; ++j)  // q_sh is zero past M
-            nq += 4 * j + den_part < M ? q_sh[den_row * QP + 4 * j + den_part] * nrm[j] : 0.0f;
-        float sum = sum0 + sum1;
-        sum += __shfl_xor(sum, 1, kWave), nq += __shfl_xor(nq, 1, kWave);
-        sum += __shfl_xor(sum, 2, kWave), nq += __shfl_xor(nq, 2, kWave);
         if (den_part == 0) den[den_row] = sum + fast_exp(pr[den_row]) * nq;
     }
     __syncthreads();
@@ -432,7 +465,9 @@ __global__ __launch_bounds__(256, 3) void assoc_window_read_kernel(
         for (int m = 0; m < 2; ++m)
 #pragma unroll
             for (int c = 0; c < 2; ++c) acc[m][c] = f32x16{};
-        // the carried basis of this lane's columns: its half of the features
+        // the carried basis of this lane's columns: feature 2 kk + h for step kk. An
+        // aligned basis is loaded half by half (features h MAXM / 2 on, 16 bytes at a
+        // time) and its pairs exchanged between the halves of the wave.
         float bs[2][MAXM / 2];
         const auto load_basis = [&] {
 #pragma unroll
@@ -442,11 +477,16 @@ __global__ __launch_bounds__(256, 3) void assoc_window_read_kernel(
 #pragma unroll
                     for (int kk = 0; kk < MAXM / 2; kk += 4) {
                         const float4 v = *reinterpret_cast<const float4*>(col + h * (MAXM / 2) + kk);
-                        bs[c][kk] = v.x, bs[c][kk + 1] = v.y, bs[c][kk + 2] = v.z, bs[c][kk + 3] = v.w;
+                        const auto lo = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.y),
+                                                                         false, false);
+                        const auto hi = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.z), __float_as_uint(v.w),
+                                                                         false, false);
+                        bs[c][kk / 2] = __uint_as_float(lo[0]), bs[c][MAXM / 4 + kk / 2] = __uint_as_float(lo[1]);
+                        bs[c][kk / 2 + 1] = __uint_as_float(hi[0]), bs[c][MAXM / 4 + kk / 2 + 1] = __uint_as_float(hi[1]);
                     }
                 } else {
 #pragma unroll
-                    for (int kk = 0; kk < MAXM / 2; ++kk) bs[c][kk] = col[min(h * (MAXM / 2) + kk, M - 1)];
+                    for (int kk = 0; kk < MAXM / 2; ++kk) bs[c][kk] = col[min(2 * kk + h, M - 1)];
                 }
             }
         };
@@ -480,7 +520,7 @@ __global__ __launch_bounds__(256, 3) void assoc_window_read_kernel(
             const float ep = fast_exp(pr[m * 32 + r32]);
 #pragma unroll
             for (int kk = 0; kk < MAXM / 2; ++kk) {
-                const int mm = h * (MAXM / 2) + kk;
+                const int mm = 2 * kk + h;
                 const float on = mm < M ? 1.0f : 0.0f;
                 const float aq = ep * q_sh[(m * 32 + r32) * QP + mm];
 #pragma unroll

@@ -776,7 +776,7 @@ namespace {
 // is kept in flight: raw words of both row kinds through one address form, the
 // next slot tile's keys and the next chunk's queries under the products, all
 // eight queries of a wave in one softmax. 64 windows of 128 x 1024 (bf16 rows in
-// place): the local read 55 -> 40 us, the salient read 51 -> 47 us.
+// place): the local read 56 -> 40 us, the salient read 50 -> 46 us.
 constexpr int kWinQ = 32;
 constexpr int kWinMaxSlots = 152;   // salient blocks: LDS 4 x 32 x 153 fp32 partial scores (78 KiB)
 constexpr int kWinLocalSlots = 64;  // local blocks: 4 x 32 x 65 (33 KiB)
@@ -1000,17 +1000,20 @@ __global__ __launch_bounds__(256, 2) void window_read_kernel(
     {
         const int m = wave * 8 + (lane >> 3);
         const int t = t0 + m;
-        const int per = (n + 7) / 8, first = (lane & 7) * per;
+        // lane p of a query takes the listed slots p, p + 8, ..: its sums are a wave
+        // reduction's, pair for pair (slots 64 apart in turn, then 32, 16, .. 1 apart)
+        const int part = lane & 7;
         float x[NJ];
         uint32_t ok = 0;
         float mx = -INFINITY;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if (j >= per) break;
-            const int idx = min(first + j, n - 1);
+            x[j] = 0.0f;
+            if (8 * j >= n) continue;
+            const int idx = min(8 * j + part, n - 1);
             const int sl = list[idx];
             x[j] = (((sc[0][m][idx] + sc[1][m][idx]) + sc[2][m][idx]) + sc[3][m][idx]) * scale;
-            const bool use = first + j < n && m < nq && sl < S + t && (!LOCAL || sl >= S + t - window);
+            const bool use = 8 * j + part < n && m < nq && sl < S + t && (!LOCAL || sl >= S + t - window);
             ok |= static_cast<uint32_t>(use) << j;
             if (use) mx = fmaxf(mx, x[j]);
         }
@@ -1021,20 +1024,23 @@ __global__ __launch_bounds__(256, 2) void window_read_kernel(
             any |= __shfl_xor(any, off, kWave);
         }
         if (any == 0) mx = 0.0f;
-        float sum = 0.0f;
+        float sums[8] = {};
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if (j >= per) break;
+            if (8 * j >= n) continue;
             x[j] = (ok >> j & 1u) != 0 ? expf(x[j] - mx) : 0.0f;
-            sum += x[j];
+            sums[j % 8] += x[j];
         }
 #pragma unroll
-        for (int off = 1; off < 8; off <<= 1) sum += __shfl_xor(sum, off, kWave);
+        for (int h2 = 4; h2 > 0; h2 >>= 1)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            if (j >= per) break;
-            if (first + j < n) sc[0][m][first + j] = sum > 0.0f ? x[j] / sum : x[j];
-        }
+            for (int i = 0; i < h2; ++i) sums[i] += sums[i + h2];
+        float sum = sums[0];
+#pragma unroll
+        for (int off = 4; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            if (8 * j + part < n) sc[0][m][8 * j + part] = sum > 0.0f ? x[j] / sum : x[j];
     }
     __syncthreads();
 

@@ -14,12 +14,13 @@ admission off, within 5e-2 relative (bf16 rounding of every projection input).
 from __future__ import annotations
 
 import dataclasses
+from pathlib import Path
 
 import numpy as np
 import pytest
 import torch
 
-from koemi_amd import _native, herm, moe, think
+from koemi_amd import _native, herm, memory, moe, think
 from oracle import herm as oherm
 
 pytestmark = pytest.mark.gpu
@@ -322,6 +323,47 @@ def test_associative_reads_of_a_basis_at_any_alignment(device, length, m):
     want = herm.associative_scan_read(proj, surprise, valid, basis, norm, width=d, features=m)
     got = herm.associative_scan_read(proj, surprise, valid, moved, norm, width=d, features=m)
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def read_bits(device):
+    """Reads and next states of small windows (name -> array), inputs made on the host."""
+    out = {}
+    for length, m, low in ((70, 16, False), (33, 16, True), (100, 32, False)):
+        b, d = 1, 8
+        g = torch.Generator().manual_seed(length * 100 + m)
+        proj = torch.randn((b, length, (3 * d + 2 * m + 2 + 3) // 4 * 4), generator=g)
+        case = (torch.rand((b, length), generator=g), torch.rand((b, length), generator=g) < 0.8,
+                torch.randn((b, d, m), generator=g), torch.rand((b, m), generator=g))
+        proj = proj.to(torch.bfloat16 if low else torch.float32).to(device)
+        got = herm.associative_scan_read(proj, *(t.to(device) for t in case), width=d, features=m)
+        for name, value in zip(("read", "basis", "normalizer"), got):
+            out[f"assoc_{length}_{m}_{name}"] = value.cpu().numpy()
+    for s, length, window, low in ((16, 70, 16, True), (16, 70, 0, True), (100, 40, 0, False), (7, 33, 33, False)):
+        b, d = 1, 16
+        g = torch.Generator().manual_seed(s * 1000 + length + window)
+        ck, cv = (torch.randn((b, s, d), generator=g) for _ in range(2))
+        k, v, q = (torch.randn((b, length, d), generator=g) for _ in range(3))
+        cvalid, flags = torch.rand((b, s), generator=g) < 0.8, torch.rand((b, length), generator=g) < 0.9
+        if low:
+            k, v = k.to(torch.bfloat16), v.to(torch.bfloat16)
+        ck, cv, cvalid, k, v, flags, q = (t.to(device) for t in (ck, cv, cvalid, k, v, flags, q))
+        read = torch.empty((b, length, d), device=device)
+        front = memory.read_local_window if window else memory.read_salient_window
+        front(ck, cv, cvalid, k, v, flags, q, out=read, **({"window": window} if window else {}))
+        out[f"window_{s}_{length}_{window}"] = read.cpu().numpy()
+    return out
+
+
+def test_reads_keep_the_order_of_their_sums(device):
+    """The denominators, the carried basis, the normalizer terms and the softmax sums of the window reads
+    add in the order of a wave reduction over 64 lanes (slots or features l, l + 64, .. in turn, then lanes
+    32, 16, .. 1 apart; basis features in pairs 2 k, 2 k + 1). The fixture holds what kernels that reduce by
+    the wave gave: a stack of layers turns another order into other admissions, so it is kept to the bit."""
+    want = np.load(Path(__file__).parent / "golden" / "window_read_bits.npz")
+    got = read_bits(device)
+    assert sorted(got) == sorted(want.files)
+    for name in want.files:
+        np.testing.assert_array_equal(got[name], want[name], err_msg=name)
 
 
 @pytest.mark.parametrize("b, length", [(3, 130), (64, 1)])
