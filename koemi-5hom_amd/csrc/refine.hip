@@ -88,28 +88,25 @@ __device__ __forceinline__ float wave_sum_each(float (&v)[N]) {
     return s;
 }
 
-// Columns [8 lane + 512 g, + 8) of a row, g < NG (zeros past D, a multiple of 8).
-template <int NG, typename T>
-__device__ __forceinline__ void load_columns(const T* __restrict__ row, int64_t D, float (&x)[NG][8]) {
+// Columns lane + 64 i of a row, i < N (zeros past D): the order in which a wave walks
+// a row one column a lane, so that the sums below have a wave-per-query walk's bits.
+template <int N, typename T>
+__device__ __forceinline__ void load_columns(const T* __restrict__ row, int64_t D, float (&x)[N]) {
+    T v[N];
 #pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const int64_t c = 512 * g + 8 * lane_id();
-        const int64_t cc = min(c, D - 8);
-        const float4 a = load4(row + cc), b = load4(row + cc + 4);
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    for (int i = 0; i < N; ++i) v[i] = row[min(static_cast<int64_t>(lane_id() + kWave * i), D - 1)];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[g][i] = c < D ? v[i] : 0.0f;
-    }
+    for (int i = 0; i < N; ++i) x[i] = lane_id() + kWave * i < D ? to_f32(v[i]) : 0.0f;
 }
 
 // The novelty of kNoveltyRun consecutive queries of a window row per wave: the
 // queries stay in registers and every key of their joint window is read (and its
 // norm formed) once, the next key's loads under this one's products. Bound by the
 // latency of that walk (window + 3 keys); [64, 128, 1024] at a window of 16, bf16
-// keys: 33 us (52 at runs of eight, 32 at two), against 112 for a wave per query that
-// reads its 16 keys alone.
+// keys: 34 us, against 109 for a wave per query that reads its 16 keys alone (runs of
+// eight take 1.6 times as long, of two about the same).
 constexpr int kNoveltyRun = 4;
-template <typename KT, int NG>
+template <typename KT, int N>
 __global__ __launch_bounds__(256, 2) void local_novelty_run_kernel(
     const float* __restrict__ carried_keys, const uint8_t* __restrict__ carried_valid, const KT* __restrict__ keys,
     int64_t key_stride, const uint8_t* __restrict__ key_valid, const float* __restrict__ queries, int64_t q_stride,
@@ -118,46 +115,40 @@ __global__ __launch_bounds__(256, 2) void local_novelty_run_kernel(
     const int64_t job = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;  // (row, run)
     if (job >= rows * runs) return;
     const int64_t r = job / runs, t0 = (job - r * runs) * kNoveltyRun;
-    float q[kNoveltyRun][NG][8], sums[kNoveltyRun];
+    float q[kNoveltyRun][N], sums[kNoveltyRun];
 #pragma unroll
     for (int j = 0; j < kNoveltyRun; ++j) {
-        load_columns<NG>(queries + (r * L + min(t0 + j, L - 1)) * q_stride, D, q[j]);
+        load_columns<N>(queries + (r * L + min(t0 + j, L - 1)) * q_stride, D, q[j]);
         sums[j] = 0.0f;
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sums[j] = fmaf(q[j][g][i], q[j][g][i], sums[j]);
+        for (int i = 0; i < N; ++i) sums[j] = fmaf(q[j][i], q[j][i], sums[j]);
     }
     const float qn = fmaxf(sqrtf(wave_sum_each(sums)), 1e-12f);  // of this lane's query
     const int64_t t = t0 + lane_id() / (kWave / kNoveltyRun), own = C + t;
     const int64_t first = max(C + t0 - window, int64_t(0));
     const int64_t last = C + min(t0 + kNoveltyRun, L) - 1;  // one past the last query's slots
-    auto load_key = [&](int64_t s, float (&k)[NG][8]) {
-        if (s < C) load_columns<NG>(carried_keys + (r * C + s) * D, D, k);
-        else load_columns<NG>(keys + (r * L + (s - C)) * key_stride, D, k);
+    auto load_key = [&](int64_t s, float (&k)[N]) {
+        if (s < C) load_columns<N>(carried_keys + (r * C + s) * D, D, k);
+        else load_columns<N>(keys + (r * L + (s - C)) * key_stride, D, k);
     };
     float best = -INFINITY;
     bool any = false;
-    float k[NG][8], next[NG][8];
+    float k[N], next[N];
     if (first < last) load_key(first, next);
     for (int64_t s = first; s < last; ++s) {  // wave-uniform
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) k[g][i] = next[g][i];
+        for (int i = 0; i < N; ++i) k[i] = next[i];
         load_key(min(s + 1, last - 1), next);
         if (!(s < C ? carried_valid[r * C + s] : key_valid[r * L + (s - C)])) continue;
         float kk = 0.0f;
 #pragma unroll
         for (int j = 0; j < kNoveltyRun; ++j) sums[j] = 0.0f;
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
+        for (int i = 0; i < N; ++i) {
+            kk = fmaf(k[i], k[i], kk);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                kk = fmaf(k[g][i], k[g][i], kk);
-#pragma unroll
-                for (int j = 0; j < kNoveltyRun; ++j) sums[j] = fmaf(k[g][i], q[j][g][i], sums[j]);
-            }
+            for (int j = 0; j < kNoveltyRun; ++j) sums[j] = fmaf(k[i], q[j][i], sums[j]);
+        }
         const float dot = wave_sum_each(sums);
         kk = wave_sum(kk);
         if (s < own && s >= own - window) {
@@ -225,15 +216,9 @@ extern "C" int koemi_local_novelty(const float* carried_keys, const uint8_t* car
     if ((jobs + 3) / 4 > 0x7fffffffLL) return fail(KOEMI_ERR_UNSUPPORTED, "local novelty grid too large");
     const dim3 grid(static_cast<unsigned>((jobs + 3) / 4));
     hipStream_t s = as_stream(stream);
-    // Runs of queries where a row fits the registers and every row starts aligned to its
-    // loads (16 bytes of fp32, 8 of bf16); a wave per query otherwise, and for the few
-    // queries of a short window.
-    const auto aligned = [](const void* p, int64_t stride, int64_t size, int64_t to) {
-        return p == nullptr || (reinterpret_cast<uintptr_t>(p) % to == 0 && stride * size % to == 0);
-    };
-    const int64_t key_size = key_dtype == KOEMI_BF16 ? 2 : 4;
-    if (length >= 4 && width % 8 == 0 && width <= 1024 && aligned(carried_keys, width, 4, 16) &&
-        aligned(queries, query_row_stride, 4, 16) && aligned(keys, key_row_stride, key_size, 4 * key_size)) {
+    // Runs of queries where a row fits the registers; a wave per query otherwise, and
+    // for the few queries of a short window. Both give the same bits.
+    if (length >= kNoveltyRun && width <= 16 * kWave) {
         const int64_t run_jobs = rows * ((length + kNoveltyRun - 1) / kNoveltyRun);
         const auto run = [&](auto kernel, const auto* typed_keys) {
             hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((run_jobs + 3) / 4)), dim3(256), 0, s, carried_keys,
@@ -241,12 +226,13 @@ extern "C" int koemi_local_novelty(const float* carried_keys, const uint8_t* car
                                rows, capacity, length, width, window);
             return check_launch("koemi_local_novelty");
         };
+        const bool half = width <= 8 * kWave;
         if (key_dtype == KOEMI_BF16) {
             const bf16* k16 = static_cast<const bf16*>(keys);
-            return width <= 512 ? run(local_novelty_run_kernel<bf16, 1>, k16) : run(local_novelty_run_kernel<bf16, 2>, k16);
+            return half ? run(local_novelty_run_kernel<bf16, 8>, k16) : run(local_novelty_run_kernel<bf16, 16>, k16);
         }
         const float* k32 = static_cast<const float*>(keys);
-        return width <= 512 ? run(local_novelty_run_kernel<float, 1>, k32) : run(local_novelty_run_kernel<float, 2>, k32);
+        return half ? run(local_novelty_run_kernel<float, 8>, k32) : run(local_novelty_run_kernel<float, 16>, k32);
     }
     if (key_dtype == KOEMI_BF16)
         hipLaunchKernelGGL(local_novelty_kernel<bf16>, grid, dim3(256), 0, s, carried_keys, carried_valid,

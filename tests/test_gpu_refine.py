@@ -73,6 +73,23 @@ def test_local_novelty_matches_the_oracle(device, rows, cap, length, d, window, 
         assert abs(float(got[1, 3])) <= 2e-6
 
 
+@pytest.mark.parametrize("d, key_bf16", [(1024, True), (520, False), (512, True), (24, False), (4, True)])
+def test_local_novelty_of_either_layout_has_the_same_bits(device, d, key_bf16):
+    """A row that fits the registers is walked for a run of queries at once, a wider one by a wave per
+    query. Both add a lane's columns d, d + 64, .. in turn and then the lanes, so a row widened with zeros
+    past the registers' 1024 columns has the same novelty to the bit."""
+    rows, cap, length = 3, 16, 29
+    g = torch.Generator().manual_seed(d)
+    ck, keys, q = (torch.randn((rows, n, d), generator=g) for n in (cap, length, length))
+    cv, kv = (torch.rand((rows, n), generator=g) < 0.8 for n in (cap, length))
+    keys = keys.to(torch.bfloat16 if key_bf16 else torch.float32)
+    wide = lambda t: torch.nn.functional.pad(t, (0, 1100 - d))
+    on = lambda *ts: (t.to(device) for t in ts)
+    got = memory.local_novelty(*on(ck, cv, keys, kv, q), window=16)
+    want = memory.local_novelty(*on(wide(ck), cv, wide(keys), kv, wide(q)), window=16)
+    assert torch.equal(got, want)
+
+
 def _refine_terms(proj, surprise, valid, novelty, fast, d, m, rate):
     p64 = proj.astype(np.float64)
     value = np.tanh(p64[..., 2 * d:3 * d])
