@@ -126,12 +126,15 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_forward_kernel(
     red[wn][r] = m;  // both halves of the wave hold the row's value
     __syncthreads();
     m = fmaxf(red[0][r], red[1][r]);
+    // one of several tiles with no logit above minus infinity: its sum is 0, and NaN
+    // where one of them is NaN (which fmaxf passes over)
+    const float ref = v_tiles > 1 && !(m > -__builtin_inff()) ? 0.0f : m;
     float sum = 0.0f;
 #pragma unroll
     for (int j = 0; j < Tile::NT; ++j)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const float e = detmath::det_expf_nonpos(tile.acc[0][j][v] - m);
+            const float e = detmath::det_expf_nonpos(tile.acc[0][j][v] - ref);
             if (j * 32 + 8 * (v / 4) + v % 4 < here) sum = sum + e;
         }
     sum = sum + __shfl_xor(sum, 32, kWave);
@@ -162,11 +165,8 @@ __global__ void surprise_head_finish_kernel(const float* __restrict__ part, cons
     const int64_t t = targets[row];
     float m = -__builtin_inff(), sum = 0.0f;
     for (int64_t i = 0; i < v_tiles; ++i) m = fmaxf(m, p[i * 3 * rows]);
-    for (int64_t i = 0; i < v_tiles; ++i) {
-        const float mi = p[i * 3 * rows], si = p[(i * 3 + 1) * rows];
-        // a tile of minus infinities alone holds a NaN sum and adds nothing to finite ones
-        if (mi > -__builtin_inff() || !(m > -__builtin_inff())) sum = sum + si * detmath::det_expf_nonpos(mi - m);
-    }
+    for (int64_t i = 0; i < v_tiles; ++i)  // a tile of minus infinities adds 0, a NaN stays
+        sum = sum + p[(i * 3 + 1) * rows] * detmath::det_expf_nonpos(p[i * 3 * rows] - m);
     const bool in = t >= 0 && t < V;
     finish_row(m, sum, in ? p[(t / columns * 3 + 2) * rows] : 0.0f, in, valid[row] != 0, log_vocab, row, rows, out, stats);
 }

@@ -287,3 +287,47 @@ def test_causal_surprise_contains_what_is_not_finite(device, dtype):
     assert torch.equal(score[~touched], clean[~touched]) and torch.equal(grad[~touched], clean_grad[~touched])
     assert bool(torch.isnan(score[touched]).all())
     assert not grad[0, 10].any() and not grad[1, 1].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows, vocab", [(70, 65), (70, 129), (70, 67), (70, 257), (9000, 257), (9000, 300), (70, 64), (9000, 256)])
+def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab):
+    """A NaN in the last weight row or the last bias, in a last tile of one column, of several and among
+    minus infinities, makes every valid row's score and gradient NaN, whatever the vocabulary's tiles; a
+    last tile whose biases are all minus infinity leaves the scores of the other columns."""
+
+    g = torch.Generator().manual_seed(rows + vocab)
+    prior = (0.5 * torch.randn((1, rows, 40), generator=g)).to(dtype).to(device)
+    weight = (0.2 * torch.randn((vocab, 40), generator=g)).to(dtype).to(device)
+    bias = (0.1 * torch.randn((vocab,), generator=g)).to(dtype).to(device)
+    tile = 64 if rows == 70 else 256
+    last = (vocab - 1) // tile * tile  # the last tile's first column
+    targets = torch.randint(0, max(last, 1), (1, rows), generator=g).to(device)
+    valid = torch.rand((1, rows), generator=g).to(device) < 0.9
+    def run(weight, bias):
+        leaf = prior.clone().requires_grad_()
+        score = think.causal_surprise(leaf, weight, bias, targets, valid)
+        return score.detach(), torch.autograd.grad(score, leaf, torch.ones_like(score))[0]
+    for where in ("weight", "bias", "bias among minus infinities"):
+        w, b = weight.clone(), bias.clone()
+        if where == "weight":
+            w[vocab - 1, 7] = float("nan")
+        else:
+            if "among" in where:
+                b[last:] = -float("inf")
+            b[vocab - 1] = float("nan")
+        score, grad = run(w, b)
+        assert torch.isnan(score[valid]).all() and torch.isnan(grad[valid]).all(), where
+        assert not score[~valid].any()
+        if where != "weight":  # a NaN weight reaches an invalid row's gradient as 0 x NaN, as in any product
+            assert not grad[~valid].any()
+    if last:
+        b = bias.clone()
+        b[last:] = -float("inf")
+        score, grad = run(weight, b)
+        z = prior.double() @ weight.double()[:last].t() + bias.double()[:last]
+        nll = torch.logsumexp(z, -1) - z.gather(-1, targets[..., None])[..., 0]
+        want = torch.where(valid, 1 - torch.exp(-nll / math.log(vocab)), 0.0)
+        # the fp32 logits of 40 terms of order one and a few roundings, then the score's own type
+        assert bool(((score.double() - want).abs() <= 2.0**-19 + (2.0**-8 if dtype == torch.bfloat16 else 0) * want).all())
+        assert torch.isfinite(grad).all()
