@@ -282,8 +282,11 @@ int koemi_moe_permute(const void* context, int context_dtype, const void* assign
  *   y_i = W_o[e] (silu(W_g[e] x_i + b_g[e]) * (W_v[e] x_i + b_v[e])) + b_o[e];
  * rows past the valid pairs are zero. Weights: gate/value [E, hidden, width],
  * their biases [E, hidden], output [E, width, hidden], its bias [E, width].
- * BF16 runs on bf16 MFMA (fp32 accumulation, the GLU product rounded to bf16
- * between the two GEMMs); F32/F16 run a fp32-accumulating scalar path.
+ * BF16 with width and hidden multiples of 64 runs on bf16 MFMA (fp32
+ * accumulation, the GLU product rounded to bf16 between the two GEMMs), a pair's
+ * expert taken from the segment that holds it. F32, F16 and every other BF16
+ * shape run on matrix-core tiles of exact products' planes (fp32 accumulation and
+ * GLU product); a pair outside its expert's segment is formed by itself there.
  * The tile scheduler reads segment_offsets on device (no host sync). */
 size_t koemi_moe_grouped_mlp_workspace_bytes(int64_t pairs, int64_t width, int64_t hidden,
                                              int64_t expert_count, int dtype);

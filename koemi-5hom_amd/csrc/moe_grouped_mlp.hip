@@ -15,7 +15,8 @@
 // Both operands are K-contiguous ("TN"), so every MFMA fragment is one 16-byte
 // LDS read per lane. The tile schedule is built on device from segment_offsets
 // (no host synchronisation): tile slot -> (expert, first row). Rows past the
-// valid pairs are zero-filled.
+// valid pairs are zero-filled. float32, float16 and shapes off the bf16 tiles run
+// on tiles of split_gemm.hpp (the any-shape path below).
 #include "common.hpp"
 #include "mfma_stage.hpp"
 #include "split_gemm.hpp"
@@ -104,8 +105,10 @@ __device__ __forceinline__ float silu_f(float v) {
 // exclusive prefix in LDS (in `scratch`, E + 1 entries of global memory, where
 // the experts are too many for it), then a binary search per slot. Segment bounds are
 // clamped to [0, pairs] so that malformed offsets can never address rows
-// outside the operands.
+// outside the operands. CHECKED: offsets that decrease give no slots at all and
+// the count kUnordered, for settle_rows_kernel.
 constexpr int kSchedThreads = 1024;
+constexpr int32_t kUnordered = -1;
 constexpr int64_t kMaxScheduleExperts = 8191;  // (E + 1) int32 tile prefixes stay within 32 KiB of LDS
 
 __device__ __forceinline__ void segment_bounds(const int64_t* __restrict__ offsets, int64_t e, int64_t pairs,
@@ -114,6 +117,7 @@ __device__ __forceinline__ void segment_bounds(const int64_t* __restrict__ offse
     hi = min(max(offsets[e + 1], lo), pairs);
 }
 
+template <bool CHECKED>
 __global__ __launch_bounds__(kSchedThreads) void build_schedule_kernel(
     const int64_t* __restrict__ offsets, int64_t E, int64_t pairs, int64_t max_slots,
     int32_t* __restrict__ slot_expert, int64_t* __restrict__ slot_row, int64_t* __restrict__ slot_end,
@@ -123,13 +127,17 @@ __global__ __launch_bounds__(kSchedThreads) void build_schedule_kernel(
     __shared__ int32_t wave_tot[kSchedThreads / kWave];
     const int tid = threadIdx.x;
     const int64_t n = E + 1;
+    int decreases = 0;
     for (int64_t e = tid; e < E; e += kSchedThreads) {
         int64_t lo, hi;
         segment_bounds(offsets, e, pairs, lo, hi);
+        if (CHECKED && offsets[e] > offsets[e + 1]) decreases = 1;
         first_tile[e] = static_cast<int32_t>((hi - lo + bm - 1) / bm);
     }
     if (tid == 0) first_tile[E] = 0;
-    __syncthreads();
+    bool ordered = true;
+    if constexpr (CHECKED) ordered = __syncthreads_or(decreases) == 0;
+    else __syncthreads();
     const int64_t per = (n + kSchedThreads - 1) / kSchedThreads;
     const int64_t b0 = min(n, tid * per), b1 = min(n, b0 + per);
     int32_t sum = 0;
@@ -142,8 +150,8 @@ __global__ __launch_bounds__(kSchedThreads) void build_schedule_kernel(
         run += v;
     }
     __syncthreads();
-    const int64_t total = first_tile[E];
-    if (tid == 0) slot_expert[max_slots] = static_cast<int32_t>(total);  // slots in use
+    const int64_t total = ordered ? first_tile[E] : 0;
+    if (tid == 0) slot_expert[max_slots] = ordered ? static_cast<int32_t>(total) : kUnordered;  // slots in use
     for (int64_t slot = tid; slot < max_slots; slot += kSchedThreads) {
         if (slot >= total) {
             slot_expert[slot] = -1;
@@ -608,7 +616,8 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
     // workgroup b runs on XCD b % 8: every XCD takes a contiguous range of
     // tiles, in groups of kGroupM slots, so that its L2 serves the operands
     // that concurrently running tiles share
-    const uint32_t slots = static_cast<uint32_t>(min(static_cast<int64_t>(slot_expert[max_slots]), max_slots));
+    const int32_t used = max(slot_expert[max_slots], 0);  // kUnordered: none
+    const uint32_t slots = static_cast<uint32_t>(min(static_cast<int64_t>(used), max_slots));
     const uint32_t tiles = slots * static_cast<uint32_t>(n_tiles);
     const uint32_t per_xcd = (tiles + 7) / 8;
     if ((blockIdx.x >> 3) >= per_xcd) return;
@@ -904,6 +913,51 @@ __global__ void zero_tail_rows_kernel(T* __restrict__ y, const int64_t* __restri
         for (int64_t c = threadIdx.x; c < D; c += blockDim.x) y[p * D + c] = static_cast<T>(0.0f);
 }
 
+// The rows that the any-shape path's tiles leave. Rows past the valid pairs are
+// zero, as above. A valid pair's expert is sorted_experts[i]: where that expert's
+// segment does not hold row i (offsets that start above 0 or decrease, or ids that
+// disagree with them), a workgroup forms the row with plain multiply-add chains.
+// Well-formed pairs cost one look at their id and segment, a thread per row.
+template <typename T>
+__global__ __launch_bounds__(256) void settle_rows_kernel(
+    const T* __restrict__ x, const int64_t* __restrict__ experts, const int64_t* __restrict__ offsets,
+    const T* __restrict__ Wg, const T* __restrict__ bg, const T* __restrict__ Wv, const T* __restrict__ bv,
+    const T* __restrict__ Wo, const T* __restrict__ bo, float* __restrict__ H, T* __restrict__ y, int64_t pairs,
+    int64_t D, int64_t Hd, int64_t ld_h, int64_t E, const int32_t* __restrict__ slots_used) {
+    __shared__ uint8_t stray[256];
+    const int tid = threadIdx.x;
+    const int64_t valid = min(max(offsets[E], int64_t(0)), pairs);
+    const bool ordered = *slots_used != kUnordered;
+    for (int64_t p = valid + blockIdx.x; p < pairs; p += gridDim.x)
+        for (int64_t c = tid; c < D; c += 256) y[p * D + c] = static_cast<T>(0.0f);
+    // the rows blockIdx.x + j gridDim.x, 256 at a time
+    for (int64_t p0 = blockIdx.x; p0 < valid; p0 += static_cast<int64_t>(gridDim.x) * 256) {
+        const int64_t p = p0 + static_cast<int64_t>(tid) * gridDim.x;
+        bool out = false;
+        if (p < valid) {
+            const int64_t e = experts[p];
+            if (e >= 0 && e < E) out = !ordered || p < offsets[e] || p >= offsets[e + 1];
+        }
+        stray[tid] = out;
+        if (__syncthreads_or(out) == 0) continue;
+        for (int j = 0; j < 256; ++j) {
+            if (!stray[j]) continue;  // the same for the whole workgroup
+            const int64_t row = p0 + static_cast<int64_t>(j) * gridDim.x, e = experts[row];
+            const T* xr = x + row * D;
+            float* hr = H + row * ld_h;
+            for (int64_t h = tid; h < Hd; h += 256) {
+                const int64_t w = e * Hd + h;
+                const float g = split_gemm::scalar_dot(xr, Wg + w * D, D, to_f32(bg[w]));
+                hr[h] = silu_f(g) * split_gemm::scalar_dot(xr, Wv + w * D, D, to_f32(bv[w]));
+            }
+            __syncthreads();
+            for (int64_t c = tid; c < D; c += 256)
+                y[row * D + c] = from_f32<T>(split_gemm::scalar_dot(hr, Wo + (e * D + c) * Hd, Hd, to_f32(bo[e * D + c])));
+        }
+        __syncthreads();  // stray is rewritten
+    }
+}
+
 inline unsigned tail_blocks(int64_t pairs) { return static_cast<unsigned>(pairs < 1024 ? (pairs > 0 ? pairs : 1) : 1024); }
 
 // Compute units of the current device (the rounds of one-workgroup-per-CU tiles).
@@ -919,9 +973,9 @@ int64_t device_cus() {
 }
 
 template <typename T, int BM>
-int run_any(const void* x, const int64_t* offsets, const void* Wg, const void* bg, const void* Wv, const void* bv,
-            const void* Wo, const void* bo, void* y, int64_t P, int64_t D, int64_t Hd, int64_t E,
-            const MlpWorkspace& ws, char* base, hipStream_t s) {
+int run_any(const void* x, const int64_t* experts, const int64_t* offsets, const void* Wg, const void* bg,
+            const void* Wv, const void* bv, const void* Wo, const void* bo, void* y, int64_t P, int64_t D, int64_t Hd,
+            int64_t E, const MlpWorkspace& ws, char* base, hipStream_t s) {
     float* H = reinterpret_cast<float*>(base + ws.hidden_off);
     int32_t* slot_expert = reinterpret_cast<int32_t*>(base + ws.slot_expert_off);
     int64_t* slot_row = reinterpret_cast<int64_t*>(base + ws.slot_row_off);
@@ -935,7 +989,7 @@ int run_any(const void* x, const int64_t* offsets, const void* Wg, const void* b
     const int64_t tiles2 = narrow ? (D + 63) / 64 : (D + 127) / 128;
     if (ws.max_slots * (tiles1 > tiles2 ? tiles1 : tiles2) > 0x7ffffff0LL)
         return fail(KOEMI_ERR_UNSUPPORTED, "too many tiles for the grouped MLP");
-    hipLaunchKernelGGL(build_schedule_kernel, dim3(1), dim3(kSchedThreads),
+    hipLaunchKernelGGL(build_schedule_kernel<true>, dim3(1), dim3(kSchedThreads),
                        lds_prefix ? static_cast<size_t>(E + 1) * sizeof(int32_t) : 0, s, offsets, E, P, ws.max_slots,
                        slot_expert, slot_row, slot_end, static_cast<int64_t>(BM),
                        lds_prefix ? nullptr : reinterpret_cast<int32_t*>(base + ws.first_tile_off));
@@ -976,9 +1030,10 @@ int run_any(const void* x, const int64_t* offsets, const void* Wg, const void* b
              : bytes2 == 8 ? second(grouped_gemm_any_kernel<false, float, T, BM, 128, 8>)
                            : second(grouped_gemm_any_kernel<false, float, T, BM, 128, 0>);
     if (st != KOEMI_OK) return st;
-    hipLaunchKernelGGL(zero_tail_rows_kernel<T>, dim3(tail_blocks(P)), dim3(256), 0, s, static_cast<T*>(y),
-                       offsets + E, P, D);
-    return check_launch("koemi_moe_grouped_mlp(zero)");
+    hipLaunchKernelGGL(settle_rows_kernel<T>, dim3(tail_blocks(P)), dim3(256), 0, s, static_cast<const T*>(x), experts,
+                       offsets, wg, static_cast<const T*>(bg), wv, static_cast<const T*>(bv), wo,
+                       static_cast<const T*>(bo), H, static_cast<T*>(y), P, D, Hd, ld_h, E, slot_expert + ws.max_slots);
+    return check_launch("koemi_moe_grouped_mlp(settle)");
 }
 
 // x_index (or null): GEMM 1 reads context row x_index[i] (of x_rows) for pair i.
@@ -1000,7 +1055,7 @@ int run_mfma(const void* x, const int64_t* x_index, int64_t x_rows, const int64_
     if (P <= kSkinnyMaxRowsPerExpert * E && E * ((Hd > D ? Hd : D) / kSkinnyCols) <= 0x7fffffffLL) {
         return run_skinny<false>(x, x_index, x_rows, offsets, Wg, bg, Wv, bv, Wo, bo, y, P, D, Hd, E, H, s, zero_tail);
     }
-    hipLaunchKernelGGL(build_schedule_kernel, dim3(1), dim3(kSchedThreads), static_cast<size_t>(E + 1) * sizeof(int32_t),
+    hipLaunchKernelGGL(build_schedule_kernel<false>, dim3(1), dim3(kSchedThreads), static_cast<size_t>(E + 1) * sizeof(int32_t),
                        s, offsets, E, P, ws.max_slots, slot_expert, slot_row, slot_end, static_cast<int64_t>(kBM),
                        static_cast<int32_t*>(nullptr));
     int st = check_launch("koemi_moe_grouped_mlp(schedule)");
@@ -1085,8 +1140,8 @@ extern "C" int koemi_moe_grouped_mlp(const void* sorted_context, const int64_t* 
     const auto run = [&](auto tag) {
         using T = decltype(tag);
         const auto go = small ? run_any<T, 64> : run_any<T, 128>;
-        return go(sorted_context, segment_offsets, gate_weights, gate_biases, value_weights, value_biases,
-                  output_weights, output_biases, output, pairs, width, hidden, expert_count, ws, base, s);
+        return go(sorted_context, sorted_experts, segment_offsets, gate_weights, gate_biases, value_weights,
+                  value_biases, output_weights, output_biases, output, pairs, width, hidden, expert_count, ws, base, s);
     };
     switch (dtype) {
         case KOEMI_F32: return run(float{});

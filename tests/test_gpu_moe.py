@@ -23,7 +23,7 @@ import torch
 import torch.nn.functional as F
 
 import oracle
-from koemi_amd import moe, workloads
+from koemi_amd import _native, moe, workloads
 
 pytestmark = pytest.mark.gpu
 GOLDEN = json.loads((Path(__file__).parent / "golden" / "kats.json").read_text())
@@ -626,3 +626,59 @@ def test_segment_check_equals_the_torch_expressions(device, pairs, offsets, limi
     unordered = any(b < a for a, b in zip(offsets, offsets[1:])) or offsets[0] < 0
     got = moe._segment_flags(ids.to(device), torch.tensor(offsets, device=device), limit)
     assert got == (outside, bad, unordered)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("offsets, valid", [
+    ([3, 8, 8, 20], True), ([20, 20, 20, 20], True), ([0, 5, 9, 17], True), ([0, 0, 0, 300], True),
+    ([0, 12, 5, 20], False), ([9, 4, 30, 2], False), ([-7, 3, 11, 40], False),
+])
+def test_any_shape_pairs_outside_their_segment(device, dtype, offsets, valid):
+    """Pair i < offsets[E] runs through expert sorted_experts[i] also where the offsets start above 0, do
+    not fit the ids or decrease (the checked call refuses the last kind), and rows past it are zero."""
+
+    E, D, H, P = 3, 30, 21, max(25, max(offsets) + 3 if valid else 25)
+    g = torch.Generator().manual_seed(sum(offsets))
+    x = torch.randn((P, D), generator=g).to(dtype)
+    experts = torch.sort(torch.randint(0, E, (P,), generator=g))[0]
+    experts[5:9] = torch.tensor([2, 0, 1, 2])
+    ws = [(0.2 * torch.randn(s, generator=g)).to(dtype) for s in ((E, H, D), (E, H), (E, H, D), (E, H), (E, D, H), (E, D))]
+    on = lambda t: t.to(device)
+    args = (on(x), on(experts), on(torch.tensor(offsets)), *map(on, ws))
+    if not valid:
+        with pytest.raises(moe.CudaMoeValidationError):
+            moe.grouped_expert_mlp_inference(*args)
+    got = moe.grouped_expert_mlp_inference(*args, validate=valid).double().cpu()
+    live = min(max(offsets[-1], 0), P)
+    gw, gb, vw, vb, ow, ob = (w.double() for w in ws)
+    for i in range(live):
+        e = int(experts[i])
+        gate, value = gw[e] @ x[i].double() + gb[e], vw[e] @ x[i].double() + vb[e]
+        want = ow[e] @ (gate * torch.sigmoid(gate) * value) + ob[e]
+        # half an ulp of the type and fp32 sums of 30 and 21 terms of order one
+        half_ulp = {torch.float32: 2.0**-24, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+        assert bool(((got[i] - want).abs() <= half_ulp * want.abs() + 2.0**-19).all()), i
+    assert not got[live:].any()
+
+
+def test_any_shape_of_more_experts_than_the_prefix_in_lds(device):
+    """8200 experts: the tiles' prefix lies in the workspace; the bf16 tile path refuses as many."""
+
+    E, D, H = 8200, 12, 8
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn((300, D), generator=g)
+    experts = torch.sort(torch.randint(0, E, (300,), generator=g))[0]
+    experts[-40:] = E - 1
+    offsets = torch.searchsorted(experts, torch.arange(E + 1))
+    ws = [0.2 * torch.randn(s, generator=g) for s in ((E, H, D), (E, H), (E, H, D), (E, H), (E, D, H), (E, D))]
+    on = lambda t: t.to(device)
+    got = moe.grouped_expert_mlp_inference(on(x), on(experts), on(offsets), *map(on, ws)).double().cpu()
+    gw, gb, vw, vb, ow, ob = (w[experts].double() for w in ws)
+    dot = lambda w, v: (w @ v[..., None])[..., 0]
+    gate, value = dot(gw, x.double()) + gb, dot(vw, x.double()) + vb
+    want = dot(ow, gate * torch.sigmoid(gate) * value) + ob
+    assert bool(((got - want).abs() <= 2.0**-24 * want.abs() + 2.0**-19).all())
+    wide = [torch.zeros(s, device=device, dtype=torch.bfloat16) for s in ((E, 64, 64), (E, 64), (E, 64, 64), (E, 64), (E, 64, 64), (E, 64))]
+    with pytest.raises(_native.NativeCallError, match="at most 8191 experts"):
+        moe.grouped_expert_mlp_inference(torch.zeros((300, 64), device=device, dtype=torch.bfloat16), on(experts),
+                                         on(offsets), *wide)
