@@ -458,6 +458,10 @@ template <typename T>
 int launch_backward(const void* g, const void* x, const void* w, const float* inv, void* dx,
                     void* dw, int64_t rows, int64_t H, float* partial, hipStream_t stream) {
     constexpr int N = Vec16<T>::N;
+    if (rows == 0) {  // the operands may be null: only grad_weight is written, with zeros
+        launch_column_sum(partial, static_cast<T*>(dw), 0, H, stream);
+        return check_launch("koemi_rmsnorm_silu_backward");
+    }
     const T* gp = static_cast<const T*>(g);
     const T* xp = static_cast<const T*>(x);
     const T* wp = static_cast<const T*>(w);
@@ -470,7 +474,7 @@ int launch_backward(const void* g, const void* x, const void* w, const float* in
     auto run = [&](auto kernel, int64_t lanes_per_row) {
         const int64_t per_block = kWave * kNormWaves / lanes_per_row;
         const int64_t need = (rows + per_block - 1) / per_block;
-        if (need < blocks) blocks = need < 1 ? 1 : need;
+        if (need < blocks) blocks = need;
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kWave * kNormWaves), 0, stream, gp, xp, wp,
                            inv, dxp, partial, rows, Hi);
         launched = true;

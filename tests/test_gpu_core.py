@@ -15,7 +15,7 @@ import torch
 import torch.nn.functional as F
 
 import oracle
-from koemi_amd import core, loader, workloads
+from koemi_amd import _native, core, loader, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -143,3 +143,16 @@ def test_rows_of_every_layout(device, dtype, rows, hidden, offset):
         got = got.detach().double().cpu()
         bound = half_ulp * want.abs() + (16 + terms) * 2.0**-24 * (1.0 + want.abs().max())
         assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hidden", [1, 512, 8200])
+def test_backward_of_no_rows_takes_null_operands(device, dtype, hidden):
+    """The C entry accepts null operands for rows == 0 and writes a zero weight gradient."""
+
+    grad_weight = torch.full((hidden,), 7.0, device=device, dtype=dtype)
+    need = _native.query("koemi_rmsnorm_silu_backward_workspace_bytes", 0, hidden)
+    workspace = torch.empty((max(need, 1),), device=device, dtype=torch.uint8)
+    _native.call("koemi_rmsnorm_silu_backward", None, None, None, None, None, grad_weight.data_ptr(), 0, hidden,
+                 _native.dtype_code(dtype), workspace.data_ptr(), need, _native.stream_of(device))
+    assert not grad_weight.any()
