@@ -331,3 +331,38 @@ def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab):
         # the fp32 logits of 40 terms of order one and a few roundings, then the score's own type
         assert bool(((score.double() - want).abs() <= 2.0**-19 + (2.0**-8 if dtype == torch.bfloat16 else 0) * want).all())
         assert torch.isfinite(grad).all()
+
+
+@pytest.mark.parametrize("kind, rows", [(k, r) for k in ("normal", "positive") for r in (1, 2, 7, 64, 1000, 4096)]
+                         + [("low planes set", r) for r in (1, 2, 7)])
+def test_fp32_products_of_the_head_round_either_way(device, kind, rows):
+    """grad_weight = G^T prior in fp32 by itself: with the identity as weight grad_prior is G to the bit.
+
+    In units of 2^-24 of the sum of a product's |terms|: every entry within 4 sqrt(rows) (Higham's sqrt(n)
+    model with a factor of 4; one term comes out within 2.3), and the mean of the signed errors over the
+    4096 entries within 0.6 for one or two terms (the matrix unit cuts off below its sum's last bit: 0.29
+    and 0.18 measured) and 0.3 for more (0.13 and less), where planes cut off at the operand end 0.7 to 1.1
+    below. "low planes set": operands a few steps below 1 + 2^-7, whose low planes are the largest; their
+    terms are nearly one constant, so what is dropped (at most 1) and cut off (1/2) does not average out,
+    bound 1.5 (cut-off planes end 6.9 below), and so would the steps' roundings of many terms, in any fp32
+    sum, hence few rows."""
+
+    g = torch.Generator().manual_seed(rows)
+    width = 64
+    if kind == "normal":
+        prior = torch.randn((1, rows, width), generator=g)
+    elif kind == "positive":
+        prior = torch.rand((1, rows, width), generator=g) + 0.5
+    else:
+        prior = 1 + 2.0**-7 - 2.0**-23 * (1 + torch.randint(0, 64, (1, rows, width), generator=g))
+    prior = prior.to(device).requires_grad_()
+    weight = torch.eye(width, device=device).requires_grad_()
+    targets = torch.zeros((1, rows), dtype=torch.int64, device=device)  # one target: a column of G has one sign
+    score = think.causal_surprise(prior, weight, torch.zeros(width, device=device), targets,
+                                  torch.ones((1, rows), dtype=torch.bool, device=device))
+    grad, grad_weight = torch.autograd.grad(score, (prior, weight), torch.ones_like(score))
+    G, p = grad.view(rows, width).double(), prior.detach().view(rows, width).double()
+    units = (grad_weight.double() - G.t() @ p) / (2.0**-24 * (G.t().abs() @ p.abs()))
+    assert float(units.abs().max()) <= 4 * math.sqrt(rows), float(units.abs().max())
+    mean = float((units * torch.sign(G.t() @ p)).mean())
+    assert abs(mean) <= (1.5 if kind == "low planes set" else 0.6 if rows <= 2 else 0.3), mean
