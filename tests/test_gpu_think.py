@@ -366,3 +366,32 @@ def test_fp32_products_of_the_head_round_either_way(device, kind, rows):
     assert float(units.abs().max()) <= 4 * math.sqrt(rows), float(units.abs().max())
     mean = float((units * torch.sign(G.t() @ p)).mean())
     assert abs(mean) <= (1.5 if kind == "low planes set" else 0.6 if rows <= 2 else 0.3), mean
+
+
+@pytest.mark.parametrize("rows, width, vocab", [(1024, 128, 1000), (128, 300, 1000), (64, 1024, 256), (16, 512, 3000)])
+def test_fp32_gradients_of_few_tiles_err_no_more_than_the_library(device, rows, width, vocab):
+    """For few output tiles the library's fp32 products split K over workgroups, which leaves short sums.
+    The head's gradients against float64 are no further off than the same formula in fp32 torch operations
+    on those products (1.1: the spread of a norm over this many entries of independent roundings)."""
+
+    g = torch.Generator().manual_seed(rows + width + vocab)
+    prior = (0.5 * torch.randn((1, rows, width), generator=g)).to(device)
+    weight = (2.0 / math.sqrt(width) * torch.randn((vocab, width), generator=g)).to(device)
+    bias = (0.1 * torch.randn((vocab,), generator=g)).to(device)
+    targets = torch.randint(0, vocab, (1, rows), generator=g).to(device)
+    valid = torch.ones((1, rows), dtype=torch.bool, device=device)
+    up = torch.randn((1, rows), generator=g).to(device)
+    def composite(p, w, b):
+        z = p.view(rows, width) @ w.t() + b
+        nll = torch.logsumexp(z, -1) - z.gather(-1, targets.view(rows, 1))[:, 0]
+        return (1 - torch.exp(-nll / math.log(vocab))).view(1, rows)
+    def grads(front, dtype):
+        leaves = [t.to(dtype).requires_grad_() for t in (prior, weight, bias)]
+        return torch.autograd.grad(front(*leaves), leaves, up.to(dtype))
+    want = grads(composite, torch.float64)
+    library = grads(composite, torch.float32)
+    got = grads(lambda p, w, b: think.causal_surprise(p, w, b, targets, valid), torch.float32)
+    for have, lib, ref in zip(got[:2], library, want):
+        err, bar = (float((x.double() - ref).norm() / ref.norm()) for x in (have, lib))
+        print(f"{rows} {width} {vocab}: {err:.2e}, library {bar:.2e}", flush=True)
+        assert err <= 1.1 * bar
