@@ -114,9 +114,11 @@ int koemi_surprise_rows_backward(const float* logits, const void* bias, const in
 /* causal_surprise (think/surprise_kernel.cu:194-328) with the content head's
  * product inside: prior [rows, width], weight [vocab, width], bias [vocab] and
  * surprise [rows] of `dtype` (F32/F16/BF16), fp32 accumulation (products of
- * 16-bit operands exact, of fp32 ones to 2^-24, rounded either way). stats fp32 [3, rows] (maximum, sum of exponentials and negative
- * log-likelihood of each row's logits) is what the backward reads. The workspace
- * (where the vocabulary takes several tiles) holds their parts of them. */
+ * 16-bit operands exact, of fp32 ones to 2^-24, rounded either way). stats fp32
+ * [3, rows] (maximum, sum of exponentials and negative log-likelihood of each
+ * row's logits) is what the backward reads. The workspace (where the vocabulary
+ * takes several tiles, or few tiles take the width in chunks) holds their parts of
+ * them. */
 size_t koemi_surprise_head_forward_workspace_bytes(int64_t rows, int64_t vocab);
 int koemi_surprise_head_forward(const void* prior, const void* weight, const void* bias, const int64_t* target_ids,
                                 const uint8_t* valid_mask, void* surprise, float* stats, int64_t rows, int64_t width,

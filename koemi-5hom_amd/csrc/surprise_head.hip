@@ -31,7 +31,7 @@ constexpr int kRows = 64;  // rows of a head tile
 // of loads in flight since no second workgroup hides them (256 rows x
 // 1024, fp32: 66 -> 26 us; a tile step costs its latency there).
 constexpr int kWide = 256, kNarrow = 64;
-constexpr int64_t kWideTiles = 128;
+constexpr int64_t kWideTiles = 256;
 
 template <typename T, int BN>
 using HeadTile = split_gemm::Tile<T, T, kRows, BN, false, false, BN == kNarrow ? 4 : 1>;
@@ -171,6 +171,122 @@ __global__ void surprise_head_finish_kernel(const float* __restrict__ part, cons
     finish_row(m, sum, in ? p[(t / columns * 3 + 2) * rows] : 0.0f, in, valid[row] != 0, log_vocab, row, rows, out, stats);
 }
 
+// Few 64 x 64 tiles and a wide state: each tile's sum over the width in chunks, so
+// that the chip is full ([64, 4096] fp32, vocabulary 256: forward 85 -> 17 us, a
+// tile's walk over its 128 K steps before). The chunks' logits go to part
+// [chunks, rows, V] and are added (column_sum.hpp) for the two kernels after it.
+constexpr int64_t kSplitWidth = 256;  // width of a chunk at least: four to eight K steps
+constexpr int64_t kMostSplitTiles = 512;
+inline int64_t head_tiles_of(int64_t rows, int64_t V) { return (rows + 63) / 64 * ((V + 63) / 64); }
+// The chunks aimed at: a workgroup to each CU, two where fp32 planes make a long walk
+// ([2048, 4096], vocabulary 256, with gradients: 213 and 188 us; [1024, 1024], 1000: 129
+// and 144; 16-bit operands: no shape gained).
+inline int64_t split_tiles(int64_t D, bool fp32) { return fp32 && D >= 2048 ? kMostSplitTiles : 256; }
+inline int64_t head_chunk(int64_t rows, int64_t D, int64_t V, bool fp32) {  // a chunk's width; D: one chunk
+    const int64_t chunks = std::min(split_tiles(D, fp32) / head_tiles_of(rows, V), D / kSplitWidth);
+    return chunks < 2 ? D : ((D + chunks - 1) / chunks + 63) / 64 * 64;
+}
+inline int64_t head_chunks(int64_t rows, int64_t D, int64_t V, bool fp32) {
+    const int64_t width = head_chunk(rows, D, V, fp32);
+    return (D + width - 1) / width;
+}
+inline int64_t logits_floats(int64_t rows, int64_t V, int64_t chunks) {  // the logits and their chunks
+    return (rows * V + 63) / 64 * 64 + chunks * rows * V;
+}
+
+template <typename T, int BYTES>
+__global__ __launch_bounds__(kThreads, 2) void surprise_head_product_kernel(
+    const T* __restrict__ prior, const T* __restrict__ weight, float* __restrict__ part, int64_t rows, int64_t D,
+    int64_t V, int64_t v_tiles, int64_t tiles, int64_t chunk_width, int vec_out) {
+    using Tile = HeadTile<T, kNarrow>;
+    constexpr int kRegion = split_gemm::store_bytes<float, 1>();
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes > 4 * kRegion ? Tile::kLdsBytes : 4 * kRegion];
+    const int64_t chunk = blockIdx.x / tiles, tile_id = blockIdx.x % tiles;
+    const int64_t row0 = tile_id / v_tiles * kRows, v0 = tile_id % v_tiles * kNarrow;
+    const int64_t k0 = chunk * chunk_width, k1 = min(D, k0 + chunk_width);  // chunk_width is a multiple of BK
+    const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
+    Tile tile;
+    tile.template run<BYTES, BYTES>(
+        lds, D, D, k0, k1, [&](int r) { return prior + min(row0 + r, rows - 1) * D; },
+        [&](int r) { return weight + min(v0 + r, V - 1) * D; }, [&](int) { return wn * 32; });
+    split_gemm::lds_barrier();  // the output rows pass through LDS
+    const int64_t row = row0 + wm * 32, first = v0 + wn * 32;
+    float o[1][16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[0][v] = tile.acc[0][0][v];
+    float* out = part + (chunk * rows + row) * V + first;
+    split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, V, rows - row, V - first, vec_out);
+    if constexpr (!Tile::kNative)
+        split_gemm::fix_not_finite(o, [&](int, int v) {
+            const int r = lane_id() & 31, c = split_gemm::acc_column(v);
+            if (row + r < rows && first + c < V)
+                out[r * V + c] = split_gemm::scalar_dot(prior + (row + r) * D + k0, weight + (first + c) * D + k0, k1 - k0, 0.0f);
+        });
+}
+
+// Scores of logits [rows, V], a wave per row.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void surprise_head_score_kernel(
+    const float* __restrict__ logits, const T* __restrict__ bias, const int64_t* __restrict__ targets,
+    const uint8_t* __restrict__ valid, T* __restrict__ out, float* __restrict__ stats, int64_t rows, int64_t V,
+    float log_vocab) {
+#pragma clang fp contract(off)
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * (kThreads / kWave) + threadIdx.x / kWave;
+    if (row >= rows) return;
+    const float* z = logits + row * V;
+    const int64_t t = targets[row];
+    const bool in = t >= 0 && t < V;
+    const float target = in ? z[t] + to_f32(bias[t]) : 0.0f;
+    float m = -__builtin_inff();
+#pragma unroll 4
+    for (int64_t c = lane_id(); c < V; c += kWave) m = fmaxf(m, z[c] + to_f32(bias[c]));
+    m = wave_max_xor(m);
+    float sum = 0.0f;
+#pragma unroll 4
+    for (int64_t c = lane_id(); c < V; c += kWave) sum = sum + detmath::det_expf_nonpos((z[c] + to_f32(bias[c])) - m);
+    sum = wave_sum_xor(sum);
+    if (lane_id() == 0) finish_row(m, sum, target, in, valid[row] != 0, log_vocab, row, rows, out, stats);
+}
+
+// The logit gradient below of logits [rows, V]: 64 rows x 64 columns a workgroup,
+// four rows to each of its waves (sixteen rows to a wave, one after the other: 15 us
+// for 128 rows x 1000).
+constexpr int kSplitGradThreads = 1024;
+template <typename T>
+__global__ __launch_bounds__(kSplitGradThreads) void surprise_head_split_grad_kernel(
+    const float* __restrict__ logits, const T* __restrict__ bias, const int64_t* __restrict__ targets,
+    const uint8_t* __restrict__ valid, const T* __restrict__ grad, const float* __restrict__ stats, float* __restrict__ G,
+    float* __restrict__ bias_partial, int64_t rows, int64_t V, int64_t v_tiles, float log_vocab) {
+#pragma clang fp contract(off)
+    constexpr int kWaves = kSplitGradThreads / kWave;
+    __shared__ float sums[kWaves][kWave];
+    const int wave = threadIdx.x / kWave;
+    const int64_t block = blockIdx.x / v_tiles, c = blockIdx.x % v_tiles * kWave + lane_id();
+    const int64_t cc = min(c, V - 1);
+    const float b = to_f32(bias[cc]);
+    float acc[kRows / kWaves];
+#pragma unroll
+    for (int i = 0; i < kRows / kWaves; ++i) {
+        const int64_t row = block * kRows + wave * (kRows / kWaves) + i, rr = min(row, rows - 1);
+        const int64_t t = targets[rr];
+        const bool live = row < rows && valid[rr] && t >= 0 && t < V;
+        const float inv_sum = 1.0f / stats[rows + rr];
+        const float gnll = to_f32(grad[rr]) * detmath::det_expf(-stats[2 * rows + rr] / log_vocab) / log_vocab;
+        const float p = detmath::det_expf_nonpos((logits[rr * V + cc] + b) - stats[rr]) * inv_sum;
+        acc[i] = live ? gnll * (p - (c == t ? 1.0f : 0.0f)) : 0.0f;
+        if (row < rows && c < V) G[row * V + c] = acc[i];
+    }
+    static_assert(kRows / kWaves == 4, "the sum below");
+    sums[wave][lane_id()] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    __syncthreads();
+#pragma unroll
+    for (int half = kWaves / 2; half > 0; half >>= 1) {
+        if (wave < half) sums[wave][lane_id()] += sums[wave + half][lane_id()];
+        __syncthreads();
+    }
+    if (wave == 0 && c < V) bias_partial[block * V + c] = sums[0][lane_id()];
+}
+
 // d score / d logits (surprise_kernel.cu:136-192), G [rows, V] fp32:
 //   G_j = g exp(-nll / ln V) / ln V (softmax_j - [j == target]),
 // zero for invalid rows, and the workgroup's 64-row column sums of it (the
@@ -242,25 +358,28 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_logits_kernel(
 
 // grad_prior [rows, D] = G [rows, V] W [V, D]. Bound by its few K steps (eight at a
 // vocabulary of 256) and the splits beside them. At the sizes above 50 us, against
-// 77 for the library's fp32 product and 11 for the cast of its result.
-template <typename T, int B, int BYTES>
+// 77 for the library's fp32 product and 11 for the cast of its result. Of few tiles
+// and a long vocabulary each takes the vocabulary [chunk * chunk_v, + chunk_v)
+// (head_workspace), Out fp32 partial sums then ([16, 4096], vocabulary 50257:
+// 2127 -> 563 us).
+template <typename T, typename Out, int B, int BYTES>
 __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
-    const float* __restrict__ G, const T* __restrict__ weight, T* __restrict__ grad_prior, int64_t rows, int64_t D,
-    int64_t V, int64_t d_tiles, int vec_out) {
+    const float* __restrict__ G, const T* __restrict__ weight, Out* __restrict__ grad_prior, int64_t rows, int64_t D,
+    int64_t V, int64_t d_tiles, int64_t tiles, int64_t chunk_v, int vec_out) {
     constexpr int BM = B, BN = B;
     using Tile = split_gemm::Tile<float, T, BM, BN, false, true, B == 64 ? 4 : 1>;
-    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
-    const int64_t row0 = blockIdx.x / d_tiles * BM, d0 = blockIdx.x % d_tiles * BN;
+    constexpr int J = Tile::NT < 2 ? 1 : 2;
+    constexpr int kRegion = split_gemm::store_bytes<Out, J>();
+    __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes > 4 * kRegion ? Tile::kLdsBytes : 4 * kRegion];
+    const int64_t chunk = blockIdx.x / tiles, tile_id = blockIdx.x % tiles;
+    const int64_t row0 = tile_id / d_tiles * BM, d0 = tile_id % d_tiles * BN;
+    const int64_t k0 = chunk * chunk_v, k1 = min(V, k0 + chunk_v);  // chunk_v is a multiple of BK
     const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
     Tile tile;
     tile.template run<BYTES, kElementLoads>(
-        lds, V, V, 0, (V + Tile::BK - 1) / Tile::BK * Tile::BK,
-        [&](int r) { return G + min(row0 + r, rows - 1) * V; }, [&](int r) { return weight + min(d0 + r, D - 1); },
-        [&](int t) { return wn * (BN / 2) + t * 32; }, 1, D);
+        lds, V, V, k0, k1, [&](int r) { return G + min(row0 + r, rows - 1) * V; },
+        [&](int r) { return weight + min(d0 + r, D - 1); }, [&](int t) { return wn * (BN / 2) + t * 32; }, 1, D);
     split_gemm::lds_barrier();  // the output rows pass through LDS
-    constexpr int J = Tile::NT < 2 ? 1 : 2;
-    constexpr int kRegion = split_gemm::store_bytes<T, J>();
-    static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
 #pragma unroll
     for (int i = 0; i < Tile::MT; ++i) {
         const int64_t block_row = row0 + wm * (BM / 2) + i * 32;
@@ -272,13 +391,13 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
             for (int j = 0; j < J; ++j)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o[j][v] = tile.acc[i][j0 + j][v];
-            T* out = grad_prior + block_row * D + first;
-            split_gemm::store_rows<T, J>(lds + wave * kRegion, o, out, D, rows - block_row, D - first, vec_out);
+            Out* out = grad_prior + (chunk * rows + block_row) * D + first;
+            split_gemm::store_rows<Out, J>(lds + wave * kRegion, o, out, D, rows - block_row, D - first, vec_out);
             split_gemm::fix_not_finite(o, [&](int j, int v) {
                 const int r = lane_id() & 31, c = j * 32 + split_gemm::acc_column(v);
                 if (block_row + r < rows && first + c < D)
-                    out[r * D + c] = from_f32<T>(
-                        split_gemm::scalar_dot(G + (block_row + r) * V, weight + first + c, V, 0.0f, 1, D));
+                    out[r * D + c] = from_f32<Out>(split_gemm::scalar_dot(
+                        G + (block_row + r) * V + k0, weight + k0 * D + first + c, k1 - k0, 0.0f, 1, D));
             });
         }
     }
@@ -287,11 +406,12 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
 // Partial sums of grad_weight [V, D] = G^T [V, rows] prior [rows, D] over the
 // rows [chunk * chunk_rows, + chunk_rows): a vocabulary this small has few
 // tiles, so the rows are split until the chip is full. At the sizes above 53 us (+ 7 for
-// the sum of the chunks), against 406 for the library's fp32 product on few tiles.
-template <typename T>
+// the sum of the chunks), against 406 for the library's fp32 product on few tiles. One
+// chunk writes the gradient itself (Out T).
+template <typename T, typename Out>
 __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
-    const float* __restrict__ G, const T* __restrict__ prior, float* __restrict__ partial, int64_t rows, int64_t D,
-    int64_t V, int64_t d_tiles, int64_t v_tiles, int64_t chunk_rows) {
+    const float* __restrict__ G, const T* __restrict__ prior, Out* __restrict__ partial, int64_t rows, int64_t D,
+    int64_t V, int64_t d_tiles, int64_t v_tiles, int64_t chunk_rows, int vec_out) {
     constexpr int BM = 128, BN = 128;
     using Tile = split_gemm::Tile<float, T, BM, BN, true, true>;
     __shared__ __attribute__((aligned(16))) char lds[Tile::kLdsBytes];
@@ -304,7 +424,7 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
         lds, rows, rows, k0, k1, [&](int r) { return G + min(v0 + r, V - 1); },
         [&](int r) { return prior + min(d0 + r, D - 1); }, [&](int t) { return wn * 64 + t * 32; }, V, D);
     split_gemm::lds_barrier();  // the output rows pass through LDS
-    constexpr int kRegion = split_gemm::store_bytes<float, 1>();
+    constexpr int kRegion = split_gemm::store_bytes<Out, 1>();
     static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
 #pragma unroll
     for (int i = 0; i < Tile::MT; ++i) {
@@ -315,26 +435,30 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
             float o[1][16];
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[0][e] = tile.acc[i][j][e];
-            float* out = partial + (chunk * V + block_v) * D + first;
-            split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, D, V - block_v, D - first, D % 8 == 0);
+            Out* out = partial + (chunk * V + block_v) * D + first;
+            split_gemm::store_rows<Out, 1>(lds + wave * kRegion, o, out, D, V - block_v, D - first, vec_out);
             split_gemm::fix_not_finite(o, [&](int, int e) {
                 const int r = lane_id() & 31, c = split_gemm::acc_column(e);
                 if (block_v + r < V && first + c < D)
-                    out[r * D + c] = split_gemm::scalar_dot(G + k0 * V + block_v + r, prior + k0 * D + first + c, k1 - k0,
-                                                            0.0f, V, D);
+                    out[r * D + c] = from_f32<Out>(split_gemm::scalar_dot(
+                        G + k0 * V + block_v + r, prior + k0 * D + first + c, k1 - k0, 0.0f, V, D));
             });
         }
     }
 }
 
-// Workspace of the backward: G, the weight gradient's chunks, the bias
-// gradient's partial rows.
+// Workspace of the backward: G, the weight gradient's chunks, the prior gradient's
+// and the logits' (each where there are several), the bias gradient's partial rows.
 struct HeadWorkspace {
     int64_t chunks, chunk_rows, blocks;
-    size_t partial_off, bias_off, total;
+    int64_t prior_tile, prior_tiles, prior_chunks, prior_chunk;  // tile rows and columns, tiles, chunks of the vocabulary
+    int64_t head_chunks;
+    size_t partial_off, prior_off, logits_off, bias_off, total;
 };
 inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 constexpr int64_t kWeightTiles = 512;              // two workgroups per CU (256: 73 us, 512: 53)
+constexpr int64_t kPriorTiles = 256;               // the prior gradient's, where the vocabulary is long
+constexpr int64_t kPriorChunk = 256;               // vocabulary columns of a chunk at least (8 K steps)
 constexpr int64_t kPartialFloats = int64_t(1) << 24;  // 64 MiB of partial sums at most
 
 inline HeadWorkspace head_workspace(int64_t rows, int64_t D, int64_t V) {
@@ -346,9 +470,24 @@ inline HeadWorkspace head_workspace(int64_t rows, int64_t D, int64_t V) {
     if (chunks < 1) chunks = 1;
     w.chunk_rows = ((rows + chunks - 1) / chunks + 31) / 32 * 32;
     w.chunks = (rows + w.chunk_rows - 1) / w.chunk_rows;
+    // 128 x 128 tiles, or 64 x 64 ones with four K steps of loads in flight where the
+    // larger would give fewer than one to each CU (4000 rows x 300, vocabulary 1000,
+    // fp32: 67 -> 39 us); then chunks of a long vocabulary
+    w.prior_tile = (rows + 127) / 128 * ((D + 127) / 128) < 256 ? 64 : 128;
+    w.prior_tiles = (rows + w.prior_tile - 1) / w.prior_tile * ((D + w.prior_tile - 1) / w.prior_tile);
+    chunks = std::min(kPriorTiles / w.prior_tiles, V / kPriorChunk);
+    if (chunks > kPartialFloats / (rows * D)) chunks = kPartialFloats / (rows * D);
+    if (chunks < 1) chunks = 1;
+    w.prior_chunk = ((V + chunks - 1) / chunks + 31) / 32 * 32;
+    w.prior_chunks = (V + w.prior_chunk - 1) / w.prior_chunk;
     w.blocks = (rows + kRows - 1) / kRows;
     w.partial_off = align256(static_cast<size_t>(rows) * V * sizeof(float));
-    w.bias_off = w.partial_off + align256(static_cast<size_t>(w.chunks) * V * D * sizeof(float));
+    w.prior_off = w.partial_off + (w.chunks > 1 ? align256(static_cast<size_t>(w.chunks) * V * D * sizeof(float)) : 0);
+    w.head_chunks = std::max(head_chunks(rows, D, V, true), head_chunks(rows, D, V, false));  // of any type
+    w.logits_off =
+        w.prior_off + (w.prior_chunks > 1 ? align256(static_cast<size_t>(w.prior_chunks) * rows * D * sizeof(float)) : 0);
+    w.bias_off =
+        w.logits_off + (w.head_chunks > 1 ? align256(static_cast<size_t>(logits_floats(rows, V, w.head_chunks)) * sizeof(float)) : 0);
     w.total = w.bias_off + static_cast<size_t>(w.blocks) * V * sizeof(float);
     return w;
 }
@@ -362,10 +501,36 @@ bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0;
                         : ((bytes) == 16 ? run(kernel<T, kNarrow, 16>)                                  \
                            : (bytes) == 8 ? run(kernel<T, kNarrow, 8>) : run(kernel<T, kNarrow, 0>)))
 
+// Logits [rows, V] at part, the chunks' behind them.
+template <typename T>
+int head_product(const T* prior, const T* weight, float* part, int64_t rows, int64_t D, int64_t V, hipStream_t s) {
+    const int64_t tiles = head_tiles_of(rows, V), chunks = head_chunks(rows, D, V, sizeof(T) == 4);
+    const int bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
+    float* const chunk_part = part + (rows * V + 63) / 64 * 64;
+    const auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles * chunks)), dim3(kThreads), 0, s, prior, weight,
+                           chunk_part, rows, D, V, (V + 63) / 64, tiles, head_chunk(rows, D, V, sizeof(T) == 4),
+                           static_cast<int>(V % 8 == 0 && aligned16(chunk_part)));
+        return check_launch("surprise head (product)");
+    };
+    const int st = bytes == 16  ? run(surprise_head_product_kernel<T, 16>)
+                   : bytes == 8 ? run(surprise_head_product_kernel<T, 8>) : run(surprise_head_product_kernel<T, 0>);
+    if (st != KOEMI_OK) return st;
+    launch_column_sum(chunk_part, part, chunks, rows * V, s);
+    return check_launch("surprise head (product sum)");
+}
+
 template <typename T>
 int head_forward(const void* prior, const void* weight, const void* bias, const int64_t* targets, const uint8_t* valid,
                  void* out, float* stats, float* part, int64_t rows, int64_t D, int64_t V, float log_vocab,
                  hipStream_t s) {
+    if (head_chunks(rows, D, V, sizeof(T) == 4) > 1) {
+        const int st = head_product(static_cast<const T*>(prior), static_cast<const T*>(weight), part, rows, D, V, s);
+        if (st != KOEMI_OK) return st;
+        hipLaunchKernelGGL(surprise_head_score_kernel<T>, dim3(grid_for(rows, kThreads / kWave)), dim3(kThreads), 0, s, part,
+                           static_cast<const T*>(bias), targets, valid, static_cast<T*>(out), stats, rows, V, log_vocab);
+        return check_launch("koemi_surprise_head_forward(scores)");
+    }
     const int columns = head_columns(rows, V);
     const int bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
     const int64_t v_tiles = (V + columns - 1) / columns;
@@ -393,42 +558,70 @@ int head_backward(const void* prior, const void* weight, const void* bias, const
     const T* p = static_cast<const T*>(prior);
     const T* w = static_cast<const T*>(weight);
     const int64_t d_tiles = (D + 127) / 128, v_tiles = (V + 127) / 128;
-    const int columns = head_columns(rows, V);
-    const int head_bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
-    const int64_t head_tiles = (V + columns - 1) / columns;
-    const auto run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ws.blocks * head_tiles)), dim3(kThreads), 0, s, p, w,
-                           static_cast<const T*>(bias), targets, valid, static_cast<const T*>(grad), stats, G,
-                           bias_partial, rows, D, V, head_tiles, log_vocab);
-        return check_launch("koemi_surprise_head_backward(logits)");
-    };
-    int st = KOEMI_HEAD_KERNEL(run, surprise_head_grad_logits_kernel, T, columns, head_bytes);
+    int st;
+    if (head_chunks(rows, D, V, sizeof(T) == 4) > 1) {
+        float* const logits = reinterpret_cast<float*>(base + ws.logits_off);
+        st = head_product(p, w, logits, rows, D, V, s);
+        if (st != KOEMI_OK) return st;
+        const int64_t tiles = (V + kWave - 1) / kWave;
+        hipLaunchKernelGGL(surprise_head_split_grad_kernel<T>, dim3(static_cast<unsigned>(ws.blocks * tiles)),
+                           dim3(kSplitGradThreads), 0, s, logits, static_cast<const T*>(bias), targets, valid,
+                           static_cast<const T*>(grad), stats, G, bias_partial, rows, V, tiles, log_vocab);
+        st = check_launch("koemi_surprise_head_backward(logits)");
+    } else {
+        const int columns = head_columns(rows, V);
+        const int head_bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
+        const int64_t head_tiles = (V + columns - 1) / columns;
+        const auto run = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ws.blocks * head_tiles)), dim3(kThreads), 0, s, p, w,
+                               static_cast<const T*>(bias), targets, valid, static_cast<const T*>(grad), stats, G,
+                               bias_partial, rows, D, V, head_tiles, log_vocab);
+            return check_launch("koemi_surprise_head_backward(logits)");
+        };
+        st = KOEMI_HEAD_KERNEL(run, surprise_head_grad_logits_kernel, T, columns, head_bytes);
+    }
     if (st != KOEMI_OK) return st;
     const int bytes = split_gemm::load_bytes<float>(G, V);
-    // 128 x 128 tiles, or 64 x 64 ones with four K steps of loads in flight where the
-    // larger would give fewer than one to each CU (4000 rows x 300, vocabulary 1000,
-    // fp32: 67 -> 39 us)
-    const int64_t b = (rows + 127) / 128 * d_tiles < 256 ? 64 : 128;
-    const int64_t prior_tiles = (D + b - 1) / b;
-    const auto prior_run = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((rows + b - 1) / b * prior_tiles)), dim3(kThreads), 0, s, G,
-                           w, static_cast<T*>(grad_prior), rows, D, V, prior_tiles,
-                           static_cast<int>(D % 8 == 0 && aligned16(grad_prior)));
+    const int64_t b = ws.prior_tile;
+    const auto prior_run = [&](auto kernel, auto* out) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ws.prior_tiles * ws.prior_chunks)), dim3(kThreads), 0, s, G,
+                           w, out, rows, D, V, (D + b - 1) / b, ws.prior_tiles, ws.prior_chunk,
+                           static_cast<int>(D % 8 == 0 && aligned16(out)));
         return check_launch("koemi_surprise_head_backward(prior)");
     };
-    st = b == 128 ? (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, 128, 16>)
-                     : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, 128, 8>)
-                                  : prior_run(surprise_head_grad_prior_kernel<T, 128, 0>))
-                  : (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, 64, 16>)
-                     : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, 64, 8>)
-                                  : prior_run(surprise_head_grad_prior_kernel<T, 64, 0>));
+    T* const gp = static_cast<T*>(grad_prior);
+    if (ws.prior_chunks > 1) {  // few tiles: 64 x 64
+        float* const part = reinterpret_cast<float*>(base + ws.prior_off);
+        st = bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, float, 64, 16>, part)
+             : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, float, 64, 8>, part)
+                          : prior_run(surprise_head_grad_prior_kernel<T, float, 64, 0>, part);
+        if (st != KOEMI_OK) return st;
+        launch_column_sum(part, gp, ws.prior_chunks, rows * D, s);
+        st = check_launch("koemi_surprise_head_backward(prior sum)");
+    } else {
+        st = b == 128 ? (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, T, 128, 16>, gp)
+                         : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, T, 128, 8>, gp)
+                                      : prior_run(surprise_head_grad_prior_kernel<T, T, 128, 0>, gp))
+                      : (bytes == 16  ? prior_run(surprise_head_grad_prior_kernel<T, T, 64, 16>, gp)
+                         : bytes == 8 ? prior_run(surprise_head_grad_prior_kernel<T, T, 64, 8>, gp)
+                                      : prior_run(surprise_head_grad_prior_kernel<T, T, 64, 0>, gp));
+    }
     if (st != KOEMI_OK) return st;
-    hipLaunchKernelGGL(surprise_head_grad_weight_kernel<T>, dim3(static_cast<unsigned>(ws.chunks * d_tiles * v_tiles)),
-                       dim3(kThreads), 0, s, G, p, partial, rows, D, V, d_tiles, v_tiles, ws.chunk_rows);
-    st = check_launch("koemi_surprise_head_backward(weight)");
-    if (st != KOEMI_OK) return st;
-    launch_column_sum(partial, static_cast<T*>(grad_weight), ws.chunks, V * D, s);
-    st = check_launch("koemi_surprise_head_backward(weight sum)");
+    const auto weight_run = [&](auto kernel, auto* out) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(ws.chunks * d_tiles * v_tiles)), dim3(kThreads), 0, s, G, p,
+                           out, rows, D, V, d_tiles, v_tiles, ws.chunk_rows,
+                           static_cast<int>(D % 8 == 0 && aligned16(out)));
+        return check_launch("koemi_surprise_head_backward(weight)");
+    };
+    T* const gw = static_cast<T*>(grad_weight);
+    if (ws.chunks > 1) {
+        st = weight_run(surprise_head_grad_weight_kernel<T, float>, partial);
+        if (st != KOEMI_OK) return st;
+        launch_column_sum(partial, gw, ws.chunks, V * D, s);
+        st = check_launch("koemi_surprise_head_backward(weight sum)");
+    } else {
+        st = weight_run(surprise_head_grad_weight_kernel<T, T>, gw);
+    }
     if (st != KOEMI_OK) return st;
     launch_column_sum(bias_partial, static_cast<T*>(grad_bias), ws.blocks, V, s);
     return check_launch("koemi_surprise_head_backward(bias sum)");
@@ -450,9 +643,13 @@ using namespace koemi;
 
 extern "C" size_t koemi_surprise_head_forward_workspace_bytes(int64_t rows, int64_t vocab) {
     if (rows < 1 || vocab < 2) return 0;
-    const int columns = head_columns(rows, vocab);
-    if (vocab <= columns) return 0;
-    return static_cast<size_t>((vocab + columns - 1) / columns) * 3 * static_cast<size_t>(rows) * sizeof(float);
+    const size_t row_bytes = static_cast<size_t>(rows) * sizeof(float);
+    // chunks of the widest state, 12 MiB at most
+    const int64_t chunks = kMostSplitTiles / head_tiles_of(rows, vocab);
+    const size_t split = chunks > 1 ? static_cast<size_t>(logits_floats(rows, vocab, chunks)) * sizeof(float) : 0;
+    const int64_t columns = head_columns(rows, vocab);
+    const size_t tiles = vocab > columns ? static_cast<size_t>((vocab + columns - 1) / columns * 3) * row_bytes : 0;
+    return std::max(split, tiles);
 }
 
 extern "C" int koemi_surprise_head_forward(const void* prior, const void* weight, const void* bias,

@@ -207,6 +207,8 @@ def test_fixed_threshold_admission_is_strict(device):
 @pytest.mark.parametrize("batch,length,width,vocab", [
     (1, 1, 1, 2), (3, 21, 8, 19), (1, 64, 64, 256), (5, 13, 72, 257), (2, 64, 300, 255), (1, 129, 136, 520),
     (4, 300, 128, 256), (3, 700, 40, 130), (2, 65, 512, 1000), (9, 600, 264, 64),
+    # few tiles of a wide state (its width in chunks) and of a long vocabulary (the prior gradient's chunks)
+    (1, 70, 2048, 257), (1, 16, 4096, 65), (2, 600, 1030, 100), (1, 40, 600, 700), (1, 1, 513, 2), (1, 33, 72, 3000),
 ])
 def test_causal_surprise_head_of_every_tile_shape(device, dtype, batch, length, width, vocab):
     """Scores and gradients at the edges of the head's tiles (64 rows, 256 columns, 128 columns of the
@@ -290,15 +292,18 @@ def test_causal_surprise_contains_what_is_not_finite(device, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("rows, vocab", [(70, 65), (70, 129), (70, 67), (70, 257), (9000, 257), (9000, 300), (70, 64), (9000, 256)])
-def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab):
+@pytest.mark.parametrize("rows, vocab, width", [
+    (70, 65, 40), (70, 129, 40), (70, 67, 40), (70, 257, 40), (9000, 257, 40), (9000, 300, 40), (70, 64, 40), (9000, 256, 40),
+    (70, 257, 600),  # the width in chunks
+])
+def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab, width):
     """A NaN in the last weight row or the last bias, in a last tile of one column, of several and among
     minus infinities, makes every valid row's score and gradient NaN, whatever the vocabulary's tiles; a
     last tile whose biases are all minus infinity leaves the scores of the other columns."""
 
     g = torch.Generator().manual_seed(rows + vocab)
-    prior = (0.5 * torch.randn((1, rows, 40), generator=g)).to(dtype).to(device)
-    weight = (0.2 * torch.randn((vocab, 40), generator=g)).to(dtype).to(device)
+    prior = (0.5 * torch.randn((1, rows, width), generator=g)).to(dtype).to(device)
+    weight = (0.2 * torch.randn((vocab, width), generator=g)).to(dtype).to(device)
     bias = (0.1 * torch.randn((vocab,), generator=g)).to(dtype).to(device)
     tile = 64 if rows == 70 else 256
     last = (vocab - 1) // tile * tile  # the last tile's first column
@@ -328,8 +333,8 @@ def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab):
         z = prior.double() @ weight.double()[:last].t() + bias.double()[:last]
         nll = torch.logsumexp(z, -1) - z.gather(-1, targets[..., None])[..., 0]
         want = torch.where(valid, 1 - torch.exp(-nll / math.log(vocab)), 0.0)
-        # the fp32 logits of 40 terms of order one and a few roundings, then the score's own type
-        assert bool(((score.double() - want).abs() <= 2.0**-19 + (2.0**-8 if dtype == torch.bfloat16 else 0) * want).all())
+        # the fp32 logits of `width` terms below one and a few roundings, then the score's own type
+        assert bool(((score.double() - want).abs() <= 2.0**-19 * width / 40 + (2.0**-8 if dtype == torch.bfloat16 else 0) * want).all())
         assert torch.isfinite(grad).all()
 
 
