@@ -98,10 +98,9 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void gate_products_kernel(
     float* z = column < half_tiles ? zr : zc;
     const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
     Tile tile;
-    tile.template run<BYTES, BYTES>(
+    const uint64_t chains = tile.template run<BYTES, BYTES>(
         lds, D, D, 0, (D + Tile::BK - 1) / Tile::BK * Tile::BK, [&](int r) { return u + min(row0 + r, rows - 1) * D; },
         [&](int r) { return w + min(n0 + r, D - 1) * D; }, [&](int t) { return wn * (B / 2) + t * 32; });
-    split_gemm::lds_barrier();  // the output rows pass through LDS
 #pragma unroll
     for (int i = 0; i < Tile::MT; ++i) {
         const int64_t block_row = row0 + wm * (B / 2) + i * 32;
@@ -111,15 +110,15 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void gate_products_kernel(
             float o[1][16];
 #pragma unroll
             for (int v = 0; v < 16; ++v) o[0][v] = tile.acc[i][j][v];
-            float* out = z + block_row * D + c0;
-            split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, D, rows - block_row, D - c0, D % 8 == 0);
-            split_gemm::fix_not_finite(o, [&](int, int v) {
-                const int r = lane_id() & 31, c = split_gemm::acc_column(v);
-                if (block_row + r < rows && c0 + c < D)
-                    out[r * D + c] = split_gemm::scalar_dot(u + (block_row + r) * D, w + (c0 + c) * D, D, 0.0f);
-            });
+            split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, z + block_row * D + c0, D, rows - block_row, D - c0,
+                                             D % 8 == 0);
         }
     }
+    split_gemm::fix_chains(chains, [&](int block, int v) {
+        const int64_t r = row0 + wm * (B / 2) + block / Tile::NT * 32 + (lane_id() & 31);
+        const int64_t c = n0 + wn * (B / 2) + block % Tile::NT * 32 + split_gemm::acc_column(v);
+        if (r < rows && c < D) z[r * D + c] = split_gemm::scalar_dot(u + r * D, w + c * D, D, 0.0f);
+    });
 }
 
 int gate_products_f32(const float* u, const float* wr, const float* wc, float* zr, float* zc, int64_t rows, int64_t D,

@@ -635,7 +635,7 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
     const TW* w0 = W0 + static_cast<int64_t>(e) * n_out * K;
     const TW* w1 = W1 + static_cast<int64_t>(e) * n_out * K;
     G tile;
-    tile.template run<GLU ? BYTES : 16, BYTES>(  // H rows are padded to 32 bytes
+    uint64_t chains = tile.template run<GLU ? BYTES : 16, BYTES>(  // H rows are padded to 32 bytes
              lds, lda, K, 0, (K + G::BK - 1) / G::BK * G::BK,
              [&](int r) { return A + min(row0 + r, row_end - 1) * lda; },
              [&](int r) {
@@ -643,7 +643,7 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
                  return w0 + min(n0 + r, n_out - 1) * K;
              },
              [&](int t) { return GLU ? t * (BN / 2) + wn * 32 : wn * (BN / 2) + t * 32; });
-    split_gemm::lds_barrier();  // the output rows pass through LDS
+    if constexpr (G::kNative) split_gemm::lds_barrier();  // the output rows pass through LDS
     constexpr int J = GLU ? 1 : G::NT;
     using Out = std::conditional_t<GLU, float, TW>;
     constexpr int kRegion = split_gemm::store_bytes<Out, J>();
@@ -679,16 +679,19 @@ __global__ __launch_bounds__(split_gemm::kThreads, 2) void grouped_gemm_any_kern
         Out* y = static_cast<Out*>(out) + block_row * ldc + first;
         split_gemm::store_rows<Out, J>(lds + (threadIdx.x / kWave) * kRegion, o, y, ldc, row_end - block_row, cols,
                                        GLU || vec_out);
-        if constexpr (!G::kNative)
-            split_gemm::fix_not_finite(o, [&](int j, int v) {
-                const int r = lane_id() & 31, c = j * 32 + split_gemm::acc_column(v);
-                if (block_row + r >= row_end) return;
-                const TA* a = A + (block_row + r) * lda;
-                float x = split_gemm::scalar_dot(a, w0 + (first + c) * K, K, to_f32(bias_g[first + c]));
-                if constexpr (GLU)
-                    x = silu_f(x) * split_gemm::scalar_dot(a, w1 + (first + c) * K, K, to_f32(bias_v[first + c]));
-                y[r * ldc + c] = from_f32<Out>(x);
-            });
+    }
+    if constexpr (!G::kNative) {
+        if constexpr (GLU) chains |= chains >> 16 | chains << 16;  // a gate or a value: the pair's output
+        split_gemm::fix_chains(chains, [&](int block, int v) {
+            if (GLU && block % G::NT != 0) return;
+            const int64_t r = row0 + wm * (BM / 2) + block / G::NT * 32 + (lane_id() & 31);
+            const int64_t c = first + block % G::NT * 32 + split_gemm::acc_column(v);
+            if (r >= row_end || c >= n_out) return;
+            const TA* a = A + r * lda;
+            float x = split_gemm::scalar_dot(a, w0 + c * K, K, to_f32(bias_g[c]));
+            if constexpr (GLU) x = silu_f(x) * split_gemm::scalar_dot(a, w1 + c * K, K, to_f32(bias_v[c]));
+            static_cast<Out*>(out)[r * ldc + c] = from_f32<Out>(x);
+        });
     }
 }
 

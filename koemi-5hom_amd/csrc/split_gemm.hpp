@@ -17,9 +17,14 @@
 // 0.41, 0.47 and 0.40 of the terms' sizes). One or two terms come out within 2.3
 // units, where a chain's are within 1 and 1.8.
 //
-// Infinities and NaN do not survive a split (inf x 0 between planes): callers
-// recompute an output that is not finite with scalar_dot, the plain
-// multiply-add chain, so that such inputs give what the chain gives.
+// Infinities and NaN do not survive a split (inf x 0 between planes), nor do
+// values that round past bf16's range. A tile with an output that is not finite
+// walks K again on one plane of what each operand is (classes): infinities and NaN
+// as they are, any other value as 0 or a power of two whose products vanish, so
+// that a NaN output becomes the infinity or NaN that multiply-adds give and the
+// finite ones keep their bits. A NaN that finite operands made is left to the caller
+// (scalar_dot). [16384, 1024] gates with their scan, every input NaN: 0.60 ms (0.44
+// finite; 60 with a chain for each output, 0.61 with the library's fp32 products).
 #pragma once
 
 #include "common.hpp"
@@ -141,6 +146,33 @@ __device__ __forceinline__ uint4 take_plane(float (&f)[8]) {
     return r;
 }
 
+// Eight values as bf16 classes: infinities and NaN as they are, others as 0 or a
+// signed 2^-100 (a product of two lies below fp32's smallest step).
+template <typename T>
+__device__ __forceinline__ uint4 classes(const Octet<T>& o) {
+    bf16x8 c;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float f = o.value(i);
+        c[i] = static_cast<__bf16>(fabsf(f) < __builtin_inff() ? f == 0.0f ? 0.0f : copysignf(0x1p-100f, f) : f);
+    }
+    return __builtin_bit_cast(uint4, c);
+}
+
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) < __builtin_inff(); }
+
+// Element v of a lane's accumulators of n-tile t: A row `lane % 32` of the
+// m-tile, B row 8 (v / 4) + 4 (lane / 32) + v % 4 of the n-tile.
+__device__ __forceinline__ int acc_column(int v) { return 8 * (v / 4) + 4 * (lane_id() / 32) + v % 4; }
+
+// start + sum_k a[k a_ld] b[k b_ld] as one fp32 multiply-add chain.
+template <typename TA, typename TB>
+__device__ __noinline__ float scalar_dot(const TA* a, const TB* b, int64_t K, float start, int64_t a_ld = 1,
+                                         int64_t b_ld = 1) {
+    for (int64_t k = 0; k < K; ++k) start = __builtin_fmaf(to_f32(a[k * a_ld]), to_f32(b[k * b_ld]), start);
+    return start;
+}
+
 // A block tile of BM rows of A by BN rows of B, K in steps of BK through one LDS
 // buffer; the next step's operands are loaded into registers before this step's
 // products and split on their way into LDS. BK = 64 where neither operand is
@@ -179,12 +211,12 @@ struct Tile {
     // or four consecutive threads share a row of a K-contiguous operand (its
     // 16-byte pieces), consecutive threads take consecutive rows of a strided one.
     template <int R, bool STRIDED>
-    __device__ static int octet_row(int i) {
-        return STRIDED ? (threadIdx.x + i * kThreads) % R : (threadIdx.x + i * kThreads) / kGroups;
+    __device__ static int octet_row(int i, int tid = threadIdx.x) {
+        return STRIDED ? (tid + i * kThreads) % R : (tid + i * kThreads) / kGroups;
     }
     template <int R, bool STRIDED>
-    __device__ static int octet_group(int i) {
-        return STRIDED ? (threadIdx.x + i * kThreads) / R : threadIdx.x % kGroups;
+    __device__ static int octet_group(int i, int tid = threadIdx.x) {
+        return STRIDED ? (tid + i * kThreads) / R : tid % kGroups;
     }
 
     // a_row(r), b_row(r): pointers to row r of the block tile's operands, for
@@ -192,9 +224,12 @@ struct Tile {
     // A_BYTES and B_BYTES; a strided
     // operand's row is the column whose value k lies at k * a_ld (b_ld).
     // b_first(t): the block tile's B row where this wave's n-tile t starts.
+    // Split operands: the workgroup's waves are joined at the end (LDS is free). Returns
+    // a bit ((i NT + j) 16 + v) for each output of the lane that the caller has to form
+    // with scalar_dot (fix_chains).
     template <int A_BYTES, int B_BYTES, typename ARow, typename BRow, typename BFirst>
-    __device__ __forceinline__ void run(char* lds, int64_t KA, int64_t KB, int64_t k_begin, int64_t k_end, ARow a_row,
-                                        BRow b_row, BFirst b_first, int64_t a_ld = 1, int64_t b_ld = 1) {
+    __device__ __forceinline__ uint64_t run(char* lds, int64_t KA, int64_t KB, int64_t k_begin, int64_t k_end,
+                                            ARow a_row, BRow b_row, BFirst b_first, int64_t a_ld = 1, int64_t b_ld = 1) {
         const int lane = lane_id(), wave = threadIdx.x / kWave;
         const int wm = wave >> 1;
         const TA* ap[OA];
@@ -303,9 +338,91 @@ struct Tile {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) acc[i][j] = total[i][j];
         }
+        uint64_t chains = 0;
+        if constexpr (!kNative) {
+            float zero[4] = {};  // NaN once an output is not finite: one multiply-add an output
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) zero[v % 4] = __builtin_fmaf(acc[i][j][v], 0.0f, zero[v % 4]);
+            const bool whole = (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.0f;
+            __shared__ __attribute__((aligned(16))) uint32_t votes[kThreads / kWave];
+            const uint32_t vote = __ballot(!whole) != 0;
+            if (lane == 0) votes[wave] = vote;
+            lds_barrier();
+            const uint4 any = *reinterpret_cast<const uint4*>(votes);
+            if (__builtin_expect((any.x | any.y | any.z | any.w) != 0, 0)) {
+                // an infinity came of finite operands (an infinite one makes NaN planes)
+                // and stays; a NaN becomes what the classes say
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            const bool nan = acc[i][j][v] != acc[i][j][v];
+                            chains |= nan ? 1ull << ((i * NT + j) * 16 + v) : 0ull;
+                            acc[i][j][v] = nan ? 0.0f : acc[i][j][v];
+                        }
+                // rows and addresses formed anew: kept from the loop above they would
+                // cost every tile their registers
+                int tid = threadIdx.x;
+                asm volatile("" : "+v"(tid));
+                for (int64_t k0 = k_begin; k0 < k_end; k0 += BK) {
+                    lds_barrier();  // every wave is done with the previous step's classes
+                    class_step<A_BYTES, BM, OA, A_STRIDED>(lds, tid, k0, KA, a_ld, a_row);
+                    class_step<B_BYTES, BN, OB, B_STRIDED>(lds_b, tid, k0, KB, b_ld, b_row);
+                    lds_barrier();
+#pragma unroll
+                    for (int kk = 0; kk < BK / 16; ++kk) {
+                        const int fg = kk * 2 + (lane >> 5);
+#pragma unroll
+                        for (int i = 0; i < MT; ++i)
+#pragma unroll
+                            for (int j = 0; j < NT; ++j)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                    *reinterpret_cast<const bf16x8*>(lds_b + at(b_first(j) + (lane & 31), fg)),
+                                    *reinterpret_cast<const bf16x8*>(lds + at(wm * (BM / 2) + i * 32 + (lane & 31), fg)),
+                                    acc[i][j], 0, 0, 0);
+                    }
+                }
+                // a NaN of finite operands (infinities of both signs, planes past bf16's range):
+                // the caller's
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v)
+                            chains &= finite(acc[i][j][v]) ? ~0ull : ~(1ull << ((i * NT + j) * 16 + v));
+                lds_barrier();
+            }
+        }
+        return chains;
     }
 
   private:
+    // One operand's classes of the K step at k0 into LDS.
+    template <int BYTES, int R, int O, bool STRIDED, typename Row>
+    __device__ static __forceinline__ void class_step(char* lds, int tid, int64_t k0, int64_t K, int64_t ld, Row row) {
+        using T = std::remove_const_t<std::remove_pointer_t<decltype(row(0))>>;
+        Octet<T> o[O];
+#pragma unroll
+        for (int i = 0; i < O; ++i) {
+            const int64_t k = k0 + octet_group<R, STRIDED>(i, tid) * 8;
+            if constexpr (STRIDED) load_octet_strided(o[i], row(octet_row<R, STRIDED>(i, tid)), ld, k, K, k0 + BK > K);
+            else load_octet<BYTES>(o[i], row(octet_row<R, STRIDED>(i, tid)), k, K);
+        }
+#pragma unroll
+        for (int i = 0; i < O; ++i) {
+            clear_past(o[i], k0 + octet_group<R, STRIDED>(i, tid) * 8, K);
+            *reinterpret_cast<uint4*>(lds + at(octet_row<R, STRIDED>(i, tid), octet_group<R, STRIDED>(i, tid))) =
+                classes(o[i]);
+        }
+    }
+
     __device__ static __forceinline__ void clear(f32x16 (&a)[MT][NT]) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -331,28 +448,15 @@ struct Tile {
     }
 };
 
-// Element v of a lane's accumulators of n-tile t: A row `lane % 32` of the
-// m-tile, B row 8 (v / 4) + 4 (lane / 32) + v % 4 of the n-tile.
-__device__ __forceinline__ int acc_column(int v) { return 8 * (v / 4) + 4 * (lane_id() / 32) + v % 4; }
-
-__device__ __forceinline__ bool finite(float v) { return fabsf(v) < __builtin_inff(); }
-
-// Runs fix(j, v) for every output of this lane that is not finite, after its
-// stores have left: a rolled loop over a bit mask, so that the rare case costs the
-// kernel no registers.
-template <int J, typename Fix>
-__device__ __forceinline__ void fix_not_finite(const float (&o)[J][16], Fix fix) {
-    static_assert(J * 16 <= 64, "one bit per output");
-    uint64_t mask = 0;
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) mask |= finite(o[j][v]) ? 0ull : 1ull << (j * 16 + v);
-    if (__builtin_expect(__ballot(mask != 0) == 0, 1)) return;
+// Runs fix(block, v) for every bit that Tile::run returned, after this lane's stores
+// have left: a rolled loop, so that the rare case costs the kernel no registers.
+template <typename Fix>
+__device__ __forceinline__ void fix_chains(uint64_t chains, Fix fix) {
+    if (__builtin_expect(__ballot(chains != 0) == 0, 1)) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    while (mask) {
-        const int b = __builtin_ctzll(mask);
-        mask &= mask - 1;
+    while (chains) {
+        const int b = __builtin_ctzll(chains);
+        chains &= chains - 1;
         fix(b / 16, b % 16);
     }
 }
@@ -409,14 +513,6 @@ __device__ __forceinline__ void store_rows(char* region, const float (&o)[J][16]
         }
     }
     asm volatile("" ::: "memory");
-}
-
-// start + sum_k a[k a_ld] b[k b_ld] as one fp32 multiply-add chain.
-template <typename TA, typename TB>
-__device__ __noinline__ float scalar_dot(const TA* a, const TB* b, int64_t K, float start, int64_t a_ld = 1,
-                                         int64_t b_ld = 1) {
-    for (int64_t k = 0; k < K; ++k) start = __builtin_fmaf(to_f32(a[k * a_ld]), to_f32(b[k * b_ld]), start);
-    return start;
 }
 
 }  // namespace split_gemm

@@ -47,19 +47,19 @@ __device__ __forceinline__ void head_logits(HeadTile<T, BN>& tile, char* lds, co
                                             const T* __restrict__ weight, int64_t row0, int64_t v0, int64_t rows,
                                             int64_t D, int64_t V) {
     const int wn = threadIdx.x / kWave & 1;
-    tile.template run<BYTES, BYTES>(
+    const uint64_t chains = tile.template run<BYTES, BYTES>(
         lds, D, D, 0, (D + HeadTile<T, BN>::BK - 1) / HeadTile<T, BN>::BK * HeadTile<T, BN>::BK,
         [&](int r) { return prior + min(row0 + r, rows - 1) * D; },
         [&](int r) { return weight + min(v0 + r, V - 1) * D; }, [&](int t) { return wn * (BN / 2) + t * 32; });
     if constexpr (!HeadTile<T, BN>::kNative) {
-        // a row or column with an infinity or a NaN: the plain chain's result
+        if (__builtin_expect(__ballot(chains != 0) == 0, 1)) return;
         const int wm = threadIdx.x / kWave >> 1;
         const int64_t row = min(row0 + wm * 32 + (lane_id() & 31), rows - 1);
 #pragma unroll
         for (int j = 0; j < HeadTile<T, BN>::NT; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v)
-                if (!split_gemm::finite(tile.acc[0][j][v]))
+                if (chains >> (j * 16 + v) & 1)
                     tile.acc[0][j][v] = split_gemm::scalar_dot(
                         prior + row * D, weight + min(v0 + wn * (BN / 2) + j * 32 + split_gemm::acc_column(v), V - 1) * D, D,
                         0.0f);
@@ -206,22 +206,21 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_product_kernel(
     const int64_t k0 = chunk * chunk_width, k1 = min(D, k0 + chunk_width);  // chunk_width is a multiple of BK
     const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
     Tile tile;
-    tile.template run<BYTES, BYTES>(
+    const uint64_t chains = tile.template run<BYTES, BYTES>(
         lds, D, D, k0, k1, [&](int r) { return prior + min(row0 + r, rows - 1) * D; },
         [&](int r) { return weight + min(v0 + r, V - 1) * D; }, [&](int) { return wn * 32; });
-    split_gemm::lds_barrier();  // the output rows pass through LDS
+    if constexpr (Tile::kNative) split_gemm::lds_barrier();  // the output rows pass through LDS
     const int64_t row = row0 + wm * 32, first = v0 + wn * 32;
     float o[1][16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) o[0][v] = tile.acc[0][0][v];
-    float* out = part + (chunk * rows + row) * V + first;
-    split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, out, V, rows - row, V - first, vec_out);
-    if constexpr (!Tile::kNative)
-        split_gemm::fix_not_finite(o, [&](int, int v) {
-            const int r = lane_id() & 31, c = split_gemm::acc_column(v);
-            if (row + r < rows && first + c < V)
-                out[r * V + c] = split_gemm::scalar_dot(prior + (row + r) * D + k0, weight + (first + c) * D + k0, k1 - k0, 0.0f);
-        });
+    split_gemm::store_rows<float, 1>(lds + wave * kRegion, o, part + (chunk * rows + row) * V + first, V, rows - row,
+                                     V - first, vec_out);
+    split_gemm::fix_chains(chains, [&](int, int v) {
+        const int64_t r = row + (lane_id() & 31), c = first + split_gemm::acc_column(v);
+        if (r < rows && c < V)
+            part[(chunk * rows + r) * V + c] = split_gemm::scalar_dot(prior + r * D + k0, weight + c * D + k0, k1 - k0, 0.0f);
+    });
 }
 
 // Scores of logits [rows, V], a wave per row.
@@ -317,7 +316,7 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_logits_kernel(
     Tile tile;
     if (tid < BN) bias_sh[tid] = to_f32(bias[min(v0 + tid, V - 1)]);
     head_logits<BYTES, BN>(tile, lds, prior, weight, row0, v0, rows, D, V);
-    split_gemm::lds_barrier();  // G passes through LDS
+    if constexpr (Tile::kNative) split_gemm::lds_barrier();  // G passes through LDS
     const int hit = t >= v0 && t < v0 + BN ? static_cast<int>(t - v0) - c0 : -1;
 #pragma unroll
     for (int j = 0; j < Tile::NT; j += J) {
@@ -376,10 +375,9 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
     const int64_t k0 = chunk * chunk_v, k1 = min(V, k0 + chunk_v);  // chunk_v is a multiple of BK
     const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
     Tile tile;
-    tile.template run<BYTES, kElementLoads>(
+    const uint64_t chains = tile.template run<BYTES, kElementLoads>(
         lds, V, V, k0, k1, [&](int r) { return G + min(row0 + r, rows - 1) * V; },
         [&](int r) { return weight + min(d0 + r, D - 1); }, [&](int t) { return wn * (BN / 2) + t * 32; }, 1, D);
-    split_gemm::lds_barrier();  // the output rows pass through LDS
 #pragma unroll
     for (int i = 0; i < Tile::MT; ++i) {
         const int64_t block_row = row0 + wm * (BM / 2) + i * 32;
@@ -391,16 +389,17 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_prior_kernel(
             for (int j = 0; j < J; ++j)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) o[j][v] = tile.acc[i][j0 + j][v];
-            Out* out = grad_prior + (chunk * rows + block_row) * D + first;
-            split_gemm::store_rows<Out, J>(lds + wave * kRegion, o, out, D, rows - block_row, D - first, vec_out);
-            split_gemm::fix_not_finite(o, [&](int j, int v) {
-                const int r = lane_id() & 31, c = j * 32 + split_gemm::acc_column(v);
-                if (block_row + r < rows && first + c < D)
-                    out[r * D + c] = from_f32<Out>(split_gemm::scalar_dot(
-                        G + (block_row + r) * V + k0, weight + k0 * D + first + c, k1 - k0, 0.0f, 1, D));
-            });
+            split_gemm::store_rows<Out, J>(lds + wave * kRegion, o, grad_prior + (chunk * rows + block_row) * D + first, D,
+                                           rows - block_row, D - first, vec_out);
         }
     }
+    split_gemm::fix_chains(chains, [&](int block, int v) {
+        const int64_t r = row0 + wm * (BM / 2) + block / Tile::NT * 32 + (lane_id() & 31);
+        const int64_t c = d0 + wn * (BN / 2) + block % Tile::NT * 32 + split_gemm::acc_column(v);
+        if (r < rows && c < D)
+            grad_prior[(chunk * rows + r) * D + c] =
+                from_f32<Out>(split_gemm::scalar_dot(G + r * V + k0, weight + k0 * D + c, k1 - k0, 0.0f, 1, D));
+    });
 }
 
 // Partial sums of grad_weight [V, D] = G^T [V, rows] prior [rows, D] over the
@@ -420,10 +419,9 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
     const int64_t k0 = chunk * chunk_rows, k1 = min(rows, k0 + chunk_rows);  // chunk_rows is a multiple of BK
     const int wave = threadIdx.x / kWave, wm = wave >> 1, wn = wave & 1;
     Tile tile;
-    tile.template run<kElementLoads, kElementLoads>(
+    const uint64_t chains = tile.template run<kElementLoads, kElementLoads>(
         lds, rows, rows, k0, k1, [&](int r) { return G + min(v0 + r, V - 1); },
         [&](int r) { return prior + min(d0 + r, D - 1); }, [&](int t) { return wn * 64 + t * 32; }, V, D);
-    split_gemm::lds_barrier();  // the output rows pass through LDS
     constexpr int kRegion = split_gemm::store_bytes<Out, 1>();
     static_assert(4 * kRegion <= Tile::kLdsBytes, "the output regions fit the operands' LDS");
 #pragma unroll
@@ -435,16 +433,17 @@ __global__ __launch_bounds__(kThreads, 2) void surprise_head_grad_weight_kernel(
             float o[1][16];
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[0][e] = tile.acc[i][j][e];
-            Out* out = partial + (chunk * V + block_v) * D + first;
-            split_gemm::store_rows<Out, 1>(lds + wave * kRegion, o, out, D, V - block_v, D - first, vec_out);
-            split_gemm::fix_not_finite(o, [&](int, int e) {
-                const int r = lane_id() & 31, c = split_gemm::acc_column(e);
-                if (block_v + r < V && first + c < D)
-                    out[r * D + c] = from_f32<Out>(split_gemm::scalar_dot(
-                        G + k0 * V + block_v + r, prior + k0 * D + first + c, k1 - k0, 0.0f, V, D));
-            });
+            split_gemm::store_rows<Out, 1>(lds + wave * kRegion, o, partial + (chunk * V + block_v) * D + first, D,
+                                           V - block_v, D - first, vec_out);
         }
     }
+    split_gemm::fix_chains(chains, [&](int block, int e) {
+        const int64_t r = v0 + wm * (BM / 2) + block / Tile::NT * 32 + (lane_id() & 31);
+        const int64_t c = d0 + wn * 64 + block % Tile::NT * 32 + split_gemm::acc_column(e);
+        if (r < V && c < D)
+            partial[(chunk * V + r) * D + c] =
+                from_f32<Out>(split_gemm::scalar_dot(G + k0 * V + r, prior + k0 * D + c, k1 - k0, 0.0f, V, D));
+    });
 }
 
 // Workspace of the backward: G, the weight gradient's chunks, the prior gradient's

@@ -682,3 +682,34 @@ def test_any_shape_of_more_experts_than_the_prefix_in_lds(device):
     with pytest.raises(_native.NativeCallError, match="at most 8191 experts"):
         moe.grouped_expert_mlp_inference(torch.zeros((300, 64), device=device, dtype=torch.bfloat16), on(experts),
                                          on(offsets), *wide)
+
+
+def test_any_shape_finite_values_past_the_planes(device):
+    """fp32 inputs within half a bf16 step of the largest value, whose first plane is infinite, come through
+    to the bit, two of them cancel, a sum past the range is that infinity, and other rows keep their bits."""
+
+    g = torch.Generator().manual_seed(2)
+    D, H, P = 40, 24, 70
+    x = torch.randn((P, D), generator=g)
+    offsets, experts = torch.tensor([0, P]), torch.zeros(P, dtype=torch.int64)
+    gate, value = torch.zeros((1, H, D)), torch.zeros((1, H, D))
+    value[0, :, 0] = 1.0  # hidden unit h: factor * x[0]
+    value[0, 5, 1] = 1.0  # one of them factor * (x[0] + x[1])
+    out = torch.zeros((1, D, H))
+    out[0, torch.arange(H), torch.arange(H)] = 1.0
+    out[0, 30, :] = 1.0  # the sum of all
+    ws = [gate, torch.full((1, H), 0.75), value, torch.zeros((1, H)), out, torch.zeros((1, D))]
+    run = lambda x: moe.grouped_expert_mlp_inference(x.to(device), experts.to(device), offsets.to(device),
+                                                     *(w.to(device) for w in ws)).cpu()
+    x[1, :2] = torch.tensor([1.0, 0.0])
+    clean = run(x)
+    factor = clean[1, 0]  # silu(0.75), about a half
+    top = torch.tensor(float(np.uint32(0x7f7fffff).view(np.float32)))
+    x[3, 0], x[3, 1] = top, -top
+    x[9, 0], x[9, 1] = -top, 0.0
+    got = run(x)
+    assert torch.equal(got[3, :5], (factor * top).expand(5)) and got[3, 5] == 0.0
+    assert torch.equal(got[9, :H], (-factor * top).expand(H))
+    assert got[3, 30] == float("inf") and got[9, 30] == -float("inf")
+    rows = [r for r in range(P) if r not in (3, 9)]
+    assert torch.equal(got[rows], clean[rows])

@@ -408,3 +408,33 @@ def test_fp32_gate_products_of_every_tile_shape(device, rows, width):
         assert torch.isnan(out[0][rows // 2]).all()
         sign = wr[:, 0].to(device) > 0
         assert torch.equal(out[0][0], torch.where(sign, 1 - 2.0**-8, 2.0**-8).float())
+
+
+def test_fp32_gates_of_values_that_are_not_finite_take_no_longer_than_the_library(device):
+    """The products of inputs with NaN or infinities walk their sums once more at the matrix rate, they
+    are not formed one output at a time: within twice the library's two fp32 products and a finite call
+    (a chain per output takes a hundred times as long)."""
+
+    rows, width = 8192, 1024
+    g = torch.Generator(device=device).manual_seed(1)
+    u = torch.randn((rows, width), generator=g, device=device)
+    wr, wc = (torch.randn((width, width), generator=g, device=device) / 32 for _ in range(2))
+    br, bc = (torch.zeros(width, device=device) for _ in range(2))
+    def ms(call):
+        best = float("inf")
+        for _ in range(5):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            call()
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+    gates = lambda x: recurrent.recurrent_gates(x, wr, br, wc, bc)
+    bar = 2 * (ms(lambda: (u @ wr.t(), u @ wc.t())) + ms(lambda: gates(u)))
+    for bad in (float("nan"), float("inf")):
+        poisoned = u.clone()
+        poisoned[:, 3] = bad
+        took = ms(lambda: gates(poisoned))
+        print(f"{bad}: {took:.3f} ms, bar {bar:.3f}", flush=True)
+        assert took <= bar
