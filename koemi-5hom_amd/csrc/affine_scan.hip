@@ -39,7 +39,9 @@ constexpr int kScanSegments = KOEMI_SCAN_SEGMENTS;  // NSEG: waves per workgroup
 // Loads are unconditional (the position is clamped into the sequence) and the
 // identity element is selected when the chunk is scanned: loads under divergent
 // branches, or selects beside them, would wait for every outstanding load,
-// including the prefetch of the next chunk.
+// including the prefetch of the next chunk. The forward widens as it loads (a 16-bit
+// register shared by two steps costs more than it saves: [32, 4096, 512] fp16 94 us,
+// 86 so, fp32 the same).
 //
 // LPC > 1 splits each wave into LPC groups of 64 / LPC lanes, each a segment of its
 // own: a workgroup owns 64 / LPC columns and NSEG * LPC segments, so a batch of few
@@ -72,15 +74,15 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
     A carry = col_ok ? static_cast<A>(h0[bi * F + fc]) : A(0);
 
     struct Raw {
-        T a[S], b[S];
+        A a[S], b[S];
     };
     auto fetch = [&](int64_t t_first, Raw& raw) {
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const int64_t t = t_first + i;
             const int64_t tc = t < L ? t : L - 1;
-            raw.a[i] = a_col[tc * a_stride];
-            raw.b[i] = b_col[tc * F];
+            raw.a[i] = static_cast<A>(a_col[tc * a_stride]);
+            raw.b[i] = static_cast<A>(b_col[tc * F]);
         }
     };
     // Scan one chunk, starting at t0, and write its states.
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(kWave * NSEG) void scan_forward_kernel(
         __syncthreads();
         // Compose the carried state through the segments before this one.
         A c = carry, c_in = carry;
-#pragma unroll 8  // all of them at once would hold every segment's transfer in registers
+#pragma unroll(NS <= 16 ? NS : 8)
         for (int j = 0; j < NS; ++j) {
             if (j == seg) c_in = c;
             c = seg_p[j][lane] * c + seg_b[j][lane];
