@@ -9,10 +9,9 @@
 //   invalid positions (valid mask given and false): a = 1, b = 0
 //
 // The two width x width products leave fp32 results in the workspace: fp32 inputs
-// on the matrix cores as split bf16 planes (split_gemm.hpp; fp32 accumulation, the
-// products as exact as fp32 ones), 16-bit ones and a few rows as plain GEMMs on rocBLAS. One HIP
-// kernel then applies
-// the biases, the bounded sigmoid, tanh and the mask and writes a and b in the
+// on the matrix cores as split bf16 planes (split_gemm.hpp; fp32 accumulation), 16-bit
+// ones and few rows of some widths as plain GEMMs on rocBLAS. One HIP kernel then
+// applies the biases, the bounded sigmoid, tanh and the mask and writes a and b in the
 // input dtype, reading each fp32 product once (16-byte loads, four columns per
 // thread). koemi_recurrent_scan (fp32) hands the two products straight to the
 // affine-scan kernel, which applies the same expressions in registers, so a
@@ -142,14 +141,18 @@ int gate_products_f32(const float* u, const float* wr, const float* wc, float* z
     return wide ? run(gate_products_kernel<64, 16>) : run(gate_products_kernel<64, 0>);
 }
 
-// zr = u W_r^T, zc = u W_c^T (row-major [rows, D], fp32); 16-bit inputs and a few rows on rocBLAS: in its
-// column-major terms Z' (D x rows) = W'^T (D x D) . u' (D x rows).
+// zr = u W_r^T, zc = u W_c^T (row-major [rows, D], fp32); 16-bit inputs and few rows of
+// some widths on rocBLAS: in its column-major terms Z' (D x rows) = W'^T (D x D) . u' (D x rows).
 int gate_products(const void* input, const void* retention_weight, const void* candidate_weight, float* zr,
                   float* zc, int64_t rows, int64_t width, int dtype, hipStream_t s) {
-    // a few rows of a wide product leave most CUs idle for a long walk over K: there
-    // rocBLAS's smaller tiles are as fast (32 rows x 1024: 28 us with the scan, 30 on
-    // these tiles; 168 x 512: 28 and 21)
-    const bool few = (rows + 63) / 64 * 2 * ((width + 63) / 64) < 64 && width > 768;
+    // Few rows between 768 and 2048 wide leave most CUs idle for a long walk over K,
+    // and rocBLAS splits K there. us with the scan, library / these tiles: [64, 768]
+    // 26.4 / 25.4, [16, 1024] 25.3 / 30.0, [256, 1024] 26.5 / 30.8, [384, 1024] 31.9 /
+    // 34.0, [168, 1280] 26.4 / 35.4, [256, 1280] 33.1 / 36.2, [384, 1280] 50.7 / 38.7,
+    // [96, 1536] 29.4 / 40.6, [128, 1536] 55.4 / 40.8, [16, 2048] 72.4 / 50.5, [16, 4096]
+    // 235.9 / 91.0. Its error is the larger (5.1e-7 from float64 at [64, 1024], 2.3e-7 on
+    // the tiles), as it is where the tiles took its place.
+    const bool few = width > 768 && width < 2048 && rows * width * width < (width <= 1280 ? 430000000 : 300000000);
     if (dtype == KOEMI_F32 && !few)
         return gate_products_f32(static_cast<const float*>(input), static_cast<const float*>(retention_weight),
                                  static_cast<const float*>(candidate_weight), zr, zc, rows, width, s);

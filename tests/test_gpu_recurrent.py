@@ -375,7 +375,8 @@ def test_recurrent_gates_reject_bad_inputs(device):
         recurrent.recurrent_gates(u, wr, br, wc, bc, valid[:, :2])
 
 
-@pytest.mark.parametrize("rows, width", [(1, 4), (63, 60), (65, 64), (130, 132), (300, 516), (64, 1028), (70, 1028), (5000, 128), (4100, 260)])
+@pytest.mark.parametrize("rows, width", [(1, 4), (63, 60), (65, 64), (130, 132), (300, 516), (64, 1028), (70, 1028), (5000, 128), (4100, 260),
+                                         (410, 1028), (405, 1028), (20, 2048), (5, 772)])
 def test_fp32_gate_products_of_every_tile_shape(device, rows, width):
     """The fp32 gates at the edges of the products' tiles (64 and 128 rows and columns, K remainders, the
     library's few rows of a wide product) against float64, with rows that hold infinities and NaN.
