@@ -209,6 +209,7 @@ def test_fixed_threshold_admission_is_strict(device):
     (4, 300, 128, 256), (3, 700, 40, 130), (2, 65, 512, 1000), (9, 600, 264, 64),
     # few tiles of a wide state (its width in chunks) and of a long vocabulary (the prior gradient's chunks)
     (1, 70, 2048, 257), (1, 16, 4096, 65), (2, 600, 1030, 100), (1, 40, 600, 700), (1, 1, 513, 2), (1, 33, 72, 3000),
+    (1, 5, 24, 20000),  # tiles joined by a wave
 ])
 def test_causal_surprise_head_of_every_tile_shape(device, dtype, batch, length, width, vocab):
     """Scores and gradients at the edges of the head's tiles (64 rows, 256 columns, 128 columns of the
@@ -295,6 +296,7 @@ def test_causal_surprise_contains_what_is_not_finite(device, dtype):
 @pytest.mark.parametrize("rows, vocab, width", [
     (70, 65, 40), (70, 129, 40), (70, 67, 40), (70, 257, 40), (9000, 257, 40), (9000, 300, 40), (70, 64, 40), (9000, 256, 40),
     (70, 257, 600),  # the width in chunks
+    (70, 1100, 40),  # tiles joined by a wave
 ])
 def test_causal_surprise_of_nan_and_masked_columns(device, dtype, rows, vocab, width):
     """A NaN in the last weight row or the last bias, in a last tile of one column, of several and among
