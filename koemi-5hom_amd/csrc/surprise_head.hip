@@ -31,12 +31,13 @@ constexpr int kRows = 64;  // rows of a head tile
 // of loads in flight since no second workgroup hides them (256 rows x
 // 1024, fp32: 66 -> 26 us; a tile step costs its latency there).
 constexpr int kWide = 256, kNarrow = 64;
-constexpr int64_t kWideTiles = 256;
 
 template <typename T, int BN>
 using HeadTile = split_gemm::Tile<T, T, kRows, BN, false, false, BN == kNarrow ? 4 : 1>;
-inline int head_columns(int64_t rows, int64_t V) {
-    return (rows + kRows - 1) / kRows * ((V + kWide - 1) / kWide) < kWideTiles ? kNarrow : kWide;
+// fp32 rows of 128 to 255 wide tiles gain from the narrow ones ([8192, 1024], vocabulary
+// 256, with gradients: 208 and 163 us), 16-bit ones only lose a launch.
+inline int head_columns(int64_t rows, int64_t V, bool fp32) {
+    return (rows + kRows - 1) / kRows * ((V + kWide - 1) / kWide) < (fp32 ? 256 : 128) ? kNarrow : kWide;
 }
 
 // The logits of the workgroup's rows and vocabulary columns [v0, v0 + BN), in
@@ -182,16 +183,19 @@ __global__ void surprise_head_finish_kernel(const float* __restrict__ part, cons
 // Few 64 x 64 tiles and a wide state: each tile's sum over the width in chunks, so
 // that the chip is full ([64, 4096] fp32, vocabulary 256: forward 85 -> 17 us, a
 // tile's walk over its 128 K steps before). The chunks' logits go to part
-// [chunks, rows, V] and are added (column_sum.hpp) for the two kernels after it.
-constexpr int64_t kSplitWidth = 256;  // width of a chunk at least: four to eight K steps
-constexpr int64_t kMostSplitTiles = 512;
+// [chunks, rows, V] and are added (column_sum.hpp) for the two kernels after it. From
+// 64 K steps on: two more launches cost a short walk more than it saves ([168, 1024]
+// fp16, vocabulary 256: 137 us a call without, 150 with).
+constexpr int64_t kLongWalk = 64;      // K steps
+constexpr int64_t kSplitWidth = 256;   // width of a chunk at least
+constexpr int64_t kMostSplitTiles = 512, kMostChunks = 16;
 inline int64_t head_tiles_of(int64_t rows, int64_t V) { return (rows + 63) / 64 * ((V + 63) / 64); }
-// The chunks aimed at: a workgroup to each CU, two where fp32 planes make a long walk
-// ([2048, 4096], vocabulary 256, with gradients: 213 and 188 us; [1024, 1024], 1000: 129
-// and 144; 16-bit operands: no shape gained).
-inline int64_t split_tiles(int64_t D, bool fp32) { return fp32 && D >= 2048 ? kMostSplitTiles : 256; }
 inline int64_t head_chunk(int64_t rows, int64_t D, int64_t V, bool fp32) {  // a chunk's width; D: one chunk
-    const int64_t chunks = std::min(split_tiles(D, fp32) / head_tiles_of(rows, V), D / kSplitWidth);
+    if (D < kLongWalk * (fp32 ? HeadTile<float, kNarrow>::BK : HeadTile<bf16, kNarrow>::BK)) return D;
+    // a workgroup to each CU, two of fp32 planes ([2048, 4096], vocabulary 256, with
+    // gradients: 213 and 188 us; 16-bit operands: no shape gained)
+    const int64_t tiles = (fp32 ? kMostSplitTiles : 256) / head_tiles_of(rows, V);
+    const int64_t chunks = std::min({tiles, D / kSplitWidth, kMostChunks});
     return chunks < 2 ? D : ((D + chunks - 1) / chunks + 63) / 64 * 64;
 }
 inline int64_t head_chunks(int64_t rows, int64_t D, int64_t V, bool fp32) {
@@ -465,7 +469,7 @@ struct HeadWorkspace {
 inline size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 constexpr int64_t kWeightTiles = 512;              // two workgroups per CU (256: 73 us, 512: 53)
 constexpr int64_t kPriorTiles = 256;               // the prior gradient's, where the vocabulary is long
-constexpr int64_t kPriorChunk = 256;               // vocabulary columns of a chunk at least (8 K steps)
+constexpr int64_t kPriorLong = 2048, kPriorChunk = 256;  // such a vocabulary, and a chunk's columns at least
 constexpr int64_t kPartialFloats = int64_t(1) << 24;  // 64 MiB of partial sums at most
 
 inline HeadWorkspace head_workspace(int64_t rows, int64_t D, int64_t V) {
@@ -482,7 +486,7 @@ inline HeadWorkspace head_workspace(int64_t rows, int64_t D, int64_t V) {
     // fp32: 67 -> 39 us); then chunks of a long vocabulary
     w.prior_tile = (rows + 127) / 128 * ((D + 127) / 128) < 256 ? 64 : 128;
     w.prior_tiles = (rows + w.prior_tile - 1) / w.prior_tile * ((D + w.prior_tile - 1) / w.prior_tile);
-    chunks = std::min(kPriorTiles / w.prior_tiles, V / kPriorChunk);
+    chunks = V < kPriorLong ? 1 : std::min(kPriorTiles / w.prior_tiles, V / kPriorChunk);
     if (chunks > kPartialFloats / (rows * D)) chunks = kPartialFloats / (rows * D);
     if (chunks < 1) chunks = 1;
     w.prior_chunk = ((V + chunks - 1) / chunks + 31) / 32 * 32;
@@ -538,7 +542,7 @@ int head_forward(const void* prior, const void* weight, const void* bias, const 
                            static_cast<const T*>(bias), targets, valid, static_cast<T*>(out), stats, rows, V, log_vocab);
         return check_launch("koemi_surprise_head_forward(scores)");
     }
-    const int columns = head_columns(rows, V);
+    const int columns = head_columns(rows, V, sizeof(T) == 4);
     const int bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
     const int64_t v_tiles = (V + columns - 1) / columns;
     const auto run = [&](auto kernel) {
@@ -580,7 +584,7 @@ int head_backward(const void* prior, const void* weight, const void* bias, const
                            static_cast<const T*>(grad), stats, G, bias_partial, rows, V, tiles, log_vocab);
         st = check_launch("koemi_surprise_head_backward(logits)");
     } else {
-        const int columns = head_columns(rows, V);
+        const int columns = head_columns(rows, V, sizeof(T) == 4);
         const int head_bytes = std::min(split_gemm::load_bytes<T>(prior, D), split_gemm::load_bytes<T>(weight, D));
         const int64_t head_tiles = (V + columns - 1) / columns;
         const auto run = [&](auto kernel) {
@@ -656,9 +660,9 @@ extern "C" size_t koemi_surprise_head_forward_workspace_bytes(int64_t rows, int6
     if (rows < 1 || vocab < 2) return 0;
     const size_t row_bytes = static_cast<size_t>(rows) * sizeof(float);
     // chunks of the widest state, 12 MiB at most
-    const int64_t chunks = kMostSplitTiles / head_tiles_of(rows, vocab);
+    const int64_t chunks = std::min(kMostSplitTiles / head_tiles_of(rows, vocab), kMostChunks);
     const size_t split = chunks > 1 ? static_cast<size_t>(logits_floats(rows, vocab, chunks)) * sizeof(float) : 0;
-    const int64_t columns = head_columns(rows, vocab);
+    const int64_t columns = head_columns(rows, vocab, true);  // no wider than a 16-bit type's
     const size_t tiles = vocab > columns ? static_cast<size_t>((vocab + columns - 1) / columns * 3) * row_bytes : 0;
     return std::max(split, tiles);
 }
