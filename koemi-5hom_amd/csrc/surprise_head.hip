@@ -4,11 +4,11 @@
 // Reference: src/koemi/cuda_kernels/think/surprise_kernel.cu:194-328 (an fp32
 // library product, a row kernel over its logits, and in the backward the
 // product again, a row kernel writing the logits' gradient and two more library
-// products). Here the logits never reach memory: a workgroup holds 64 rows x 256
-// vocabulary columns in its accumulators, scores them there and keeps (max, sum
-// of exponentials, negative log-likelihood) per row for the backward, whose
-// first kernel forms the logits again and writes their gradient G (fp32). The
-// weight gradients contract G with the states and the weights, with G split into
+// products). Here the forward's logits stay on chip (few rows of a wide state aside):
+// a workgroup holds 64 rows x 256 or 64 vocabulary columns in its accumulators, scores
+// them there and keeps (max, sum of exponentials, negative log-likelihood) per row
+// for the backward, whose first kernel forms the logits again and writes their
+// gradient G (fp32). The weight gradients contract G with the states and the weights, with G split into
 // three bf16 planes that sum to it exactly (split_gemm.hpp): bf16 and fp16
 // states and weights are never widened in memory, and a product with fp32 drops
 // at most 2^-24 of itself, without bias.

@@ -122,7 +122,7 @@ def _rows_backward(
 
 
 def _head_forward(prior: Tensor, weight: Tensor, bias: Tensor, targets: Tensor, valid: Tensor) -> tuple[Tensor, Tensor]:
-    """Scores [B, L] and the rows' [3, B L] statistics for the backward, the logits kept on chip."""
+    """Scores [B, L] and the rows' [3, B L] statistics for the backward."""
 
     batch, sequence, width = prior.shape
     rows, vocab = batch * sequence, weight.shape[0]
